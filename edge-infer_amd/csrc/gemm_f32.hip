@@ -3,16 +3,15 @@
 // W is a checkpoint matrix in its stored [out, in] layout (the reference multiplies
 // the same bytes through cublasGemmEx with OP_T, operators/src/cuda/execution.cu:299-324).
 //
-// Every output element is accumulated over k in ascending order by one thread, so a
-// row's result does not depend on which other rows are in the batch, nor on which of the
-// kernels below computed it: two tiled ones (64 x 64 outputs a block; 128 x 128 for many rows
-// with K in fours) and the weight-streaming one for up to 8 rows (decode), which reads every
-// weight row in kilobyte pieces.
+// The order of an output's sum depends on K and the alignment alone, so a row's result does not
+// depend on which other rows are in the batch, nor on which of the kernels below computed it:
+// matrix-core kernels for K in fours (few rows, many rows), and one of plain multiply-adds, k in
+// ascending order, for every other size.
 #include "common.h"
 
 namespace {
 
-constexpr int BM = 64, BN = 64, BK = 16, TM = 4, TN = 4;
+constexpr int BM = 64, BN = 64, BK = 16, TM = 4, TN = 4;      // (sizes that are no multiple of 4)
 
 __global__ void __launch_bounds__(256)
 gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
@@ -64,146 +63,249 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
   }
 }
 
-// Many rows (prefill): tiles of 128 x 128 outputs, 8 x 8 of them a thread (as two by two
-// groups of 4 x 4, so that LDS is read in 16-byte pieces), the next K-tile on its way in
-// registers while this one is multiplied.  The same sums in the same order as above.
-constexpr int GM = 128, GN = 128, GK = 16, GS = GM + 4;
+// K in fours (every real model): float32 matrix products, v_mfma_f32_16x16x4_f32, whose
+// operands and sums are IEEE float32 like those of a fused multiply-add, at twice the rate of
+// v_fma_f32 (packed float32 instructions are not used).  Operands go from global memory straight
+// into the lanes that multiply them: lane (i = lane % 16, g = lane / 16) reads the four
+// neighbouring values k0 + 4 g .. + 3 of row i, and product s of a step of 16 takes the values
+// k0 + 4 g + s of the four lane groups, so one 16-byte load feeds four products.
+//
+// The sum of an output is cut into kSegs pieces of K, each a chain of products from zero, added as
+// a tree, ((c0 + c1) + (c2 + c3)) + ((c4 + c5) + (c6 + c7)).  The pieces depend on K alone and
+// both kernels below add them the same way, so a row gives the same bits in either kernel,
+// whatever other rows there are; the waves of a block take the pieces side by side.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kSegs = 8, kStep = 16, kFewRowTiles = 4;
 
-__global__ void __launch_bounds__(256)
-gemm_f32_large_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                      float* __restrict__ C, int M, int N, int K, long long lda, long long ldw,
-                      long long ldc) {
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  __shared__ __attribute__((aligned(16))) float As[GK * GS];
-  __shared__ __attribute__((aligned(16))) float Ws[GK * GS];
-  const int t = threadIdx.x, ty = t / 16, tx = t % 16;
-  const int m0 = blockIdx.y * GM, n0 = blockIdx.x * GN;
+__host__ __device__ inline int steps_a_segment(int K) {
+  return ((K + kStep - 1) / kStep + kSegs - 1) / kSegs;
+}
+
+// The chain of one piece of K for RT x CT tiles of 16 x 16 outputs: rows of A from the pointers
+// `a` (one a tile, at the lane's own row and k offset), rows of W from `w`.  The operands of the
+// next step are on their way while this one is multiplied.
+template <int RT, int CT>
+__device__ __forceinline__ void chain(const float* const (&a)[RT], const float* const (&w)[CT], int first,
+                                      int last, int k_lane, int K, f32x4 (&acc)[RT][CT]) {
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
-  float acc[8][8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
-  // thread -> two 16-byte pieces of each tile: row f / 4, floats 4 (f % 4) .. + 3, f = t, t + 256
-  f32x4 a_next[2], w_next[2];
-  auto fetch = [&](int k0) {
+    for (int j = 0; j < CT; ++j) acc[i][j] = zero;
+  if (first >= last) return;
+  f32x4 ax[2][RT], wx[2][CT];
+  // (a step beyond the last one is the last one again: asked for, never multiplied)
+  auto fetch = [&](int step, f32x4 (&ad)[RT], f32x4 (&wd)[CT]) {
+    const int k = min(step, last - 1) * kStep;
+    if (k + kStep <= K) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int f = t + 256 * i, row = f / 4, k = k0 + 4 * (f % 4);
-      a_next[i] = (m0 + row < M && k < K)
-                      ? *reinterpret_cast<const f32x4*>(A + static_cast<size_t>(m0 + row) * lda + k)
-                      : zero;
-      w_next[i] = (n0 + row < N && k < K)
-                      ? *reinterpret_cast<const f32x4*>(W + static_cast<size_t>(n0 + row) * ldw + k)
-                      : zero;
+      for (int j = 0; j < CT; ++j) wd[j] = *reinterpret_cast<const f32x4*>(w[j] + k);
+#pragma unroll
+      for (int i = 0; i < RT; ++i) ad[i] = *reinterpret_cast<const f32x4*>(a[i] + k);
+    } else {                                 // K's own end: the lanes beyond it bring zeros
+      const bool live = k + k_lane < K;
+#pragma unroll
+      for (int j = 0; j < CT; ++j) wd[j] = live ? *reinterpret_cast<const f32x4*>(w[j] + k) : zero;
+#pragma unroll
+      for (int i = 0; i < RT; ++i) ad[i] = live ? *reinterpret_cast<const f32x4*>(a[i] + k) : zero;
     }
   };
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += GK) {
-    __syncthreads();                      // the previous tile has been read
+  auto multiply = [&](const f32x4 (&ad)[RT], const f32x4 (&wd)[CT]) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int f = t + 256 * i, row = f / 4, kq = 4 * (f % 4);
+    for (int s = 0; s < 4; ++s)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        As[(kq + e) * GS + row] = a_next[i][e];
-        Ws[(kq + e) * GS + row] = w_next[i][e];
-      }
-    }
-    __syncthreads();
-    if (k0 + GK < K) fetch(k0 + GK);
+      for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int k = 0; k < GK; ++k) {
-      const f32x4 a0 = *reinterpret_cast<const f32x4*>(&As[k * GS + ty * 4]);
-      const f32x4 a1 = *reinterpret_cast<const f32x4*>(&As[k * GS + 64 + ty * 4]);
-      const f32x4 w0 = *reinterpret_cast<const f32x4*>(&Ws[k * GS + tx * 4]);
-      const f32x4 w1 = *reinterpret_cast<const f32x4*>(&Ws[k * GS + 64 + tx * 4]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          acc[i][j] = fmaf(a0[i], w0[j], acc[i][j]);
-          acc[i][4 + j] = fmaf(a0[i], w1[j], acc[i][4 + j]);
-          acc[4 + i][j] = fmaf(a1[i], w0[j], acc[4 + i][j]);
-          acc[4 + i][4 + j] = fmaf(a1[i], w1[j], acc[4 + i][4 + j]);
-        }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int m = m0 + (i / 4) * 64 + ty * 4 + i % 4;
-    if (m >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int n = n0 + (j / 4) * 64 + tx * 4 + j % 4;
-      if (n < N) C[static_cast<size_t>(m) * ldc + n] = acc[i][j];
+        for (int j = 0; j < CT; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wd[j][s], ad[i][s], acc[i][j], 0, 0, 0);
+  };
+  fetch(first, ax[0], wx[0]);
+  for (int step = first; step < last; step += 2) {
+    fetch(step + 1, ax[1], wx[1]);
+    multiply(ax[0], wx[0]);
+    if (step + 1 < last) {
+      fetch(step + 2, ax[0], wx[0]);
+      multiply(ax[1], wx[1]);
     }
   }
 }
 
-// Up to 8 rows of A (decode).  One wave per block and 16 rows of W: the wave loads 16 x 256
-// floats of W a tile (a contiguous kilobyte per row and instruction) into registers, a tile
-// ahead of the one it multiplies from LDS.  Lane (n = lane % 16, g = lane / 16) sums output
-// column n of rows g and g + 4 over k in ascending order with the same fused multiply-adds
-// as the tiled kernel, so both give the same bits.
-constexpr int FN = 16, FK = 256, FS = FK + 4;     // LDS row stride: 16-byte rows, no bank conflicts
-
-template <int RPG>   // rows of A per lane group: 1 (M <= 4) or 2 (M <= 8)
-__global__ void __launch_bounds__(EI_WAVE)
-gemm_f32_few_rows_kernel(const float* __restrict__ A, const float* __restrict__ W,
-                         float* __restrict__ C, int M, int N, int K, long long lda,
-                         long long ldw, long long ldc) {
-  typedef float f32x4 __attribute__((ext_vector_type(4)));
-  __shared__ __attribute__((aligned(16))) float Ws[FN * FS];
-  __shared__ __attribute__((aligned(16))) float Xs[4 * RPG * FS];
-  const int lane = threadIdx.x, n = lane % FN, g = lane / FN;
-  const int n0 = blockIdx.x * FN;
-  const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
-  f32x4 w_next[FN], x_next[4 * RPG];
-  // lane takes floats 4 * lane .. + 3 of the tile of every row (rows past the end: zeros)
-  auto fetch = [&](int k0) {
-    const int k = k0 + 4 * lane;
+// Many rows: a block of four waves makes 16 RT x 16 CT outputs, every wave all of them for two
+// neighbouring pieces of K, the first of which waits in LDS for the second.  No operand goes
+// through LDS: a wave's step reads 1 KB a tile row or column for 4 RT CT products of 32 cycles, 4
+// bytes a cycle and SIMD at 4 x 4 tiles.  Two blocks fit a compute unit, so one's first loads and
+// last sums lie under the other's products.
+template <int RT, int CT>
+__global__ void __launch_bounds__(256)
+gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
+                     int M, int N, int K, long long lda, long long ldw, long long ldc, int col_tiles) {
+  __shared__ f32x4 parts[kSegs / 2][RT * CT][EI_WAVE];
+  const int lane = threadIdx.x % EI_WAVE, wave = threadIdx.x / EI_WAVE;
+  const int i16 = lane % 16, g = lane / 16;
+  // Blocks go to the eight dies in turn.  Of few row tiles, those that share a column tile follow
+  // each other on one die, whose L2 then serves W to all but the first (100 x 151,936 x 1,024:
+  // 564 -> 524 us); of many, the column tiles come first, which keeps a die's share of both
+  // operands small.
+  const int row_tiles = (M + 16 * RT - 1) / (16 * RT);
+  int row_tile, col_tile;
+  if (row_tiles <= kFewRowTiles) {
+    const int die = blockIdx.x % 8, there = blockIdx.x / 8;
+    row_tile = there % row_tiles;
+    col_tile = there / row_tiles * 8 + die;
+    if (col_tile >= col_tiles) return;
+  } else {
+    row_tile = blockIdx.x / col_tiles;
+    col_tile = blockIdx.x % col_tiles;
+  }
+  const int m0 = row_tile * 16 * RT, n0 = col_tile * 16 * CT;
+  const float* a[RT];
+  const float* w[CT];
 #pragma unroll
-    for (int i = 0; i < FN; ++i)
-      w_next[i] = (n0 + i < N && k < K)
-                      ? *reinterpret_cast<const f32x4*>(W + static_cast<size_t>(n0 + i) * ldw + k)
-                      : zero;
+  for (int i = 0; i < RT; ++i)      // (rows beyond the last: that row again, never stored)
+    a[i] = A + static_cast<size_t>(min(m0 + 16 * i + i16, M - 1)) * lda + 4 * g;
 #pragma unroll
-    for (int m = 0; m < 4 * RPG; ++m)
-      x_next[m] = (m < M && k < K)
-                      ? *reinterpret_cast<const f32x4*>(A + static_cast<size_t>(m) * lda + k)
-                      : zero;
-  };
-  float acc[RPG];
+  for (int j = 0; j < CT; ++j) w[j] = W + static_cast<size_t>(min(n0 + 16 * j + i16, N - 1)) * ldw + 4 * g;
+  const int steps = (K + kStep - 1) / kStep, per = steps_a_segment(K);
+  f32x4 sum[RT][CT];
+  const int from = 2 * wave * per;
+  chain<RT, CT>(a, w, min(from, steps), min(from + per, steps), 4 * g, K, sum);
 #pragma unroll
-  for (int r = 0; r < RPG; ++r) acc[r] = 0.f;
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += FK) {
-    __syncthreads();                      // the previous tile has been read
+  for (int i = 0; i < RT; ++i)
 #pragma unroll
-    for (int i = 0; i < FN; ++i) *reinterpret_cast<f32x4*>(&Ws[i * FS + 4 * lane]) = w_next[i];
+    for (int j = 0; j < CT; ++j) parts[wave][i * CT + j][lane] = sum[i][j];
+  chain<RT, CT>(a, w, min(from + per, steps), min(from + 2 * per, steps), 4 * g, K, sum);
 #pragma unroll
-    for (int m = 0; m < 4 * RPG; ++m)
-      *reinterpret_cast<f32x4*>(&Xs[m * FS + 4 * lane]) = x_next[m];
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) sum[i][j] += parts[wave][i * CT + j][lane];
+  // the tree: neighbours first
+#pragma unroll
+  for (int apart = 1; apart < kSegs / 2; apart *= 2) {
+    if (wave % (2 * apart) == apart) {
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) parts[wave][i * CT + j][lane] = sum[i][j];
+    }
     __syncthreads();
-    if (k0 + FK < K) fetch(k0 + FK);      // on its way while this tile is multiplied
-#pragma unroll 8
-    for (int k4 = 0; k4 < FK / 4; ++k4) {
-      const f32x4 w = *reinterpret_cast<const f32x4*>(&Ws[n * FS + 4 * k4]);
+    if (wave % (2 * apart) == 0) {
 #pragma unroll
-      for (int r = 0; r < RPG; ++r) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(&Xs[(g + 4 * r) * FS + 4 * k4]);
-        acc[r] = fmaf(x[0], w[0], acc[r]);
-        acc[r] = fmaf(x[1], w[1], acc[r]);
-        acc[r] = fmaf(x[2], w[2], acc[r]);
-        acc[r] = fmaf(x[3], w[3], acc[r]);
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) sum[i][j] += parts[wave + apart][i * CT + j][lane];
+    }
+  }
+  if (wave != 0) return;
+  const bool quads = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int m = m0 + 16 * i + i16;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      const int n = n0 + 16 * j + 4 * g;
+      float* dst = C + static_cast<size_t>(m) * ldc + n;
+      if (quads && n + 4 <= N) {
+        *reinterpret_cast<f32x4*>(dst) = sum[i][j];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) dst[e] = sum[i][j][e];
       }
     }
   }
+}
+
+// Few rows (decode): bound by how fast the weights arrive.  A block of eight waves owns 16 CT rows
+// of W, a wave a piece of K; X of up to 16 RT rows is read from the caches beside it (twice as
+// many rows of W for every X where that leaves enough blocks).  Two steps are asked for while
+// two are multiplied: more of them cost waves a SIMD and read slower (622 MB, one row: 2 + 2
+// steps 119 us, 4 + 4 steps 140, 8 + 8 steps 157).
+template <int RT, int CT>
+__global__ void __launch_bounds__(512)
+gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
+                    int M, int N, int K, long long lda, long long ldw, long long ldc) {
+  constexpr int kDeep = 2;
+  __shared__ f32x4 parts[kSegs][RT * CT][EI_WAVE];
+  const int lane = threadIdx.x % EI_WAVE, wave = threadIdx.x / EI_WAVE;
+  const int i16 = lane % 16, g = lane / 16;
+  const int n0 = blockIdx.x * 16 * CT;
+  const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+  const float* w[CT];
 #pragma unroll
-  for (int r = 0; r < RPG; ++r) {
-    const int m = g + 4 * r;
-    if (m < M && n0 + n < N) C[static_cast<size_t>(m) * ldc + n0 + n] = acc[r];
+  for (int j = 0; j < CT; ++j) w[j] = W + static_cast<size_t>(min(n0 + 16 * j + i16, N - 1)) * ldw + 4 * g;
+  const float* a[RT];
+  bool row_live[RT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    row_live[i] = 16 * i + i16 < M;
+    a[i] = A + static_cast<size_t>(min(16 * i + i16, M - 1)) * lda + 4 * g;
+  }
+  const int steps = (K + kStep - 1) / kStep, per = steps_a_segment(K);
+  const int first = min(wave * per, steps), last = min(first + per, steps);
+  f32x4 acc[RT][CT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) acc[i][j] = zero;
+  f32x4 wx[2][kDeep][CT], ax[2][kDeep][RT];
+  auto fetch = [&](int step, f32x4 (&wd)[kDeep][CT], f32x4 (&ad)[kDeep][RT]) {
+#pragma unroll
+    for (int u = 0; u < kDeep; ++u) {
+      const int k = (step + u) * kStep;
+      const bool live = step + u < last && k + 4 * g < K;
+#pragma unroll
+      for (int j = 0; j < CT; ++j) wd[u][j] = live ? *reinterpret_cast<const f32x4*>(w[j] + k) : zero;
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+        ad[u][i] = (live && row_live[i]) ? *reinterpret_cast<const f32x4*>(a[i] + k) : zero;
+    }
+  };
+  auto multiply = [&](int step, const f32x4 (&wd)[kDeep][CT], const f32x4 (&ad)[kDeep][RT]) {
+#pragma unroll
+    for (int u = 0; u < kDeep; ++u) {
+      if (step + u < last) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int j = 0; j < CT; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wd[u][j][s], ad[u][i][s], acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  fetch(first, wx[0], ax[0]);
+  for (int step = first; step < last; step += 2 * kDeep) {
+    if (step + kDeep < last) fetch(step + kDeep, wx[1], ax[1]);
+    multiply(step, wx[0], ax[0]);
+    if (step + kDeep < last) {
+      if (step + 2 * kDeep < last) fetch(step + 2 * kDeep, wx[0], ax[0]);
+      multiply(step + kDeep, wx[1], ax[1]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) parts[wave][i * CT + j][lane] = acc[i][j];
+  __syncthreads();
+  const bool quads = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+  for (int at = threadIdx.x; at < RT * CT * EI_WAVE; at += 512) {
+    const int tile = at / EI_WAVE, l = at % EI_WAVE;
+    f32x4 c[kSegs];
+#pragma unroll
+    for (int s = 0; s < kSegs; ++s) c[s] = parts[s][tile][l];
+    const f32x4 sum = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
+    const int m = 16 * (tile / CT) + l % 16, n = n0 + 16 * (tile % CT) + 4 * (l / 16);
+    if (m >= M) continue;
+    float* dst = C + static_cast<size_t>(m) * ldc + n;
+    if (quads && n + 4 <= N) {
+      *reinterpret_cast<f32x4*>(dst) = sum;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < N) dst[e] = sum[e];
+    }
   }
 }
 
@@ -214,23 +316,47 @@ extern "C" int ei_gemm_f32(const float* A, const float* W, float* C, int M, int 
   EI_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32: sizes must be positive");
   EI_REQUIRE(A && W && C, "gemm_f32: null pointer");
   EI_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_f32: leading dimension too small");
-  // few rows: the weight-streaming kernel (16-byte loads: K and the leading dimensions in
-  // fours, pointers aligned)
+  // 16-byte loads: K and the leading dimensions in fours, pointers aligned
   const bool fours = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 &&
                      ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-  if (M <= 8 && fours) {
-    const unsigned blocks = static_cast<unsigned>((N + FN - 1) / FN);
-    if (M <= 4)
-      gemm_f32_few_rows_kernel<1><<<blocks, EI_WAVE, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc);
-    else
-      gemm_f32_few_rows_kernel<2><<<blocks, EI_WAVE, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc);
+  if (fours && M <= 64) {
+    // (two strips a block where the chip still gets eight blocks a unit)
+    const bool wide = (N + 31LL) / 32 >= 8LL * ei_compute_units();
+#define EI_FEW(RT, CT)                                                                   \
+  gemm_f32_few_kernel<RT, CT><<<static_cast<unsigned>((N + 16LL * CT - 1) / (16 * CT)), 512, 0, stream>>>( \
+      A, W, C, M, N, K, lda, ldw, ldc)
+    if (M <= 16) {
+      if (wide) EI_FEW(1, 2);
+      else EI_FEW(1, 1);
+    } else if (M <= 32) {
+      if (wide) EI_FEW(2, 2);
+      else EI_FEW(2, 1);
+    } else {
+      if (wide) EI_FEW(4, 2);
+      else EI_FEW(4, 1);
+    }
+#undef EI_FEW
     EI_LAUNCH_CHECK();
   }
-  if (M > 64 && fours) {
-    const long long rows = (M + GM - 1) / GM;
-    EI_REQUIRE(rows <= 65535, "gemm_f32: too many rows for one launch");
-    dim3 tiles((N + GN - 1) / GN, static_cast<unsigned>(rows));
-    gemm_f32_large_kernel<<<tiles, 256, 0, stream>>>(A, W, C, M, N, K, lda, ldw, ldc);
+  if (fours) {
+    // the largest tile that leaves no compute unit without a block
+    const long long units = ei_compute_units();
+    auto blocks_of = [&](int rt, int ct) {
+      return ((M + 16LL * rt - 1) / (16 * rt)) * ((N + 16LL * ct - 1) / (16 * ct));
+    };
+    auto grid_of = [&](int rt, int ct) {
+      const long long rows = (M + 16LL * rt - 1) / (16 * rt), cols = (N + 16LL * ct - 1) / (16 * ct);
+      return rows * (rows <= kFewRowTiles ? (cols + 7) / 8 * 8 : cols);
+    };
+    EI_REQUIRE(grid_of(2, 2) <= 0x7fffffff || blocks_of(4, 4) <= 0x7ffffff0,
+               "gemm_f32: too many outputs for one launch");
+#define EI_TILE(RT, CT)                                                                     \
+  gemm_f32_tile_kernel<RT, CT><<<static_cast<unsigned>(grid_of(RT, CT)), 256, 0, stream>>>( \
+      A, W, C, M, N, K, lda, ldw, ldc, (N + 16 * CT - 1) / (16 * CT))
+    if (blocks_of(4, 4) >= units) EI_TILE(4, 4);
+    else if (blocks_of(2, 4) >= units) EI_TILE(2, 4);
+    else EI_TILE(2, 2);
+#undef EI_TILE
     EI_LAUNCH_CHECK();
   }
   const long long gy = (M + BM - 1) / BM;
