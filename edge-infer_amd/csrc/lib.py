@@ -73,6 +73,11 @@ _SIGNATURES = {
         "ei_ssm_scan": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p,
                         c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p,
                         c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+        "ei_ssm_chunk_floats": [c_int, c_int],
+        "ei_ssm_chunks": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p,
+                          c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p,
+                          c_void_p, c_void_p, c_void_p, c_longlong, c_int, c_int, c_int, c_int,
+                          c_int, c_int, c_int, c_int, c_void_p],
         "ei_ssm_out": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p,
                        c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     },
@@ -95,6 +100,10 @@ _SIGNATURES = {
         "ei_la_scan": [c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p, c_void_p,
                        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                        c_int, c_int, c_void_p],
+        "ei_la_chunk_floats": [c_int, c_int],
+        "ei_la_chunks": [c_void_p, c_longlong, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                         c_void_p, c_void_p, c_void_p, c_longlong, c_int, c_int, c_int, c_int,
+                         c_int, c_int, c_void_p],
         "ei_la_activate": [c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p, c_int, c_int,
                            c_void_p],
         "ei_la_out": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_longlong, c_longlong,
@@ -178,6 +187,10 @@ _SIGNATURES = {
     "mlstm": {
         "ei_mlstm_state_floats": [c_int, c_int, c_int],
         "ei_mlstm_proj_width": [c_int, c_int, c_int],
+        "ei_mlstm_chunk_floats": [c_int, c_int],
+        "ei_mlstm_chunks": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p,
+                            c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_longlong, c_int,
+                            c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_void_p],
         "ei_mlstm_walk": [c_void_p, c_int, c_int, c_longlong, c_void_p, c_void_p, c_void_p,
                           c_longlong, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                           c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_void_p],
@@ -1088,6 +1101,40 @@ def mlstm_walk(proj, i_bias, f_bias, state, seq_in, seq_out, seq_count, seq_row0
     _check(lib, status, "mlstm_walk")
 
 
+def mlstm_chunk_scratch(rows, seqs, heads, key_dim, value_dim) -> int:
+    """float32 elements of scratch that `mlstm_chunks` wants for a step of so many rows."""
+    return _chunk_scratch("mlstm", "ei_mlstm_chunk_floats", rows, seqs, heads, key_dim, value_dim)
+
+
+def mlstm_chunks(proj, i_bias, f_bias, state, seq_in, seq_out, seq_count, seq_row0, o_raw, scratch,
+                 heads, key_dim, value_dim, cap, q_scale, bottom_eps, longest: int) -> None:
+    """What `mlstm_walk` does, by chunks of 64 tokens: heads of 64 or 128 elements, a projection
+    [rows, width] in one piece whose width is a multiple of 4; longest: the most rows that a
+    sequence of the step brings."""
+    lib = library("mlstm")
+    n, width, nsplit, _ = _rows_of(proj, "proj")
+    if nsplit != 1 or width != mlstm_proj_width(heads, key_dim, value_dim):
+        raise KernelError("mlstm_chunks: the projection's shape does not fit")
+    if state.dim() != 2 or state.shape[1] < mlstm_state_floats(heads, key_dim, value_dim):
+        raise KernelError("mlstm_chunks: state rows too short")
+    n_seqs = seq_count.numel()
+    if seq_in.numel() < n_seqs or seq_out.numel() < n_seqs or seq_row0.numel() < n_seqs:
+        raise KernelError("mlstm_chunks: sequence metadata shorter than the sequences")
+    if tuple(o_raw.shape) != (n, heads * value_dim):
+        raise KernelError("mlstm_chunks: o_raw must be [rows, heads * value_dim]")
+    if i_bias.numel() != heads or f_bias.numel() != heads:
+        raise KernelError("mlstm_chunks: one gate bias a head")
+    status = lib.ei_mlstm_chunks(
+        _gpu(proj, "proj"), _code(proj, "proj"), _gpu(i_bias, "i_bias", torch.float32),
+        _gpu(f_bias, "f_bias", torch.float32), _gpu(state, "state", torch.float32), state.shape[1],
+        _gpu(seq_in, "seq_in", torch.int32), _gpu(seq_out, "seq_out", torch.int32),
+        _gpu(seq_count, "seq_count", torch.int32), _gpu(seq_row0, "seq_row0", torch.int32),
+        _gpu(o_raw, "o_raw", torch.float32), _gpu(scratch, "scratch", torch.float32),
+        scratch.numel(), n, n_seqs, heads, key_dim, value_dim, float(cap), float(q_scale),
+        float(bottom_eps), int(longest), _stream())
+    _check(lib, status, "mlstm_chunks")
+
+
 def mlstm_out(o_raw, proj, norm_w, eps, row_seq, out, heads, key_dim, value_dim) -> None:
     """out = rmsnorm per head (o_raw) * norm_w [heads * value_dim] * sigmoid(gate columns of
     proj), in out's type."""
@@ -1783,6 +1830,38 @@ def ssm_scan(conv, proj, a_log, dt_bias, d_skip, state, shape: SsmShape, seq_in,
     _check(lib, status, "ssm_scan")
 
 
+def ssm_chunk_scratch(rows, seqs, shape: SsmShape) -> int:
+    """float32 elements of scratch that `ssm_chunks` wants for a step of so many rows."""
+    return _chunk_scratch("ssm", "ei_ssm_chunk_floats", rows, seqs, shape.heads, shape.head_dim, shape.state)
+
+
+def ssm_chunks(conv, proj, a_log, dt_bias, d_skip, state, shape: SsmShape, seq_in, seq_out,
+               seq_count, seq_row0, y_raw, scratch, longest: int) -> None:
+    """What `ssm_scan` does, by chunks of 64 tokens: states of 64 or 128 rows and columns;
+    longest: the most rows that a sequence of the step brings."""
+    lib = library("ssm")
+    n = y_raw.shape[0]
+    nsplit, stride = _ssm_proj(proj, n, shape)
+    n_seqs = seq_in.numel()
+    if tuple(conv.shape) != (n, shape.channels) or tuple(y_raw.shape) != (n, shape.inner):
+        raise KernelError("ssm_chunks: conv or y_raw has the wrong shape")
+    for name, per_head in (("a_log", a_log), ("dt_bias", dt_bias), ("d_skip", d_skip)):
+        if per_head.numel() != shape.heads:
+            raise KernelError(f"ssm_chunks: {name} must have one value a head")
+    if min(seq_out.numel(), seq_count.numel(), seq_row0.numel()) < n_seqs:
+        raise KernelError("ssm_chunks: metadata shorter than the step")
+    status = lib.ei_ssm_chunks(
+        _gpu(conv, "conv", torch.float32), _gpu(proj, "proj"), _code(proj, "proj"), nsplit, stride,
+        shape.proj_width, _gpu(a_log, "a_log", torch.float32),
+        _gpu(dt_bias, "dt_bias", torch.float32), _gpu(d_skip, "d_skip", torch.float32),
+        _ssm_state(state, shape), state.shape[1], _gpu(seq_in, "seq_in", torch.int32),
+        _gpu(seq_out, "seq_out", torch.int32), _gpu(seq_count, "seq_count", torch.int32),
+        _gpu(seq_row0, "seq_row0", torch.int32), _gpu(y_raw, "y_raw", torch.float32),
+        _gpu(scratch, "scratch", torch.float32), scratch.numel(), n, n_seqs, *shape.sizes,
+        int(longest), _stream())
+    _check(lib, status, "ssm_chunks")
+
+
 def ssm_out(y_raw, proj, norm_w, eps, shape: SsmShape, parts, row_seq, out) -> None:
     """out [n, inner] = rmsnorm over each of `parts` equal parts of (y_raw * silu(z)) * norm_w,
     z the first `inner` columns of `proj`."""
@@ -1951,6 +2030,46 @@ def input_conv(h, weight, state, part: int, parts: int, row_pos, row_seq, seq_in
         _gpu(seq_start, "seq_start", torch.int32), _gpu(seq_count, "seq_count", torch.int32),
         _gpu(seq_row0, "seq_row0", torch.int32), _gpu(out, "out"), n, width, n_seqs, _stream())
     _check(lib, status, "input_conv")
+
+
+# Recurrences by chunks of a prompt's tokens (csrc/recurrence_chunks.h): the scratch that the
+# chunks' states take, and the head sizes that the kernels know.
+CHUNK_TOKENS = 64
+CHUNK_SIZES = (64, 128)
+
+
+def _chunk_scratch(library_name: str, symbol: str, rows: int, seqs: int, heads: int, dk: int,
+                   dv: int) -> int:
+    each = getattr(library(library_name), symbol)(dk, dv)
+    return (rows // CHUNK_TOKENS + seqs) * heads * each
+
+
+def la_chunk_scratch(rows, seqs, heads, key_dim, value_dim) -> int:
+    """float32 elements of scratch that `la_chunks` wants for a step of so many rows."""
+    return _chunk_scratch("linear_attention", "ei_la_chunk_floats", rows, seqs, heads, key_dim, value_dim)
+
+
+def la_chunks(act, decay, state, seq_in, seq_out, seq_count, seq_row0, o_raw, scratch, heads,
+              key_dim, value_dim, longest: int) -> None:
+    """What `la_scan` does with activated rows, by chunks of 64 tokens: heads of 64 or 128
+    elements; longest: the most rows that a sequence of the step brings."""
+    lib = library("linear_attention")
+    n, stride = act.shape
+    n_seqs = seq_count.numel()
+    if tuple(o_raw.shape) != (n, heads * value_dim) or decay.numel() != heads:
+        raise KernelError("la_chunks: shapes do not fit")
+    if state.dim() != 2 or state.shape[1] != la_state_floats(heads, key_dim, value_dim):
+        raise KernelError("la_chunks: state rows must hold heads * key_dim * value_dim floats")
+    if seq_in.numel() < n_seqs or seq_out.numel() < n_seqs or seq_row0.numel() < n_seqs:
+        raise KernelError("la_chunks: sequence metadata shorter than the sequences")
+    status = lib.ei_la_chunks(
+        _gpu(act, "act", torch.float32), stride, _gpu(decay, "decay", torch.float32),
+        _gpu(state, "state", torch.float32), _gpu(seq_in, "seq_in", torch.int32),
+        _gpu(seq_out, "seq_out", torch.int32), _gpu(seq_count, "seq_count", torch.int32),
+        _gpu(seq_row0, "seq_row0", torch.int32), _gpu(o_raw, "o_raw", torch.float32),
+        _gpu(scratch, "scratch", torch.float32), scratch.numel(), n, n_seqs, heads, key_dim,
+        value_dim, int(longest), _stream())
+    _check(lib, status, "la_chunks")
 
 
 def la_state_floats(heads: int, key_dim: int, value_dim: int) -> int:

@@ -11,6 +11,7 @@
 // holds (a whole prompt, a portion, one token), so a position's result does not depend on how
 // its sequence was cut.
 #include "common.h"
+#include "recurrence_chunks.h"
 
 namespace {
 
@@ -281,5 +282,38 @@ extern "C" int ei_la_out(const float* o_raw, const void* proj, int proj_dtype, i
   else if (proj_dtype == EI_BF16 && out_dtype == EI_BF16) EI_LO(bf16_t, bf16_t);
   else EI_REQUIRE(false, "la_out: unsupported dtype combination");
 #undef EI_LO
+  EI_LAUNCH_CHECK();
+}
+
+// The recurrence over a prompt's rows in chunks (see recurrence_chunks.h).  act: float32 [N,
+// row_stride] with q, k and v as `ei_la_activate` leaves them; scratch: `scratch_floats` floats, at
+// least (N / 64 + n_seqs) * H chunks; longest: the most rows that a sequence brings.
+extern "C" int ei_la_chunk_floats(int DK, int DV) {
+  return static_cast<int>(ei::chunks::chunk_floats(ei::chunks::kFixed, DK, DV));
+}
+
+extern "C" int ei_la_chunks(const float* act, long long row_stride, const float* decay, float* state,
+                            const int32_t* seq_in, const int32_t* seq_out, const int32_t* seq_count,
+                            const int32_t* seq_row0, float* o_raw, float* scratch,
+                            long long scratch_floats, int N, int n_seqs, int H, int DK, int DV,
+                            int longest, hipStream_t stream) {
+  EI_REQUIRE(act && decay && state && seq_in && seq_out && seq_count && seq_row0 && o_raw && scratch,
+             "la_chunks: null pointer");
+  EI_REQUIRE(N > 0 && n_seqs > 0 && H > 0 && longest > 0 && longest <= N, "la_chunks: sizes must be positive");
+  EI_REQUIRE(ei::chunks::sizes_fit(DK, DV), "la_chunks: heads of 64 or 128 elements");
+  EI_REQUIRE(row_stride >= 2LL * H * DK + 1LL * H * DV && row_stride % 4 == 0 &&
+                 (reinterpret_cast<uintptr_t>(act) & 15) == 0 && (reinterpret_cast<uintptr_t>(scratch) & 15) == 0,
+             "la_chunks: rows narrower than q, k and v, or unaligned");
+  EI_REQUIRE(H <= 65535 && n_seqs <= 65535, "la_chunks: too many heads or sequences");
+  EI_REQUIRE(scratch_floats >= (N / 64 + 1LL * n_seqs) * H * ei_la_chunk_floats(DK, DV),
+             "la_chunks: scratch too small");
+  using namespace ei::chunks;
+  const Rows at_row{static_cast<size_t>(row_stride), 0, H * DK, 2 * H * DK, 1};
+  Gates gates{};
+  gates.c0 = decay;
+  const State table{state, static_cast<size_t>(H) * DK * DV, static_cast<size_t>(DK) * DV};
+  const Sequences seqs{seq_in, seq_out, seq_count, seq_row0};
+  launch_sized<kFixed, float>(DK, DV, act, at_row, gates, table, seqs, scratch, o_raw, n_seqs, H,
+                              longest, stream);
   EI_LAUNCH_CHECK();
 }

@@ -26,6 +26,7 @@
 // `mlstm_out`: a wave a (row, head): RMS norm of the read-out, a weight as wide as all heads,
 // a sigmoid gate from the projection, one rounding.
 #include "common.h"
+#include "recurrence_chunks.h"
 
 namespace {
 
@@ -466,6 +467,61 @@ extern "C" int ei_mlstm_walk(const void* proj, int dtype, int nsplit, long long 
   else EI_REQUIRE(false, "mlstm_walk: unknown dtype");
 #undef EI_WALK_COLS
 #undef EI_WALK
+  EI_LAUNCH_CHECK();
+}
+
+// The walk over a prompt's rows in chunks (see recurrence_chunks.h): what `ei_mlstm_walk` does for
+// heads of 64 or 128 elements and a projection in one piece whose rows are multiples of 4
+// elements.  scratch: `scratch_floats` floats, at least (rows / 64 + n_seqs) * heads chunks;
+// longest: the most rows that a sequence brings.
+extern "C" int ei_mlstm_chunk_floats(int dim, int vdim) {
+  return static_cast<int>(ei::chunks::chunk_floats(ei::chunks::kMatrix, dim, vdim));
+}
+
+extern "C" int ei_mlstm_chunks(const void* proj, int dtype, const float* i_bias, const float* f_bias,
+                               float* state, long long state_stride, const int32_t* seq_in,
+                               const int32_t* seq_out, const int32_t* seq_count,
+                               const int32_t* seq_row0, float* o_raw, float* scratch,
+                               long long scratch_floats, int rows, int n_seqs, int heads, int dim,
+                               int vdim, float cap, float q_scale, float bottom_eps, int longest,
+                               hipStream_t stream) {
+  EI_REQUIRE(n_seqs > 0 && heads > 0 && rows >= 1 && longest >= 1 && longest <= rows, "mlstm_chunks: bad sizes");
+  EI_REQUIRE(ei::chunks::sizes_fit(dim, vdim), "mlstm_chunks: heads of 64 or 128 elements");
+  EI_REQUIRE(cap > 0.f, "mlstm_chunks: the cap of the gates must be positive");
+  EI_REQUIRE(proj && i_bias && f_bias && state && seq_in && seq_out && seq_count && seq_row0 && o_raw &&
+                 scratch,
+             "mlstm_chunks: null pointer");
+  EI_REQUIRE(dtype == EI_F32 || dtype == EI_BF16, "mlstm_chunks: unknown dtype");
+  EI_REQUIRE(state_stride >= ei_mlstm_state_floats(heads, dim, vdim), "mlstm_chunks: state rows too short");
+  const Columns col_of = columns_of(heads, dim, vdim);
+  EI_REQUIRE(col_of.width % 4 == 0 && (reinterpret_cast<uintptr_t>(proj) & 15) == 0 &&
+                 (reinterpret_cast<uintptr_t>(scratch) & 15) == 0,
+             "mlstm_chunks: unaligned rows");
+  EI_REQUIRE(heads <= 65535 && n_seqs <= 65535, "mlstm_chunks: too many heads or sequences");
+  EI_REQUIRE(scratch_floats >= (rows / 64 + 1LL * n_seqs) * heads * ei_mlstm_chunk_floats(dim, vdim),
+             "mlstm_chunks: scratch too small");
+  using namespace ei::chunks;
+  const Rows at_row{static_cast<size_t>(col_of.width), col_of.q, col_of.k, col_of.v, 1};
+  Gates gates{};
+  gates.c0 = i_bias;
+  gates.c1 = f_bias;
+  gates.raw = proj;
+  gates.raw_bf16 = dtype == EI_BF16;
+  gates.nsplit = 1;
+  gates.stride = static_cast<size_t>(col_of.width);
+  gates.at = col_of.i;
+  gates.at2 = col_of.f;
+  gates.cap = cap;
+  gates.q_scale = q_scale;
+  gates.bottom_eps = bottom_eps;
+  const State table{state, static_cast<size_t>(state_stride), head_state_floats(dim, vdim)};
+  const Sequences seqs{seq_in, seq_out, seq_count, seq_row0};
+  if (dtype == EI_F32)
+    launch_sized<kMatrix, float>(dim, vdim, static_cast<const float*>(proj), at_row, gates, table, seqs,
+                                 scratch, o_raw, n_seqs, heads, longest, stream);
+  else
+    launch_sized<kMatrix, bf16_t>(dim, vdim, static_cast<const bf16_t*>(proj), at_row, gates, table,
+                                  seqs, scratch, o_raw, n_seqs, heads, longest, stream);
   EI_LAUNCH_CHECK();
 }
 

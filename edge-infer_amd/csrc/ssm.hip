@@ -15,6 +15,7 @@
 // writes the whole row `seq_out` names, so a prompt may come whole, in portions or token by
 // token, and a step that fails changes nothing.
 #include "common.h"
+#include "recurrence_chunks.h"
 
 namespace {
 
@@ -437,6 +438,52 @@ extern "C" int ei_ssm_scan(const float* conv, const void* proj, int in_dtype, in
   else EI_REQUIRE(false, "ssm_scan: unknown dtype");
 #undef EI_SSM_SCAN
 #undef EI_SSM_SCAN_AS
+  EI_LAUNCH_CHECK();
+}
+
+// The recurrence over a prompt's rows in chunks (see recurrence_chunks.h): what `ei_ssm_scan` does
+// for states of 64 or 128 rows and heads of 64 or 128 columns.  scratch: `scratch_floats` floats, at
+// least (N / 64 + n_seqs) * heads chunks; longest: the most rows that a sequence brings.
+extern "C" int ei_ssm_chunk_floats(int P, int Nst) {
+  return static_cast<int>(ei::chunks::chunk_floats(ei::chunks::kSelective, Nst, P));
+}
+
+extern "C" int ei_ssm_chunks(const float* conv, const void* proj, int in_dtype, int nsplit,
+                             long long split_stride, long long row_stride, const float* a_log,
+                             const float* dt_bias, const float* d_skip, float* state,
+                             long long state_stride, const int32_t* seq_in, const int32_t* seq_out,
+                             const int32_t* seq_count, const int32_t* seq_row0, float* y_raw,
+                             float* scratch, long long scratch_floats, int N, int n_seqs, int heads,
+                             int groups, int P, int Nst, int taps, int longest, hipStream_t stream) {
+  EI_SSM_SHAPE("ssm_chunks");
+  EI_REQUIRE(conv && proj && a_log && dt_bias && d_skip && state && seq_in && seq_out && seq_count &&
+                 seq_row0 && y_raw && scratch && n_seqs > 0 && nsplit >= 1 && N > 0 && longest > 0 &&
+                 longest <= N,
+             "ssm_chunks: bad arguments");
+  EI_REQUIRE(ei::chunks::sizes_fit(Nst, P), "ssm_chunks: states of 64 or 128 rows and columns");
+  EI_REQUIRE(in_dtype == EI_F32 || in_dtype == EI_BF16, "ssm_chunks: unknown dtype");
+  EI_REQUIRE((reinterpret_cast<uintptr_t>(conv) & 15) == 0 && (reinterpret_cast<uintptr_t>(scratch) & 15) == 0,
+             "ssm_chunks: unaligned rows");
+  EI_REQUIRE(heads <= 65535 && n_seqs <= 65535, "ssm_chunks: too many heads or sequences");
+  EI_REQUIRE(scratch_floats >= (N / 64 + 1LL * n_seqs) * heads * ei_ssm_chunk_floats(P, Nst),
+             "ssm_chunks: scratch too small");
+  using namespace ei::chunks;
+  // C is the query, B the key, x the value
+  const Rows at_row{static_cast<size_t>(C), inner + groups * Nst, inner, 0, heads / groups};
+  Gates gates{};
+  gates.c0 = a_log;
+  gates.c1 = dt_bias;
+  gates.c2 = d_skip;
+  gates.raw = proj;
+  gates.raw_bf16 = in_dtype == EI_BF16;
+  gates.nsplit = nsplit;
+  gates.split_stride = static_cast<size_t>(split_stride);
+  gates.stride = static_cast<size_t>(row_stride);
+  gates.at = inner + C;
+  const State table{state, static_cast<size_t>(state_stride), static_cast<size_t>(P) * Nst};
+  const Sequences seqs{seq_in, seq_out, seq_count, seq_row0};
+  launch_sized<kSelective, float>(Nst, P, conv, at_row, gates, table, seqs, scratch, y_raw, n_seqs,
+                                  heads, longest, stream);
   EI_LAUNCH_CHECK();
 }
 

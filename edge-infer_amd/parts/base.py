@@ -274,3 +274,7 @@ class StepContext:
         workspace's are ignored."""
         for which in buffers:
             self.workspace.release(which)
+
+    def longest(self) -> int:
+        """The most tokens that a sequence brings in this step (host value)."""
+        return max((seq.count for seq in self.sequences), default=0)

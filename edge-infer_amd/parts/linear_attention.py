@@ -27,6 +27,10 @@ from .linear import Linear
 
 class LinearAttention:
     ACTIVATE_ROWS = 64       # from so many rows of a prompt step on, q, k and v are activated aside
+    # from so many tokens of one sequence on, by chunks and not token by token (16 heads of 128 x
+    # 128: 64 tokens of one sequence 20 us by tokens and 30 by chunks, 8 x 512 398 and 131, 2,048
+    # 785 and 77)
+    CHUNK_FROM = 96
 
     @property
     def capture_safe(self):
@@ -78,6 +82,8 @@ class LinearAttention:
             device=device, dtype=torch.float32).contiguous()
         self.out_norm = params["out_norm.weight"].to(device=device, dtype=torch.float32).contiguous()
         self.gate_column = 2 * spec.qk_width + spec.v_width
+        self.chunks_fit = (spec.key_dim in lib.CHUNK_SIZES and spec.value_dim in lib.CHUNK_SIZES
+                           and all(d >= 0.0 for d in spec.decay))
 
     def forward(self, ctx, x, entry):
         if not entry.writes_cache:
@@ -94,9 +100,15 @@ class LinearAttention:
             rows = ctx.buffer("la.act", (n, self.gate_column), torch.float32)
             lib.la_activate(proj, rows)
             activated = True
-        lib.la_scan(rows, self.decay, state, meta.seq_state_in, meta.seq_state_out, meta.seq_count,
-                    meta.seq_row0, o_raw, spec.n_heads, spec.key_dim, spec.value_dim,
-                    activated=activated)
+        sequences = (meta.seq_state_in, meta.seq_state_out, meta.seq_count, meta.seq_row0)
+        sizes = (spec.n_heads, spec.key_dim, spec.value_dim)
+        longest = ctx.longest() if activated and self.chunks_fit else 0
+        if longest >= self.CHUNK_FROM:
+            scratch = ctx.buffer("la.chunks", (lib.la_chunk_scratch(n, ctx.n_seqs, *sizes),), torch.float32)
+            lib.la_chunks(rows, self.decay, state, *sequences, o_raw, scratch, *sizes, longest)
+            ctx.release(scratch)
+        else:
+            lib.la_scan(rows, self.decay, state, *sequences, o_raw, *sizes, activated=activated)
         if activated:
             ctx.release(rows)
         gated = ctx.buffer("la.gated", (n, spec.v_width))

@@ -40,6 +40,11 @@ class MatrixMemory:
     def capture_rows(self):
         return min(self.proj.capture_rows, self.o.capture_rows)
 
+    # from so many tokens of one sequence on, by chunks and not token by token (16 heads of 128 x
+    # 128 in bfloat16: 64 tokens of one sequence 48 us by tokens and 40 by chunks, 8 x 512 495 and
+    # 154, 2,048 1,300 and 92)
+    CHUNK_FROM = 64
+
     @classmethod
     def parameters(cls, spec, hidden):
         return {
@@ -88,6 +93,8 @@ class MatrixMemory:
         self.forget_bias = f32(params["forget_gate.bias"])
         self.out_norm = f32(params["out_norm.weight"])
         self.q_scale = float(spec.key_dim) ** -0.5
+        self.chunks_fit = (spec.key_dim in lib.CHUNK_SIZES and spec.value_dim in lib.CHUNK_SIZES
+                           and self.proj.out_features % 4 == 0)
 
     def forward(self, ctx, x, entry):
         if not entry.writes_cache:
@@ -97,9 +104,17 @@ class MatrixMemory:
         state = ctx.cache.state(entry.cache)                 # [2 (slots + 1), state floats]
         proj = self.proj.forward(ctx, x, "mlstm.proj")
         o_raw = ctx.buffer("mlstm.o_raw", (n, spec.v_width), torch.float32)
-        lib.mlstm_walk(proj, self.in_bias, self.forget_bias, state, meta.seq_state_in,
-                       meta.seq_state_out, meta.seq_count, meta.seq_row0, o_raw, spec.n_heads,
-                       spec.key_dim, spec.value_dim, spec.gate_cap, self.q_scale, spec.bottom_eps)
+        sequences = (meta.seq_state_in, meta.seq_state_out, meta.seq_count, meta.seq_row0)
+        sizes = (spec.n_heads, spec.key_dim, spec.value_dim)
+        how = (spec.gate_cap, self.q_scale, spec.bottom_eps)
+        longest = ctx.longest() if self.chunks_fit and not ctx.decode and proj.dim() == 2 else 0
+        if longest >= self.CHUNK_FROM:
+            scratch = ctx.buffer("mlstm.chunks", (lib.mlstm_chunk_scratch(n, ctx.n_seqs, *sizes),), torch.float32)
+            lib.mlstm_chunks(proj, self.in_bias, self.forget_bias, state, *sequences, o_raw, scratch,
+                             *sizes, *how, longest)
+            ctx.release(scratch)
+        else:
+            lib.mlstm_walk(proj, self.in_bias, self.forget_bias, state, *sequences, o_raw, *sizes, *how)
         gated = ctx.buffer("mlstm.gated", (n, spec.v_width))
         lib.mlstm_out(o_raw, proj, self.out_norm, spec.out_norm_eps, meta.row_seq, gated,
                       spec.n_heads, spec.key_dim, spec.value_dim)

@@ -57,6 +57,11 @@ class StateSpace:
             "o_proj.weight": ParamSpec((hidden, spec.inner)),
         }
 
+    # from so many tokens of one sequence on, by chunks and not token by token (16 heads of 128
+    # columns, state 128: 64 tokens of one sequence 30 us by tokens and 35 by chunks, 8 x 512 305
+    # and 143, 2,048 790 and 82)
+    CHUNK_FROM = 96
+
     @classmethod
     def cache_request(cls, spec):
         return StateRequest(shape=(cls.shape_of(spec).state_floats,), two_versions=True)
@@ -82,6 +87,7 @@ class StateSpace:
         self.check(spec)
         self.spec = spec
         self.shape = self.shape_of(spec)
+        self.chunks_fit = spec.state in lib.CHUNK_SIZES and spec.head_dim in lib.CHUNK_SIZES
         self.proj = Linear(params["in_proj.weight"], dtype, device)
         self.o = Linear(params["o_proj.weight"], dtype, device)
 
@@ -107,8 +113,15 @@ class StateSpace:
         lib.ssm_conv(proj, self.conv_w, self.conv_b, state, shape, meta.row_pos, meta.row_seq,
                      rows_in, rows_out, meta.seq_start, meta.seq_count, meta.seq_row0, conv)
         y_raw = ctx.buffer("ssm.y_raw", (n, shape.inner), torch.float32)
-        lib.ssm_scan(conv, proj, self.a_log, self.dt_bias, self.skip, state, shape, rows_in,
-                     rows_out, meta.seq_count, meta.seq_row0, y_raw)
+        constants = (self.a_log, self.dt_bias, self.skip)
+        sequences = (rows_in, rows_out, meta.seq_count, meta.seq_row0)
+        longest = ctx.longest() if self.chunks_fit and not ctx.decode else 0
+        if longest >= self.CHUNK_FROM:
+            scratch = ctx.buffer("ssm.chunks", (lib.ssm_chunk_scratch(n, ctx.n_seqs, shape),), torch.float32)
+            lib.ssm_chunks(conv, proj, *constants, state, shape, *sequences, y_raw, scratch, longest)
+            ctx.release(scratch)
+        else:
+            lib.ssm_scan(conv, proj, *constants, state, shape, *sequences, y_raw)
         ctx.release(conv)
         gated = ctx.buffer("ssm.gated", (n, shape.inner))
         lib.ssm_out(y_raw, proj, self.out_norm, self.spec.norm_eps, shape, self.spec.norm_parts,

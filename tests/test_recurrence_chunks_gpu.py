@@ -1,0 +1,199 @@
+"""Recurrences by chunks of 64 tokens against the token-by-token recurrence in float64, at the edges
+of chunks and of the head sizes, and models whose prompts take them against the walk."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+F64 = torch.float64
+DEV = "cuda"
+COUNTS = ([1, 64, 0, 65, 130, 63], [257])
+
+
+def recurrence(q, k, v, decay, take, state, counts):
+    """S_t = decay_t S_(t-1) + take_t k_t v_t^T, o_t = S_t^T q_t for sequences one behind the
+    other; `state` [sequences, H, d, e] becomes the last one.  All float64."""
+    out, row = torch.zeros(q.shape[0], q.shape[1], v.shape[2], dtype=F64), 0
+    for s, count in enumerate(counts):
+        for _ in range(count):
+            state[s] = (decay[row][:, None, None] * state[s]
+                        + take[row][:, None, None] * k[row][:, :, None] * v[row][:, None, :])
+            out[row] = (state[s] * q[row][:, :, None]).sum(dim=1)
+            row += 1
+    return out
+
+
+def metadata(counts):
+    """(rows read, rows written, counts, first rows): two versions a sequence, a spare between."""
+    starts = [sum(counts[:i]) for i in range(len(counts))]
+    make = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    n = len(counts)
+    return make([3 * i for i in range(n)]), make([3 * i + 1 for i in range(n)]), make(counts), make(starts)
+
+
+def off(got, want):
+    return ((got.double().cpu() - want).norm() / want.norm()).item()
+
+
+def check(rows, out, want, table, before, state, counts, tolerance):
+    assert not bool(torch.isnan(out).any())
+    assert off(out, want) <= tolerance
+    live = [s for s, c in enumerate(counts) if c]
+    assert off(table[[3 * s + 1 for s in live]][:, :state.shape[1]], state[live]) <= tolerance
+    kept = [r for r in range(table.shape[0]) if r not in {3 * s + 1 for s in live}]
+    assert torch.equal(table[kept], before[kept])       # nothing but the rows that are written
+
+
+# A sum of up to 192 products in four chains of float32 and a carry a chunk: some ten roundings on
+# the way of a typical term, each half of 2^-23 and of either sign; 16 of them in one direction
+# would be 1e-6.
+TOLERANCE = 1e-6
+
+
+@pytest.mark.parametrize("counts", COUNTS)
+@pytest.mark.parametrize("dk,dv", [(64, 64), (64, 128), (128, 64), (128, 128)])
+def test_fixed_decays(dk, dv, counts):
+    from edge_infer_amd.csrc import lib
+    H, rows = 3, sum(counts)
+    g = torch.Generator().manual_seed(dk + dv + rows)
+    act = torch.randn(rows, H * (2 * dk + dv), generator=g)
+    decay = torch.tensor([0.0, 0.9, 1.0])
+    table = torch.randn(3 * len(counts), H * dk * dv, generator=g)
+    state = table[0::3].double().view(len(counts), H, dk, dv).clone()
+    a = act.double()
+    want = recurrence(a[:, :H * dk].view(rows, H, dk), a[:, H * dk:2 * H * dk].view(rows, H, dk),
+                      a[:, 2 * H * dk:].view(rows, H, dv), decay.double().expand(rows, H),
+                      torch.ones(rows, H, dtype=F64), state, counts).reshape(rows, -1)
+    moved, out = table.to(DEV), torch.full((rows, H * dv), float("nan"), device=DEV)
+    scratch = torch.full((lib.la_chunk_scratch(rows, len(counts), H, dk, dv),), float("nan"), device=DEV)
+    lib.la_chunks(act.to(DEV), decay.to(DEV), moved, *metadata(counts), out, scratch, H, dk, dv, max(counts))
+    check(rows, out, want, moved.cpu(), table, state.reshape(len(counts), -1), counts, TOLERANCE)
+
+
+@pytest.mark.parametrize("counts", COUNTS)
+@pytest.mark.parametrize("P,N", [(64, 64), (128, 64), (64, 128), (128, 128)])
+@pytest.mark.parametrize("slices", [0, 2])
+def test_selective_decays(P, N, counts, slices):
+    """Steps from 1e-9 to 20 and more, whose decays reach from 1 to nothing within a chunk."""
+    from edge_infer_amd.csrc import lib
+    shape, rows = lib.SsmShape(4, 2, P, N, 4), sum(counts)
+    H, G = 4, 2
+    g = torch.Generator().manual_seed(P + N + rows)
+    conv = torch.randn(rows, shape.channels, generator=g)
+    proj = torch.randn(max(1, slices), rows, shape.proj_width, generator=g) * 8.0
+    if not slices:
+        proj = proj[0].to(torch.bfloat16)
+    dt_raw = (proj.double().sum(0) if slices else proj.double())[:, -H:]
+    a_log = torch.rand(H, generator=g) * 4.0 - 3.0
+    bias, skip = torch.rand(H, generator=g) - 2.0, torch.rand(H, generator=g)
+    dt = torch.nn.functional.softplus(dt_raw + bias.double())
+    decay = torch.exp(-torch.exp(a_log.double()) * dt)
+    table = torch.randn(3 * len(counts), shape.state_floats, generator=g)
+    state = table[0::3, :H * P * N].double().view(len(counts), H, P, N).transpose(2, 3).clone()
+    c = conv.double()
+    x = c[:, :H * P].view(rows, H, P)
+    B = c[:, H * P:H * P + G * N].view(rows, G, N).repeat_interleave(H // G, dim=1)
+    C = c[:, H * P + G * N:].view(rows, G, N).repeat_interleave(H // G, dim=1)
+    want = (recurrence(C, B, x, decay, dt, state, counts) + skip.double()[:, None] * x).reshape(rows, -1)
+    moved, out = table.to(DEV), torch.full((rows, H * P), float("nan"), device=DEV)
+    scratch = torch.full((lib.ssm_chunk_scratch(rows, len(counts), shape),), float("nan"), device=DEV)
+    lib.ssm_chunks(conv.to(DEV), proj.to(DEV), a_log.to(DEV), bias.to(DEV), skip.to(DEV), moved, shape,
+                   *metadata(counts), out, scratch, max(counts))
+    got = moved.cpu()
+    live = [3 * s + 1 for s, n in enumerate(counts) if n]
+    assert torch.equal(got[live][:, H * P * N:], table[live][:, H * P * N:])    # the tails are not its own
+    check(rows, out, want, got, table, state.transpose(2, 3).reshape(len(counts), -1), counts, TOLERANCE)
+
+
+@pytest.mark.parametrize("counts", COUNTS)
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 128), (128, 64), (64, 128)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_exponential_gates(dk, dv, counts, dtype):
+    from edge_infer_amd.csrc import lib
+    H, rows, cap, eps = 2, sum(counts), 15.0, 1e-6
+    g = torch.Generator().manual_seed(dk + dv + rows)
+    proj = torch.randn(rows, lib.mlstm_proj_width(H, dk, dv), generator=g)
+    at = 2 * H * dk + H * dv
+    proj[:, at:at + 2 * H] *= 6.0
+    proj = proj.to(dtype)
+    i_bias, f_bias = torch.randn(H, generator=g), torch.rand(H, generator=g) * 4.0
+    floats = lib.mlstm_state_floats(H, dk, dv)
+    table = torch.randn(3 * len(counts), floats, generator=g)
+    p = proj.double()
+    q = p[:, :H * dk].view(rows, H, dk) * dk ** -0.5
+    k, v = p[:, H * dk:2 * H * dk].view(rows, H, dk), p[:, 2 * H * dk:at].view(rows, H, dv)
+    log_in = cap * torch.tanh((p[:, at:at + H] + i_bias.double()) / cap)
+    log_forget = torch.nn.functional.logsigmoid(cap * torch.tanh((p[:, at + H:at + 2 * H] + f_bias.double()) / cap))
+    want, state, row = torch.zeros(rows, H, dv, dtype=F64), table[0::3].double(), 0
+    heads = state.view(len(counts), H, floats // H)
+    for s, count in enumerate(counts):
+        S = heads[s, :, :dk * dv].reshape(H, dv, dk).transpose(1, 2).clone()
+        n, m = heads[s, :, dk * dv:dk * dv + dk].clone(), heads[s, :, dk * dv + dk].clone()
+        for _ in range(count):
+            new = torch.maximum(log_forget[row] + m, log_in[row])
+            keep, take = torch.exp(log_forget[row] + m - new), torch.exp(log_in[row] - new)
+            S = keep[:, None, None] * S + take[:, None, None] * k[row][:, :, None] * v[row][:, None, :]
+            n, m = keep[:, None] * n + take[:, None] * k[row], new
+            bottom = torch.maximum((n * q[row]).sum(-1).abs(), torch.exp(-m)) + eps
+            want[row] = (S * q[row][:, :, None]).sum(dim=1) / bottom[:, None]
+            row += 1
+        heads[s, :, :dk * dv], heads[s, :, dk * dv:dk * dv + dk] = S.transpose(1, 2).reshape(H, -1), n
+        heads[s, :, dk * dv + dk] = m
+    moved, out = table.to(DEV), torch.full((rows, H * dv), float("nan"), device=DEV)
+    scratch = torch.full((lib.mlstm_chunk_scratch(rows, len(counts), H, dk, dv),), float("nan"), device=DEV)
+    lib.mlstm_chunks(proj.to(DEV), i_bias.to(DEV), f_bias.to(DEV), moved, *metadata(counts), out, scratch,
+                     H, dk, dv, cap, dk ** -0.5, eps, max(counts))
+    got = moved.cpu()
+    pad = dk * dv + dk + 1                              # (what pads a head's state is not written)
+    for s, count in enumerate(counts):
+        if count:
+            got[3 * s + 1].view(H, -1)[:, pad:] = state[s].view(H, -1)[:, pad:].float()
+    # logarithms up to 15 are rounded to float32 before their exponentials (1e-6 of the weight);
+    # a denominator that nearly vanishes enlarges its row's error, so rows are compared by their median
+    row_off = ((out.double().cpu() - want.view(rows, -1)).norm(dim=1) / want.view(rows, -1).norm(dim=1))
+    assert row_off.median().item() <= 4e-6 and off(got[1::3][[s for s, c in enumerate(counts) if c]],
+                                                   state[[s for s, c in enumerate(counts) if c]]) <= 4e-6
+    assert not bool(torch.isnan(out).any())
+
+
+def designs():
+    ff = {"kind": "dense", "ff": 64}
+    yield {"architecture": "Zadenex", "vocab": 97, "width": 64, "norm": {"eps": 1e-6},
+           "embedding": {"scale": 1.0}, "residual_mult": 0.5, "loop": None,
+           "layers": [{"type": "mlstm", "mixer": {"heads": 2, "dim": 64, "vdim": 128, "gate_cap": 15.0},
+                       "mlp": ff}]}
+    yield {"architecture": "Vafepel", "vocab": 97, "width": 64, "norm": {"eps": 1e-6}, "logit_scale": 1.0,
+           "logit_softcap": 30.0,
+           "layers": [{"type": "mamba2", "mixer": {"heads": 2, "vdim": 64, "state": 128, "groups": 2,
+                                                   "conv": 4, "norm_groups": 2},
+                       "mlp": {"kind": "dense", "ff": 64, "limit": 7.0}}]}
+    left = {"heads": 2, "kv_heads": 1, "dim": 64, "vdim": 64, "scale": 0.125}
+    yield {"architecture": "Gopuzen", "vocab": 97, "width": 64, "norm": {"eps": 1e-6},
+           "embedding": {"scale": 1.0}, "canon": {"taps": 2},
+           "layers": [{"type": "parallel", "mlp": ff,
+                       "mixer": {"left": left, "right": {"heads": 2, "dim": 64, "vdim": 128,
+                                                         "decay": [0.99, 0.9]}}}]}
+
+
+@pytest.mark.parametrize("cfg", designs(), ids=lambda c: c["architecture"])
+def test_a_prompt_whole_and_in_portions(cfg):
+    """A prompt of 200 tokens beside one of 5 (by chunks), the same in portions of at most 40 tokens
+    (token by token), and a token after it: float32 logits within what two orders of float32 sums
+    differ by (some 50 sums of a few roundings each)."""
+    import edge_infer_amd as ei
+    from edge_infer_amd.config import resolve_architecture
+    model = ei.random_model(resolve_architecture(cfg).config_class.from_dict(cfg), seed=4, dtype="float32")
+    g = torch.Generator().manual_seed(9)
+    ids = [torch.randint(0, 97, (n,), generator=g).tolist() for n in (201, 6)]
+
+    def logits(portion):
+        session = ei.Session(model, max_tokens=1024, max_seqs=2)
+        slots, out = [session.begin(), session.begin()], []
+        for at in range(0, 200, portion):
+            entries = [(s, i[at:min(at + portion, len(i) - 1)], [min(portion, len(i) - 1 - at) - 1])
+                       for s, i in zip(slots, ids) if at < len(i) - 1]
+            out.append(session.step(entries))
+        out.append(session.step([(s, i[-1:], [0]) for s, i in zip(slots, ids)]))
+        return torch.cat([out[-2][:1], out[-1]])
+    whole, cut = logits(200), logits(40)
+    assert ((whole - cut).norm() / cut.norm()).item() <= 1e-5
