@@ -29,6 +29,7 @@
 //   delta_out    the read-out's norm and gate
 #include "common.h"
 #include "few_rows.h"
+#include "delta_chunks.h"
 
 namespace {
 
@@ -1016,6 +1017,59 @@ extern "C" int ei_delta_rule(const float* conv, int OW, int key_decay, const voi
 
 // proj: [nsplit] slices of rows WP wide whose gate logits begin at gate_col; sigmoid_gate: the gate
 // is their sigmoid, not their silu.
+// The recurrence with one decay a head over a prompt's rows in chunks (see delta_chunks.h), for
+// heads of 64 or 128 elements.  scratch: `scratch_floats` floats, at least (rows / 64 + n_seqs) * H
+// chunks; longest: the most rows that a sequence brings.
+extern "C" int ei_delta_chunk_floats(int D, int DV) { return ei::delta_chunks::chunk_floats(D, DV); }
+
+extern "C" int ei_delta_chunks(const float* conv, int OW, const void* proj, int in_dtype, int nsplit,
+                               long long split_stride, int WP, int beta_col, int decay_col,
+                               const float* a_log, const float* dt_bias, float* state,
+                               long long state_stride, const int32_t* seq_in,
+                               const int32_t* seq_out, const int32_t* seq_count,
+                               const int32_t* seq_row0, float* o_raw, float* scratch,
+                               long long scratch_floats, int rows, int n_seqs, int H, int G, int D,
+                               int DV, float q_scale, float unit_eps, int longest,
+                               hipStream_t stream) {
+  EI_REQUIRE(conv && proj && a_log && dt_bias && state && seq_in && seq_out && seq_count && seq_row0 &&
+                 o_raw && scratch,
+             "delta_chunks: null pointer");
+  EI_REQUIRE(rows > 0 && n_seqs > 0 && H > 0 && G > 0 && H % G == 0 && nsplit >= 1 && longest > 0 &&
+                 longest <= rows,
+             "delta_chunks: bad sizes");
+  EI_REQUIRE(ei::delta_chunks::sizes_fit(D, DV), "delta_chunks: heads of 64 or 128 elements");
+  EI_REQUIRE(in_dtype == EI_F32 || in_dtype == EI_BF16, "delta_chunks: unknown dtype");
+  EI_REQUIRE(OW % 4 == 0 && OW >= 2 * G * D + H * DV && state_stride % 4 == 0 &&
+                 ((reinterpret_cast<uintptr_t>(conv) | reinterpret_cast<uintptr_t>(scratch) |
+                   reinterpret_cast<uintptr_t>(state)) & 15) == 0,
+             "delta_chunks: rows too narrow or unaligned");
+  EI_REQUIRE(H <= 65535 && n_seqs <= 65535 && (longest + 63) / 64 <= 65535,
+             "delta_chunks: too many heads, sequences or rows");
+  EI_REQUIRE(scratch_floats >= (rows / 64 + 1LL * n_seqs) * H * ei_delta_chunk_floats(D, DV),
+             "delta_chunks: scratch too small");
+  namespace dc = ei::delta_chunks;
+  const dc::Rows in{conv, static_cast<size_t>(OW), 0, G * D, 2 * G * D, H / G, q_scale, unit_eps};
+  ei::chunks::Gates gates{};
+  gates.c0 = a_log;
+  gates.c1 = dt_bias;
+  gates.raw = proj;
+  gates.raw_bf16 = in_dtype == EI_BF16;
+  gates.nsplit = nsplit;
+  gates.split_stride = static_cast<size_t>(split_stride);
+  gates.stride = static_cast<size_t>(WP);
+  gates.at = beta_col;
+  gates.at2 = decay_col;
+  const ei::chunks::State table{state, static_cast<size_t>(state_stride), static_cast<size_t>(D) * DV};
+  const ei::chunks::Sequences seqs{seq_in, seq_out, seq_count, seq_row0};
+#define EI_DC(DK_, DV_) dc::launch<DK_, DV_>(in, gates, table, seqs, scratch, o_raw, n_seqs, H, longest, stream)
+  if (D == 128 && DV == 128) EI_DC(128, 128);
+  else if (D == 128) EI_DC(128, 64);
+  else if (DV == 128) EI_DC(64, 128);
+  else EI_DC(64, 64);
+#undef EI_DC
+  EI_LAUNCH_CHECK();
+}
+
 extern "C" int ei_delta_out(const float* o_raw, const void* proj, int in_dtype, int nsplit,
                             long long split_stride, int WP, int gate_col, int sigmoid_gate,
                             const float* norm_w, float eps, const int32_t* row_seq, void* out, int out_dtype, int N,

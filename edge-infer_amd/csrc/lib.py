@@ -142,6 +142,11 @@ _SIGNATURES = {
                           c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p,
                           c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
                           c_void_p],
+        "ei_delta_chunk_floats": [c_int, c_int],
+        "ei_delta_chunks": [c_void_p, c_int, c_void_p, c_int, c_int, c_longlong, c_int, c_int, c_int,
+                            c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p,
+                            c_void_p, c_void_p, c_void_p, c_longlong, c_int, c_int, c_int, c_int,
+                            c_int, c_int, c_float, c_float, c_int, c_void_p],
         "ei_delta_out": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_int, c_int, c_int, c_void_p,
                          c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     },
@@ -1713,6 +1718,40 @@ def delta_rule(conv, proj, a_log, dt_bias, state, shape: DeltaShape, seq_in, seq
                                shape.n_kv_heads, shape.key_dim, shape.value_dim, float(q_scale),
                                float(unit_eps), _stream())
     _check(lib, status, "delta_rule")
+
+
+def delta_chunk_scratch(rows, seqs, shape: DeltaShape) -> int:
+    """float32 elements of scratch that `delta_chunks` wants for a step of so many rows."""
+    return _chunk_scratch("delta_rule", "ei_delta_chunk_floats", rows, seqs, shape.n_heads,
+                          shape.key_dim, shape.value_dim)
+
+
+def delta_chunks(conv, proj, a_log, dt_bias, state, shape: DeltaShape, seq_in, seq_out, seq_count,
+                 seq_row0, o_raw, q_scale: float, unit_eps: float, scratch, longest: int) -> None:
+    """What `delta_rule` does with one decay a head, by chunks of 64 tokens: heads of 64 or 128
+    elements; longest: the most rows that a sequence of the step brings."""
+    lib = library("delta_rule")
+    rows = conv.shape[0]
+    n_seqs = seq_count.numel()
+    if shape.low_rank:
+        raise KernelError("delta_chunks: one decay a head")
+    if tuple(conv.shape) != (rows, shape.conv_width) or tuple(o_raw.shape) != (rows, shape.v_width):
+        raise KernelError("delta_chunks: conv must be [rows, channels] and o_raw [rows, heads * value_dim]")
+    if a_log.numel() != shape.n_heads or dt_bias.numel() != shape.n_heads:
+        raise KernelError("delta_chunks: one decay rate and bias per head")
+    if seq_row0.numel() < n_seqs:
+        raise KernelError("delta_chunks: sequence metadata shorter than the sequences")
+    pointer, code, nsplit, stride, row_stride = _delta_proj(proj, rows, shape)
+    status = lib.ei_delta_chunks(
+        _gpu(conv, "conv", torch.float32), shape.conv_width, pointer, code, nsplit, stride, row_stride,
+        shape.beta_col, shape.decay_col, _gpu(a_log, "a_log", torch.float32),
+        _gpu(dt_bias, "dt_bias", torch.float32), _delta_state(state, shape), shape.state_floats,
+        *_delta_rows(seq_in, seq_out, n_seqs), _gpu(seq_count, "seq_count", torch.int32),
+        _gpu(seq_row0, "seq_row0", torch.int32), _gpu(o_raw, "o_raw", torch.float32),
+        _gpu(scratch, "scratch", torch.float32), scratch.numel(), rows, n_seqs, shape.n_heads,
+        shape.n_kv_heads, shape.key_dim, shape.value_dim, float(q_scale), float(unit_eps),
+        int(longest), _stream())
+    _check(lib, status, "delta_chunks")
 
 
 def delta_out(o_raw, proj, norm_w, eps, shape: DeltaShape, row_seq, out, sigmoid_gate=False,

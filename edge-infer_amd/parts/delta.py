@@ -99,6 +99,11 @@ class GatedDelta:
         # (S is a megabyte a layer and sequence at real sizes: two versions instead of copies)
         return StateRequest(shape=(cls.shape_of(spec).state_floats,), two_versions=True)
 
+    # from so many tokens of one sequence on, by chunks and not token by token, where a head has one
+    # decay (16 heads of 128 x 128: 64 tokens of one sequence 25 us by tokens and 33 by chunks, 8 x
+    # 512 298 and 158, 2,048 671 and 129)
+    CHUNK_FROM = 96
+
     @classmethod
     def kernel_libraries(cls, spec, dtype):
         return ("delta_rule", *Linear.kernel_libraries(dtype))
@@ -145,6 +150,8 @@ class GatedDelta:
         self.decay_bias = f32(params["decay_bias"])
         self.out_norm = f32(params["out_norm.weight"])
         self.q_scale = float(spec.key_dim) ** -0.5
+        self.chunks_fit = (not self.shape.low_rank and spec.key_dim in lib.CHUNK_SIZES
+                           and spec.value_dim in lib.CHUNK_SIZES)
 
     def _low_rank_rows(self, params):
         """The fused projection's rows where `DeltaShape` places them, zeros between."""
@@ -208,9 +215,14 @@ class GatedDelta:
                            meta.seq_row0)
         o_raw = ctx.buffer("delta.o_raw", (n, shape.v_width), torch.float32)
         rates = (None, None) if shape.low_rank else (self.decay_log_rate, self.decay_bias)
-        lib.delta_rule(conv, proj, *rates, state, shape,
-                       rows_in, rows_out, meta.seq_count, meta.seq_row0, o_raw, self.q_scale,
-                       self.spec.unit_eps)
+        how = (rows_in, rows_out, meta.seq_count, meta.seq_row0, o_raw, self.q_scale, self.spec.unit_eps)
+        longest = ctx.longest() if self.chunks_fit and not ctx.decode else 0
+        if longest >= self.CHUNK_FROM:
+            scratch = ctx.buffer("delta.chunks", (lib.delta_chunk_scratch(n, ctx.n_seqs, shape),), torch.float32)
+            lib.delta_chunks(conv, proj, *rates, state, shape, *how, scratch, longest)
+            ctx.release(scratch)
+        else:
+            lib.delta_rule(conv, proj, *rates, state, shape, *how)
         ctx.release(conv)
         gated = ctx.buffer("delta.gated", (n, shape.v_width))
         lib.delta_out(o_raw, proj, self.out_norm, self.spec.out_norm_eps, shape, meta.row_seq,

@@ -156,8 +156,58 @@ def test_exponential_gates(dk, dv, counts, dtype):
     assert not bool(torch.isnan(out).any())
 
 
+@pytest.mark.parametrize("counts,slices", [(COUNTS[0], 0), (COUNTS[0], 3), (COUNTS[1], 0), ([70] * 36, 0)])
+@pytest.mark.parametrize("dk,dv", [(64, 64), (64, 128), (128, 64), (128, 128)])
+def test_delta_rule(dk, dv, counts, slices):
+    """With keys that repeat (the triangular system at its worst) and decays from 1 to nothing; the
+    many short sequences take 32 columns a block."""
+    from edge_infer_amd.csrc import lib
+    H, G, rows = 4, 2, sum(counts)
+    shape = lib.DeltaShape(H, G, dk, dv, 4)
+    g = torch.Generator().manual_seed(dk + dv + rows)
+    conv = torch.randn(rows, shape.conv_width, generator=g)
+    conv[::3, G * dk:2 * G * dk] = conv[:1, G * dk:2 * G * dk]
+    proj = torch.randn(max(1, slices), rows, shape.width, generator=g) * 4.0
+    if not slices:
+        proj = proj[0].to(torch.bfloat16)
+    gates = proj.double().sum(0) if slices else proj.double()
+    a_log, bias = torch.rand(H, generator=g) * 4.0 - 3.0, torch.rand(H, generator=g) * 4.0 - 4.0
+    beta = torch.sigmoid(gates[:, shape.beta_col:shape.beta_col + H])
+    decay = torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(
+        gates[:, shape.decay_col:shape.decay_col + H] + bias.double()))
+    c, qk = conv.double(), G * dk
+
+    def unit(x):
+        return (x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(H // G, dim=1)
+    q, k = unit(c[:, :qk].view(rows, G, dk)) * dk ** -0.5, unit(c[:, qk:2 * qk].view(rows, G, dk))
+    v = c[:, 2 * qk:2 * qk + H * dv].view(rows, H, dv)
+    table = torch.randn(3 * len(counts), shape.state_floats, generator=g)
+    state = table[0::3, :H * dk * dv].double().view(len(counts), H, dv, dk).transpose(2, 3).clone()
+    want, row = torch.zeros(rows, H, dv, dtype=F64), 0
+    for s, count in enumerate(counts):
+        for _ in range(count):
+            S = decay[row][:, None, None] * state[s]
+            u = beta[row][:, None] * (v[row] - (S * k[row][:, :, None]).sum(dim=1))
+            state[s] = S + k[row][:, :, None] * u[:, None, :]
+            want[row] = (state[s] * q[row][:, :, None]).sum(dim=1)
+            row += 1
+    moved, out = table.to(DEV), torch.full((rows, H * dv), float("nan"), device=DEV)
+    scratch = torch.full((lib.delta_chunk_scratch(rows, len(counts), shape),), float("nan"), device=DEV)
+    lib.delta_chunks(conv.to(DEV), proj.to(DEV), a_log.to(DEV), bias.to(DEV), moved, shape,
+                     *metadata(counts), out, dk ** -0.5, 1e-6, scratch, max(counts))
+    got = moved.cpu()
+    live = [3 * s + 1 for s, n in enumerate(counts) if n]
+    tails = slice(H * dk * dv, None)
+    assert torch.equal(got[live][:, tails], table[live][:, tails])    # the tails are not its own
+    check(rows, out, want.reshape(rows, -1), got, table, state.transpose(2, 3).reshape(len(counts), -1),
+          counts, TOLERANCE)
+
+
 def designs():
     ff = {"kind": "dense", "ff": 64}
+    yield {"architecture": "Tirurax", "vocab": 97, "width": 64, "norm": {"eps": 1e-6},
+           "layers": [{"type": "delta", "mixer": {"heads": 4, "kv_heads": 2, "dim": 64, "vdim": 128, "conv": 4},
+                       "mlp": ff}]}
     yield {"architecture": "Zadenex", "vocab": 97, "width": 64, "norm": {"eps": 1e-6},
            "embedding": {"scale": 1.0}, "residual_mult": 0.5, "loop": None,
            "layers": [{"type": "mlstm", "mixer": {"heads": 2, "dim": 64, "vdim": 128, "gate_cap": 15.0},
