@@ -257,6 +257,179 @@ attn_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_pages,
   }
 }
 
+// One position an item (decoding), keys and values of D = 64 or 128 elements: the kernel above keeps
+// most of its threads and every load waiting for the few rows there are (3 sequences of 300 tokens, 16
+// heads of 128 in float32: 83 us).  Here 16 lanes share a key, D / 16 elements each, and the keys of
+// a page go to the 16 groups of four waves, four each, all of whose keys and values are asked for at
+// once; a group keeps a softmax of its own for up to GB heads, which are joined through LDS in a
+// fixed order at the end.
+template <typename T, int E> struct Share;          // the elements of lane l of 16
+template <int E> struct Share<float, E> {           // pieces of 4: lanes side by side
+  static __device__ __forceinline__ int place(int l, int e) { return e / 4 * 64 + 4 * l + e % 4; }
+  static __device__ __forceinline__ void load(const float* p, int l, float (&v)[E]) {
+#pragma unroll
+    for (int i = 0; i < E; i += 4) {
+      const float4 x = *reinterpret_cast<const float4*>(p + i * 16 + 4 * l);
+      v[i] = x.x; v[i + 1] = x.y; v[i + 2] = x.z; v[i + 3] = x.w;
+    }
+  }
+};
+template <int E> struct Share<bf16_t, E> {
+  static __device__ __forceinline__ int place(int l, int e) { return E * l + e; }
+  static __device__ __forceinline__ void load(const bf16_t* p, int l, float (&v)[E]) {
+    ei::VecN<bf16_t, E>::load(p + E * l, v);
+  }
+};
+
+__device__ __forceinline__ float row16_sum(float v) {
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xb1, 0xf, 0xf, false));
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4e, 0xf, 0xf, false));
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, false));
+  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xf, 0xf, false));
+  return v;
+}
+
+template <typename T, int D, int GB>
+__global__ void __launch_bounds__(kThreads)
+attn_single_kernel(const T* __restrict__ q, const T* __restrict__ k_pages,
+                   const T* __restrict__ v_pages, const int32_t* __restrict__ item_seq,
+                   const int32_t* __restrict__ item_row0, const int32_t* __restrict__ item_npos,
+                   const int32_t* __restrict__ row_pos, const int32_t* __restrict__ page_table,
+                   int table_width, T* __restrict__ out, float* __restrict__ part_o,
+                   float* __restrict__ part_ml, int nq, int nkv, int head_blocks, int window,
+                   int chunk, const float* __restrict__ slopes, const float* __restrict__ sinks,
+                   float scale, int n_splits, const float* __restrict__ gate, int pool,
+                   const T* __restrict__ pool_k, const T* __restrict__ pool_v,
+                   const int32_t* __restrict__ pool_table, int pool_only, int keep, float cap) {
+  constexpr int E = D / 16, kGroups = kThreads / 16, kKeys = EI_PAGE / kGroups;
+  __shared__ float m_lds[kGroups][GB], l_lds[kGroups][GB];
+  __shared__ float o_lds[kGroups][GB][D];
+  const int item = blockIdx.x, split = blockIdx.z;
+  const int g = blockIdx.y / head_blocks, head0 = blockIdx.y % head_blocks * GB, G = nq / nkv;
+  const int seq = item_seq[item];
+  if (seq < 0 || item_npos[item] <= 0) return;          // padding
+  const int row = item_row0[item], pos = row_pos[row];
+  const int l = threadIdx.x % 16, group = threadIdx.x / 16;
+  const int lo_key = max(window > 0 ? max(0, pos - window + 1) : 0, chunk > 0 ? pos / chunk * chunk : 0);
+  const int blocks = pool > 0 && window > 0 ? max(0, pos - window + 1) / pool : 0;   // pooled entries it sees
+  float qv[GB][E], acc[GB][E], m[GB], sum[GB], slope[GB];
+#pragma unroll
+  for (int h = 0; h < GB; ++h) {
+    const int head = g * G + min(head0 + h, G - 1);
+    Share<T, E>::load(q + (static_cast<size_t>(row) * nq + head) * D, l, qv[h]);
+    slope[h] = slopes ? slopes[head] : 0.f;
+    m[h] = kLowest;
+    sum[h] = 0.f;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      qv[h][e] *= scale;
+      acc[h][e] = 0.f;
+    }
+  }
+  // a page's keys key0 .. key0 + 63, of which those below `limit` hold something
+  auto page = [&](const T* kp, const T* vp, int key0, int limit, bool pooled) {
+    float kv[kKeys][E], vv[kKeys][E], s[kKeys][GB];
+    bool seen[kKeys];
+#pragma unroll
+    for (int u = 0; u < kKeys; ++u) {
+      const int at = u * kGroups + group, key = key0 + at;
+      seen[u] = key < limit && (pooled || key >= lo_key || key < keep);
+#pragma unroll
+      for (int e = 0; e < E; ++e) kv[u][e] = vv[u][e] = 0.f;
+      if (seen[u]) {
+        Share<T, E>::load(kp + static_cast<size_t>(at) * D, l, kv[u]);
+        Share<T, E>::load(vp + static_cast<size_t>(at) * D, l, vv[u]);
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < GB; ++h) {
+      float top = m[h];
+#pragma unroll
+      for (int u = 0; u < kKeys; ++u) {
+        float dots[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < E; ++e) dots[e % 4] += qv[h][e] * kv[u][e];
+        float dot = row16_sum((dots[0] + dots[1]) + (dots[2] + dots[3]));
+        if (cap > 0.f) dot = cap * tanhf(dot / cap);
+        if (!pooled) dot -= slope[h] * static_cast<float>(pos - (key0 + u * kGroups + group));
+        s[u][h] = seen[u] ? dot : -INFINITY;
+        top = fmaxf(top, s[u][h]);
+      }
+      const float alpha = expf(m[h] - top);
+      m[h] = top;
+      sum[h] *= alpha;
+#pragma unroll
+      for (int e = 0; e < E; ++e) acc[h][e] *= alpha;
+#pragma unroll
+      for (int u = 0; u < kKeys; ++u) {
+        const float p = expf(s[u][h] - top);
+        sum[h] += p;
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[h][e] += p * vv[u][e];
+      }
+    }
+  };
+  if (!pool_only) {
+    // (as above: pages with kept positions first, then the window's; a slice an equal share)
+    const int lo_page = lo_key / EI_PAGE, hi_page = pos / EI_PAGE;
+    const int kept_pages = min(lo_page, (keep + EI_PAGE - 1) / EI_PAGE);
+    const int total = kept_pages + hi_page - lo_page + 1;
+    const int per = (total + n_splits - 1) / n_splits;
+    const int end = min((split + 1) * per, total);
+    for (int i = split * per; i < end; ++i) {
+      const int p = i < kept_pages ? i : lo_page + i - kept_pages;
+      const int phys = page_table[static_cast<size_t>(seq) * table_width + p];
+      if (phys < 0) continue;
+      const size_t at = (static_cast<size_t>(phys) * nkv + g) * EI_PAGE * D;
+      page(k_pages + at, v_pages + at, p * EI_PAGE, pos + 1, false);
+    }
+  }
+  for (int p = split; p * EI_PAGE < blocks; p += n_splits) {
+    const int phys = pool_table[static_cast<size_t>(seq) * table_width + p];
+    if (phys < 0) continue;
+    const size_t at = (static_cast<size_t>(phys) * nkv + g) * EI_PAGE * D;
+    page(pool_k + at, pool_v + at, p * EI_PAGE, blocks, true);
+  }
+#pragma unroll
+  for (int h = 0; h < GB; ++h) {
+    if (l == 0) {
+      m_lds[group][h] = m[h];
+      l_lds[group][h] = sum[h];
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) o_lds[group][h][Share<T, E>::place(l, e)] = acc[h][e];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < GB * D; i += kThreads) {
+    const int h = i / D, d = i % D;
+    if (head0 + h >= G) continue;
+    const int head = g * G + head0 + h;
+    const bool sunk = sinks && split == 0 && !pool_only;
+    float top = sunk ? fmaxf(kLowest, sinks[head]) : kLowest;
+#pragma unroll
+    for (int w = 0; w < kGroups; ++w) top = fmaxf(top, m_lds[w][h]);
+    float total = sunk ? expf(sinks[head] - top) : 0.f, o = 0.f;
+#pragma unroll
+    for (int w = 0; w < kGroups; ++w) {
+      const float share = expf(m_lds[w][h] - top);
+      total += share * l_lds[w][h];
+      o += share * o_lds[w][h][d];
+    }
+    if (n_splits == 1 && !pool_only) {
+      float inv = total > 0.f ? 1.f / total : 0.f;
+      if (gate) inv *= 1.0f / (1.0f + expf(-gate[static_cast<size_t>(row) * nq + head]));
+      out[(static_cast<size_t>(row) * nq + head) * D + d] = ei::from_f32<T>(o * inv);
+    } else {
+      const size_t slot = (static_cast<size_t>(row) * nq + head) * n_splits + split;
+      part_o[slot * D + d] = o;
+      if (d == 0) {
+        part_ml[slot * 2] = top;
+        part_ml[slot * 2 + 1] = total;
+      }
+    }
+  }
+}
+
 // One wave per (row, head): o = sum_s o_s e^{m_s - m} / sum_s l_s e^{m_s - m}.
 template <typename T>
 __global__ void attn_merge_kernel(const float* __restrict__ part_o,
@@ -298,7 +471,7 @@ extern "C" int ei_attn_positions_per_item(int G) {
 
 // q: [N, nq, D], out: [N, nq, DV]; key pages: [n_pages, nkv, 64, D], value pages:
 // [n_pages, nkv, 64, DV]; items: see the kernel.  chunk 0, slopes and sinks null: none.
-// n_splits > 1 needs part_o [N, nq, n_splits, DV] and part_ml [N, nq, n_splits, 2]
+// single: no item holds more than one position.  n_splits > 1 needs part_o [N, nq, n_splits, DV] and part_ml [N, nq, n_splits, 2]
 // float32 and items that hold one position each (decode); the merge follows.
 extern "C" int ei_attention(const void* q, const void* k_pages, const void* v_pages, int dtype,
                             const int32_t* item_seq, const int32_t* item_row0,
@@ -309,7 +482,7 @@ extern "C" int ei_attention(const void* q, const void* k_pages, const void* v_pa
                             const float* sinks, float scale, int n_splits, int key_heads,
                             int values_in_keys, const float* gate, int pool, const void* pool_k,
                             const void* pool_v, const int32_t* pool_table, int pool_only,
-                            int keep, float cap, hipStream_t stream) {
+                            int keep, float cap, int single, hipStream_t stream) {
   EI_REQUIRE(n_items > 0 && N > 0 && nq > 0 && nkv > 0, "attention: sizes must be positive");
   EI_REQUIRE(nq % nkv == 0, "attention: query heads must be a multiple of kv heads");
   EI_REQUIRE(key_heads == 1 || key_heads == nkv,
@@ -334,13 +507,47 @@ extern "C" int ei_attention(const void* q, const void* k_pages, const void* v_pa
                                          key_heads == 1 && !values_in_keys)),
              "attention: pooled blocks need a window, their cache and keys of one kv head");
   const int G = nq / nkv;
+  const uintptr_t bases = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pages) |
+                          reinterpret_cast<uintptr_t>(v_pages) | reinterpret_cast<uintptr_t>(pool_k) |
+                          reinterpret_cast<uintptr_t>(pool_v);
+  const bool few = single && key_heads == 1 && !values_in_keys && D == DV && (D == 64 || D == 128) &&
+                   (bases & 15) == 0;
+  if (few) {
+    const int gb = G >= 4 ? 4 : (G >= 2 ? 2 : 1), per_group = (G + gb - 1) / gb;
+    EI_REQUIRE(static_cast<long long>(nkv) * per_group <= 65535, "attention: too many heads");
+    const dim3 items(n_items, nkv * per_group, n_splits);
+#define EI_SINGLE(T, DD, GB)                                                                      \
+  attn_single_kernel<T, DD, GB><<<items, kThreads, 0, stream>>>(                                  \
+      static_cast<const T*>(q), static_cast<const T*>(k_pages), static_cast<const T*>(v_pages),   \
+      item_seq, item_row0, item_npos, row_pos, page_table, table_width, static_cast<T*>(out),     \
+      part_o, part_ml, nq, nkv, per_group, window, chunk, slopes, sinks, scale, n_splits, gate,   \
+      pool, static_cast<const T*>(pool_k), static_cast<const T*>(pool_v), pool_table, pool_only,  \
+      keep, cap)
+#define EI_SINGLE_D(T, DD)                 \
+  do {                                     \
+    if (gb == 4) EI_SINGLE(T, DD, 4);      \
+    else if (gb == 2) EI_SINGLE(T, DD, 2); \
+    else EI_SINGLE(T, DD, 1);              \
+  } while (0)
+    if (dtype == EI_F32) {
+      if (D == 128) EI_SINGLE_D(float, 128);
+      else EI_SINGLE_D(float, 64);
+    } else if (dtype == EI_BF16) {
+      if (D == 128) EI_SINGLE_D(bf16_t, 128);
+      else EI_SINGLE_D(bf16_t, 64);
+    } else {
+      EI_REQUIRE(false, "attention: unknown dtype");
+    }
+#undef EI_SINGLE_D
+#undef EI_SINGLE
+  }
   const int Gb = G < kRows ? G : kRows;
   const int head_blocks = (G + Gb - 1) / Gb;
   const int BC = chunk_keys(DQ > DV ? DQ : DV);
   const size_t lds =
       sizeof(float) * (static_cast<size_t>(kRows) * DQ + static_cast<size_t>(BC) * (DQ + 1) +
                        static_cast<size_t>(BC) * DV + static_cast<size_t>(kRows) * (BC + 1));
-  if (lds > 64 * 1024) {      // beyond the default bound of a launch: ask for it, once
+  if (lds > 64 * 1024 && !few) {      // beyond the default bound of a launch: ask for it, once
     static bool raised = false;
     if (!raised) {
       const int most = 160 * 1024;
@@ -357,7 +564,9 @@ extern "C" int ei_attention(const void* q, const void* k_pages, const void* v_pa
   EI_REQUIRE(lds <= 160 * 1024, "attention: head sizes too large for the LDS");
   EI_REQUIRE(static_cast<long long>(nkv) * head_blocks <= 65535, "attention: too many heads");
   dim3 grid(n_items, nkv * head_blocks, n_splits);
-  if (dtype == EI_F32) {
+  if (few) {
+    // (launched above)
+  } else if (dtype == EI_F32) {
     attn_generic_kernel<float><<<grid, kThreads, lds, stream>>>(
         static_cast<const float*>(q), static_cast<const float*>(k_pages),
         static_cast<const float*>(v_pages), item_seq, item_row0, item_npos, row_pos, page_table,

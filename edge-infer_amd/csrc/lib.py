@@ -157,7 +157,7 @@ _SIGNATURES = {
                          c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
                          c_int, c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_float,
                          c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int,
-                         c_int, c_float, c_void_p],
+                         c_int, c_float, c_int, c_void_p],
         "ei_pool_store": [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
                           c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p, c_int,
                           c_void_p],
@@ -697,7 +697,7 @@ def attention(q, k_pages, v_pages, item_seq, item_row0, item_npos, n_items, row_
               n_splits=1, part_o=None, part_ml=None, value_dim=None, chunk=None, slopes=None,
               sinks=None, key_heads=1, values_in_keys=False, gate=None, pool=None,
               pool_k=None, pool_v=None, pool_table=None, pool_only=False, keep_first=0,
-              softcap=None) -> None:
+              softcap=None, single=False) -> None:
     """Generic causal attention over the paged cache (see attention_generic.hip).
     value_dim: head size of the values and of `out` (None: head_dim); chunk: a query sees only
     the keys of its own block of that many positions; slopes, sinks: float32 [n_heads], the
@@ -713,7 +713,8 @@ def attention(q, k_pages, v_pages, item_seq, item_row0, item_npos, n_items, row_
     value_dim] and part_ml [rows, heads, 2] receive every row's unnormalised sums over the
     pooled entries, the largest score and the sum of weights (n_splits 1).  keep_first: with a
     window, the keys of the sequence's first positions that stay visible however far back.
-    softcap c: a scaled score s becomes c tanh(s / c)."""
+    softcap c: a scaled score s becomes c tanh(s / c).  single: no item holds more than one
+    position (a decode step)."""
     lib = library("attention_generic")
     if softcap is not None and not softcap > 0:
         raise KernelError("attention: a cap on the scores must be positive")
@@ -778,7 +779,7 @@ def attention(q, k_pages, v_pages, item_seq, item_row0, item_npos, n_items, row_
         None if gate is None else _gpu(gate, "gate", torch.float32), int(pool or 0),
         _gpu(pool_k, "pool_k") if pool else None, _gpu(pool_v, "pool_v") if pool else None,
         _gpu(pool_table, "pool_table", torch.int32) if pool else None, int(bool(pool_only)),
-        int(keep_first) if window else 0, float(softcap or 0.0), _stream())
+        int(keep_first) if window else 0, float(softcap or 0.0), int(bool(single)), _stream())
     _check(lib, status, "attention")
 
 

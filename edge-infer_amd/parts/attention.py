@@ -620,7 +620,7 @@ class Attention:
                                   spec.n_kv_heads, spec.head_dim, window=spec.window,
                                   scale=self.scale, part_o=pool_o, part_ml=pool_ml,
                                   value_dim=spec.v_dim, pool_only=True, softcap=spec.softcap,
-                                  **pooled)
+                                  single=ctx.decode, **pooled)
                     aside = dict(pool_o=pool_o, pool_ml=pool_ml)
         elif (ctx.decode and self.matrix_cores and FUSED_DECODE and qkv.dim() == 3
                 and qkv.dtype == torch.float32 and not self.whole_store and not self.has_extras):
@@ -682,7 +682,7 @@ class Attention:
                                   meta.row_pos, meta.row_seq, page_table, out, spec.n_heads,
                                   spec.n_kv_heads, spec.head_dim, window=spec.window,
                                   scale=self.scale, n_splits=splits, part_o=part_o,
-                                  part_ml=part_ml, **more)
+                                  part_ml=part_ml, single=True, **more)
         else:
             key_ways = self.prefill_key_ways([seq.count for seq in ctx.sequences])
             section = self._items_section(key_ways)
