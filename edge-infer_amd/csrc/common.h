@@ -133,6 +133,20 @@ __device__ __forceinline__ float gated_product(float gate, float up, const GateA
   return swish<TO>(g, act.alpha) * (u + 1.0f);
 }
 
+// Activations of a plain feed-forward (codes of the C interface).
+constexpr int kRelu2 = 0, kRelu = 1, kSilu = 2, kGeluTanh = 3;
+
+__device__ __forceinline__ float activate(float x, int kind) {
+  if (kind == kRelu2) {
+    const float r = fmaxf(x, 0.f);
+    return r * r;
+  }
+  if (kind == kRelu) return fmaxf(x, 0.f);
+  if (kind == kSilu) return x / (1.0f + expf(-x));
+  // 0.5 x (1 + tanh(sqrt(2 / pi) (x + 0.044715 x^3)))
+  return 0.5f * x * (1.0f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
+}
+
 // Sine and cosine of an angle given in turns (of 2 pi): the whole turns are taken off in float64.
 // For float32 results the library's functions; for bfloat16 results the hardware's (which take
 // turns), good to about 1e-6 and swallowed by the rounding.

@@ -28,6 +28,7 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
+constexpr int kSums = 0, kGated = 1, kGatedBias = 2, kPlain = 3;    // see skinny_gemm_kernel
 constexpr int kPackedTile = 16 * 32;      // elements of one packed tile: 16 rows x 32 k, 1 KB
 
 // MB * 16 rows of X per workgroup, any K range.  A workgroup is WAVES waves, each owning
@@ -41,15 +42,23 @@ constexpr int kPackedTile = 16 * 32;      // elements of one packed tile: 16 row
 // Few K slices: for many rows the float32 partial sums (rows x N x 4 bytes a slice, written
 // in 64-byte pieces and read again by the consumer) cost more than the weights they save.
 //
-// GATED (one K slice only): the strips of W alternate between 16 gate rows and the 16 up rows
-// that belong to them; even waves hold gate sums, their odd neighbours the up sums (with two
-// strips a wave holds both), and the block writes their gated product (`act`) as bfloat16
-// [M, N/2] to `gated_out` instead of any sums.
-template <int MB, int WAVES, bool PACKED, bool GATED, int STRIPS, int KT>
+// What a block does with its sums is END.  kSums: writes them.  The others have one K slice:
+// kGated: the strips of W alternate between 16 gate rows and the 16 up rows that belong to them;
+// even waves hold gate sums, their odd neighbours the up sums (with two strips a wave holds both),
+// and the block writes their gated product (`act`) as bfloat16 [M, N/2] to `gated_out`.
+// kGatedBias: the same from sums that start at `bias` (float32 [N]; a kernel of its own, since
+// the form with 128 rows and two strips has no registers to spare).  kPlain: every strip stands
+// for itself, `gated_out` [M, N] takes ei::activate(sum), with sums that start at `bias` unless
+// it is null.
+// The next kernel then reads one bfloat16 matrix; the alternative writes float32 sums and reads
+// them again in a launch of its own, 3.4 to 5 us a layer of a decode step.
+template <int MB, int WAVES, bool PACKED, int END, int STRIPS, int KT>
 __global__ void __launch_bounds__(WAVES * EI_WAVE)
 skinny_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X,
                    float* __restrict__ out, bf16_t* __restrict__ gated_out, int M, int N, int K,
-                   int k_per_split, int row_groups, ei::GateAct act) {
+                   int k_per_split, int row_groups, ei::GateAct act,
+                   const float* __restrict__ bias) {
+  constexpr bool GATED = END == kGated || END == kGatedBias;
   constexpr int JN = KT / 32;             // MFMA steps per K-tile
   static_assert(KT == 256 || (KT == 128 && PACKED), "K-tiles of 256, or 128 with packed weights");
   constexpr int ROWS_X = MB * 16;
@@ -100,6 +109,18 @@ skinny_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X,
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int s = 0; s < STRIPS; ++s) acc[mb][s] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if constexpr (END == kGatedBias || END == kPlain) {
+    if (bias) {
+#pragma unroll
+      for (int s = 0; s < STRIPS; ++s) {
+        f32x4 start;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) start[r] = bias[min(n_tile + 16 * s + 4 * c + r, N - 1)];
+#pragma unroll
+        for (int mb = 0; mb < MB; ++mb) acc[mb][s] = start;
+      }
+    }
+  }
 
   bf16x8 w[2][JN][STRIPS];
   u32x4 x_regs[XLOADS];
@@ -327,6 +348,31 @@ skinny_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X,
     }
   }
 
+  if constexpr (END == kPlain) {
+#pragma unroll
+    for (int s = 0; s < STRIPS; ++s) {
+      const int n0 = n_tile + 16 * s + 4 * c;
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const int m = row0 + mb * 16 + r16;
+        if (m >= M) continue;
+        bf16_t v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = ei::f32_to_bf16(ei::activate(acc[mb][s][r], act.kind));
+        bf16_t* p = gated_out + static_cast<size_t>(m) * N + n0;
+        if (n0 + 3 < N && (N & 3) == 0) {
+          *reinterpret_cast<uint2*>(p) =
+              uint2{static_cast<uint32_t>(v[0]) | (static_cast<uint32_t>(v[1]) << 16),
+                    static_cast<uint32_t>(v[2]) | (static_cast<uint32_t>(v[3]) << 16)};
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n0 + r < N) p[r] = v[r];
+        }
+      }
+    }
+    return;
+  }
   if constexpr (GATED && STRIPS == 2) {
     // the wave holds the gate sums (strip 0) and the up sums (strip 1) of its 16 outputs
     if (n_tile + 16 < N) {
@@ -491,10 +537,10 @@ extern "C" int ei_skinny_gemm_splits(int M, int N, int K, int max_splits) {
 
 namespace {
 
-template <int MB, bool PACKED, bool GATED, int STRIPS, int KT = 256>
+template <int MB, bool PACKED, int END, int STRIPS, int KT = 256>
 void launch_tile_kernel(const bf16_t* w, const bf16_t* x, float* out, bf16_t* gated_out, int M,
                         int N, int K, int k_per_split, int splits, const ei::GateAct& act,
-                        hipStream_t stream) {
+                        const float* bias, hipStream_t stream) {
   const int n_strips = ((N + 15) / 16 + STRIPS - 1) / STRIPS;     // what a wave owns
   const int row_groups = (M + MB * 16 - 1) / (MB * 16);
   const int waves = tile_kernel_waves(n_strips, splits, row_groups,
@@ -503,31 +549,34 @@ void launch_tile_kernel(const bf16_t* w, const bf16_t* x, float* out, bf16_t* ga
   if (row_groups > 1) strip_blocks = (strip_blocks + 7) / 8 * 8;   // whole rounds of the dies
   dim3 grid(strip_blocks * row_groups, splits);
   if (waves == 4)
-    skinny_gemm_kernel<MB, 4, PACKED, GATED, STRIPS, KT><<<grid, 4 * EI_WAVE, 0, stream>>>(
-        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act);
+    skinny_gemm_kernel<MB, 4, PACKED, END, STRIPS, KT><<<grid, 4 * EI_WAVE, 0, stream>>>(
+        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias);
   else if (waves == 6)
-    skinny_gemm_kernel<MB, 6, PACKED, GATED, STRIPS, KT><<<grid, 6 * EI_WAVE, 0, stream>>>(
-        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act);
+    skinny_gemm_kernel<MB, 6, PACKED, END, STRIPS, KT><<<grid, 6 * EI_WAVE, 0, stream>>>(
+        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias);
   else
-    skinny_gemm_kernel<MB, 8, PACKED, GATED, STRIPS, KT><<<grid, 8 * EI_WAVE, 0, stream>>>(
-        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act);
+    skinny_gemm_kernel<MB, 8, PACKED, END, STRIPS, KT><<<grid, 8 * EI_WAVE, 0, stream>>>(
+        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias);
 }
 
-template <bool PACKED, bool GATED>
+template <bool PACKED, int END>
 int launch_skinny(const void* X, const void* W, float* out, void* gated_out, int M, int N, int K,
-                  int splits, hipStream_t stream, const ei::GateAct& act = ei::GateAct{0, 0.f, 1.f}) {
-  EI_REQUIRE(act.kind >= 0 && act.kind <= 2, "gemm_bf16_skinny_gated: unknown activation");
+                  int splits, hipStream_t stream, const ei::GateAct& act = ei::GateAct{0, 0.f, 1.f},
+                  const float* bias = nullptr) {
+  EI_REQUIRE(act.kind >= 0 && act.kind <= (END == kPlain ? 3 : 2),
+             "gemm_bf16_skinny_gated: unknown activation");
   EI_REQUIRE(M >= 1 && M <= kMaxRows, "gemm_bf16_skinny: rows must lie in 1..256");
   EI_REQUIRE(N >= 1 && K >= 8 && K % 8 == 0, "gemm_bf16_skinny: K must be a multiple of 8");
-  EI_REQUIRE(X && W && (GATED ? gated_out != nullptr : out != nullptr), "gemm_bf16_skinny: null pointer");
+  EI_REQUIRE(X && W && (END != kSums ? gated_out != nullptr : out != nullptr), "gemm_bf16_skinny: null pointer");
 
   EI_REQUIRE((reinterpret_cast<uintptr_t>(X) & 15) == 0 && (reinterpret_cast<uintptr_t>(W) & 15) == 0 &&
                  (reinterpret_cast<uintptr_t>(out) & 15) == 0 &&
                  (reinterpret_cast<uintptr_t>(gated_out) & 15) == 0,
              "gemm_bf16_skinny: pointers must be 16-byte aligned");
-  if (GATED) {
+  if (END != kSums) {
     EI_REQUIRE(splits == 1, "gemm_bf16_skinny_gated: K cannot be sliced");
-    EI_REQUIRE(N % 32 == 0, "gemm_bf16_skinny_gated: N must be a multiple of 32 (gate and up strips)");
+    EI_REQUIRE(N % 32 == 0 || END == kPlain,
+               "gemm_bf16_skinny_gated: N must be a multiple of 32 (gate and up strips)");
   }
   const TileMode mode = PACKED ? packed_mode(M, N) : TileMode{M <= 16 ? 1 : (M <= 32 ? 2 : 4), 1, 256};
   const int MB = mode.mb;
@@ -541,19 +590,19 @@ int launch_skinny(const void* X, const void* W, float* out, void* gated_out, int
   if (mode.strips == 2) {
     if constexpr (PACKED) {
       if (MB == 4)
-        launch_tile_kernel<4, PACKED, GATED, 2, 128>(w, x, out, g, M, N, K, k_per_split, splits, act, stream);
+        launch_tile_kernel<4, PACKED, END, 2, 128>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
       else
-        launch_tile_kernel<8, PACKED, GATED, 2, 128>(w, x, out, g, M, N, K, k_per_split, splits, act, stream);
+        launch_tile_kernel<8, PACKED, END, 2, 128>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
     }
   } else if (MB == 1) {
-    launch_tile_kernel<1, PACKED, GATED, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, stream);
+    launch_tile_kernel<1, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
   } else if (MB == 2) {
-    launch_tile_kernel<2, PACKED, GATED, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, stream);
+    launch_tile_kernel<2, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
   } else if (MB == 4) {
-    launch_tile_kernel<4, PACKED, GATED, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, stream);
+    launch_tile_kernel<4, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
   } else {
     if constexpr (PACKED)
-      launch_tile_kernel<8, PACKED, GATED, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, stream);
+      launch_tile_kernel<8, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
   }
   EI_LAUNCH_CHECK();
 }
@@ -565,7 +614,7 @@ int launch_skinny(const void* X, const void* W, float* out, void* gated_out, int
 // (beyond 64 rows several blocks share the weights through the L2 of their die).
 extern "C" int ei_gemm_bf16_skinny(const void* X, const void* W, float* out, int M, int N, int K,
                                    int splits, hipStream_t stream) {
-  return launch_skinny<false, false>(X, W, out, nullptr, M, N, K, splits, stream);
+  return launch_skinny<false, kSums>(X, W, out, nullptr, M, N, K, splits, stream);
 }
 
 // The same product with W in the streaming layout: tiles of 16 rows x 32 k (1 KB each, rows
@@ -577,18 +626,31 @@ extern "C" int ei_gemm_bf16_skinny(const void* X, const void* W, float* out, int
 // memory channel busy; rows of W that are 2^n bytes apart do not.
 extern "C" int ei_gemm_bf16_skinny_packed(const void* X, const void* Wp, float* out, int M, int N,
                                           int K, int splits, hipStream_t stream) {
-  return launch_skinny<true, false>(X, Wp, out, nullptr, M, N, K, splits, stream);
+  return launch_skinny<true, kSums>(X, Wp, out, nullptr, M, N, K, splits, stream);
 }
 
 // Gated feed-forward in one pass: W [N, K] holds, in strips of 16 rows, the gate rows of 16
 // outputs followed by their up rows (N = 2 * outputs, a multiple of 32); act [M, N/2]
 // bfloat16 = the gated product (`kind`, `limit`, `alpha` as in GateAct) of X . gate^T and
-// X . up^T.  All of K in one slice.  `packed`: W is in the
-// streaming layout of ei_gemm_bf16_skinny_packed.
+// X . up^T, each plus its bias where `bias` (float32 [N], the order of W's rows) is given.  All
+// of K in one slice.  `packed`: W is in the streaming layout of ei_gemm_bf16_skinny_packed.
 extern "C" int ei_gemm_bf16_skinny_gated(const void* X, const void* W, void* act, int M, int N,
                                          int K, int packed, int kind, float limit, float alpha,
-                                         hipStream_t stream) {
+                                         const float* bias, hipStream_t stream) {
   const ei::GateAct how{kind, limit, alpha};
-  if (packed) return launch_skinny<true, true>(X, W, nullptr, act, M, N, K, 1, stream, how);
-  return launch_skinny<false, true>(X, W, nullptr, act, M, N, K, 1, stream, how);
+  if (packed && bias)
+    return launch_skinny<true, kGatedBias>(X, W, nullptr, act, M, N, K, 1, stream, how, bias);
+  if (packed) return launch_skinny<true, kGated>(X, W, nullptr, act, M, N, K, 1, stream, how);
+  if (bias)
+    return launch_skinny<false, kGatedBias>(X, W, nullptr, act, M, N, K, 1, stream, how, bias);
+  return launch_skinny<false, kGated>(X, W, nullptr, act, M, N, K, 1, stream, how);
+}
+
+// A feed-forward's first product with its activation: out [M, N] bfloat16 = activate(X . W^T +
+// bias), `kind` a code of ei::activate, `bias` float32 [N] or null.  All of K in one slice.
+extern "C" int ei_gemm_bf16_skinny_act(const void* X, const void* W, void* out, int M, int N, int K,
+                                       int packed, int kind, const float* bias, hipStream_t stream) {
+  const ei::GateAct how{kind, 0.f, 1.f};
+  if (packed) return launch_skinny<true, kPlain>(X, W, nullptr, out, M, N, K, 1, stream, how, bias);
+  return launch_skinny<false, kPlain>(X, W, nullptr, out, M, N, K, 1, stream, how, bias);
 }

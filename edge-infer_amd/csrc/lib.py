@@ -252,7 +252,9 @@ _SIGNATURES = {
         "ei_gemm_bf16_skinny_packed": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                        c_void_p],
         "ei_gemm_bf16_skinny_gated": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
-                                      c_int, c_float, c_float, c_void_p],
+                                      c_int, c_float, c_float, c_void_p, c_void_p],
+        "ei_gemm_bf16_skinny_act": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                    c_int, c_void_p, c_void_p],
     },
     "sampling": {
         "ei_argmax": [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p],
@@ -2509,12 +2511,21 @@ def gemm_bf16_skinny_packed(x: torch.Tensor, packed: torch.Tensor, n: int,
 GATE_STRIP = 16     # gate rows and up rows alternate in strips of this many (one MFMA tile)
 
 
+def _fused_weight(w, n: int, k: int, packed: bool, bias, what: str) -> None:
+    expect = (8 * ((k + 255) // 256), (n + 15) // 16, 4, 16, 8) if packed else (n, k)
+    if tuple(w.shape) != expect:
+        raise KernelError(f"{what}: weight {list(w.shape)}, expected {list(expect)}")
+    if bias is not None and tuple(bias.shape) != (n,):
+        raise KernelError(f"{what}: bias {list(bias.shape)}, expected [{n}]")
+
+
 def gemm_bf16_skinny_gated(x: torch.Tensor, w: torch.Tensor, n: int, act: torch.Tensor,
                            packed: bool, activation: str = "silu", limit: float = 0.0,
-                           alpha: float = 1.0) -> None:
+                           alpha: float = 1.0, bias: Optional[torch.Tensor] = None) -> None:
     """act[m, i] = silu(x[m] . gate_i) * (x[m] . up_i) (or another `activation` of `swiglu`) for a weight [n, k] whose rows are, in
     strips of 16, the gate rows of 16 outputs followed by their up rows; `w` is that matrix or
-    (packed) its `pack_weight` copy.  For at most 256 rows; K is not sliced, so it pays where
+    (packed) its `pack_weight` copy; `bias` (float32 [n], in the order of the rows) is what the
+    sums start from.  For at most 256 rows; K is not sliced, so it pays where
     `skinny_gemm_splits` is 1."""
     lib = library("gemm_bf16")
     m, k = x.shape
@@ -2523,14 +2534,33 @@ def gemm_bf16_skinny_gated(x: torch.Tensor, w: torch.Tensor, n: int, act: torch.
     if tuple(act.shape) != (m, n // 2) or n % (2 * GATE_STRIP):
         raise KernelError(f"gemm_bf16_skinny_gated: {list(x.shape)} x [{n}, {k}] -> "
                           f"{list(act.shape)} do not agree")
-    expect = (8 * ((k + 255) // 256), (n + 15) // 16, 4, 16, 8) if packed else (n, k)
-    if tuple(w.shape) != expect:
-        raise KernelError(f"gemm_bf16_skinny_gated: weight {list(w.shape)}, expected {list(expect)}")
+    _fused_weight(w, n, k, packed, bias, "gemm_bf16_skinny_gated")
     status = lib.ei_gemm_bf16_skinny_gated(_gpu(x, "x", torch.bfloat16), _gpu(w, "w", torch.bfloat16),
                                            _gpu(act, "act", torch.bfloat16), m, n, k, int(packed),
-                                           GATE_ACTIVATIONS[activation], float(limit),
-                                           float(alpha), _stream())
+                                           GATE_ACTIVATIONS[activation], float(limit), float(alpha),
+                                           None if bias is None else _gpu(bias, "bias", torch.float32),
+                                           _stream())
     _check(lib, status, "gemm_bf16_skinny_gated")
+
+
+def gemm_bf16_skinny_act(x: torch.Tensor, w: torch.Tensor, n: int, out: torch.Tensor,
+                         packed: bool, kind: str, bias: Optional[torch.Tensor] = None) -> None:
+    """out [m, n] = act(x . w^T + bias) for at most 256 rows, `kind` as for `activation`; `w`,
+    `packed` and `bias` as for `gemm_bf16_skinny_gated`.  K is not sliced."""
+    lib = library("gemm_bf16")
+    m, k = x.shape
+    if kind not in ACTIVATIONS:
+        raise KernelError(f"gemm_bf16_skinny_act: unknown kind '{kind}'; known: {sorted(ACTIVATIONS)}")
+    if tuple(out.shape) != (m, n):
+        raise KernelError(f"gemm_bf16_skinny_act: {list(x.shape)} x [{n}, {k}] -> "
+                          f"{list(out.shape)} do not agree")
+    _fused_weight(w, n, k, packed, bias, "gemm_bf16_skinny_act")
+    status = lib.ei_gemm_bf16_skinny_act(_gpu(x, "x", torch.bfloat16), _gpu(w, "w", torch.bfloat16),
+                                         _gpu(out, "out", torch.bfloat16), m, n, k, int(packed),
+                                         ACTIVATIONS[kind],
+                                         None if bias is None else _gpu(bias, "bias", torch.float32),
+                                         _stream())
+    _check(lib, status, "gemm_bf16_skinny_act")
 
 
 # ---------------------------------------------------------------------------

@@ -508,20 +508,6 @@ __global__ void cast_rows_kernel(const float* __restrict__ in, TO* __restrict__ 
   for (size_t i = start; i < n; i += step) out[i] = ei::from_f32<TO>(in[i]);
 }
 
-// activation kinds of the C interface
-constexpr int kRelu2 = 0, kRelu = 1, kSilu = 2, kGeluTanh = 3;
-
-__device__ __forceinline__ float activate(float x, int kind) {
-  if (kind == kRelu2) {
-    const float r = fmaxf(x, 0.f);
-    return r * r;
-  }
-  if (kind == kRelu) return fmaxf(x, 0.f);
-  if (kind == kSilu) return x / (1.0f + expf(-x));
-  // 0.5 x (1 + tanh(sqrt(2 / pi) (x + 0.044715 x^3)))
-  return 0.5f * x * (1.0f + tanhf(0.7978845608028654f * (x + 0.044715f * x * x * x)));
-}
-
 // out = act(sum over slices of in), elementwise.
 template <typename TI, typename TO>
 __global__ void activation_kernel(const TI* __restrict__ in, int nsplit, size_t split_stride,
@@ -539,7 +525,7 @@ __global__ void activation_kernel(const TI* __restrict__ in, int nsplit, size_t 
       for (int u = 0; u < 8; ++u)
         if (s0 + u < nsplit) x += v[u];
     }
-    out[i] = ei::from_f32<TO>(activate(x, kind));
+    out[i] = ei::from_f32<TO>(ei::activate(x, kind));
   }
 }
 
@@ -568,7 +554,7 @@ __global__ void activation_vec_kernel(const TI* __restrict__ in, int nsplit, siz
         }
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = activate(x[i], kind);
+    for (int i = 0; i < 8; ++i) x[i] = ei::activate(x[i], kind);
     ei::VecN<TO, 8>::store(out + idx * 8, x);
   }
 }

@@ -31,8 +31,18 @@ STREAM_COPY = os.environ.get("EDGE_INFER_STREAM_COPY", "1") != "0"
 # The gated product does not slice K.  Where the planner would slice, one kernel still beats
 # the sliced product plus the activation kernel while the matrix is small enough for a launch
 # to weigh as much as the slicing gains (measured at 1 to 32 rows: 12.6 MB 5.6 against 7.2 us,
-# 100 MB 17.2 against 20.9, 357 MB 62.2 against 61.2, 524 MB 90.4 against 83.9).
+# 100 MB 17.2 against 20.9, 357 MB 62.2 against 61.2, 524 MB 90.4 against 83.9; with a bias, at
+# 64 rows: 4 MB 7.8 against 8.8, 25 MB 11.9 against 14.7, at 256 rows 14.4 and 23.2 against 15.4
+# and 24.5).
 GATED_UNSLICED_BYTES = 200 * 1000 * 1000
+# A plain activation reads and writes as many sums as the product has outputs, so the sliced form
+# holds out longer there.  With slices the one kernel is taken for up to 32 rows (1024 -> 2048:
+# 1 row 5.1 against 5.4 us, 32 rows 6.0 against 6.2, 64 rows 7.2 against 7.0, 200 rows 15.3 against
+# 13.1) and, where there are 4096 outputs or more (a strip of 16 for every compute unit), for up
+# to 64 (1024 -> 4096: 7.3 against 8.9; 2048 -> 6144: 11.5 against 13.3, but at 200 rows 24.0
+# against 22.5); unsliced at every row count (2048 -> 16384: 12.5 against 14.6 us at 1 row, 26.1
+# against 33.9 at 256).
+PLAIN_SLICED_ROWS, PLAIN_WIDE, PLAIN_SLICED_ROWS_WIDE = 32, 4096, 64
 
 
 class Linear:
@@ -125,23 +135,42 @@ class Linear:
         else:
             torch.addmm(self.bias, x, self.weight.t(), out=out)
 
+    def _unsliced(self, rows: int) -> bool:
+        """Whether the few-rows kernel applies with all of K in one slice, for an epilogue on the
+        whole sums (not for float32, many rows, a large matrix whose K the planner would slice)."""
+        return (self.dtype == torch.bfloat16 and lib.skinny_gemm_ok(rows, self.in_features)
+                and (self.weight.numel() * 2 <= GATED_UNSLICED_BYTES or
+                     lib.skinny_gemm_splits(rows, self.out_features, self.in_features) == 1))
+
     def forward_gated(self, ctx, x: torch.Tensor, out_name: str, **activation):
         """For a weight whose rows alternate, in strips of `lib.GATE_STRIP`, between gate rows
-        and their up rows: silu(gate) * up (or another `activation` with its limit and alpha) as
-        [N, out/2] of the storage type straight from
-        the few-rows kernel, or None where that kernel does not apply (float32, many rows, a
-        bias, a large matrix whose K the planner would slice); the caller then takes
-        `forward` and the activation kernel."""
+        and their up rows: silu(gate) * up (or another `activation` with its limit and alpha), the
+        bias included, as [N, out/2] of the storage type straight from
+        the few-rows kernel, or None where that kernel does not apply (see `_unsliced`); the
+        caller then takes `forward` and the activation kernel."""
         rows = x.shape[0]
-        if (self.dtype != torch.bfloat16 or self.bias is not None or not lib.skinny_gemm_ok(rows, self.in_features)
-                or self.out_features % (2 * lib.GATE_STRIP)
-                or (self.weight.numel() * 2 > GATED_UNSLICED_BYTES and
-                    lib.skinny_gemm_splits(rows, self.out_features, self.in_features) != 1)):
+        if not self._unsliced(rows) or self.out_features % (2 * lib.GATE_STRIP):
             return None
         act = ctx.buffer(out_name, (rows, self.out_features // 2), torch.bfloat16)
         packed = self.packed is not None
         lib.gemm_bf16_skinny_gated(x, self.packed if packed else self.weight, self.out_features,
-                                   act, packed, **activation)
+                                   act, packed, bias=self.bias_f32, **activation)
+        return act
+
+    def forward_activated(self, ctx, x: torch.Tensor, out_name: str, kind: str):
+        """act(x . W^T + bias) as [N, out] of the storage type straight from the few-rows kernel,
+        or None where that kernel does not apply or the sliced product and the activation kernel
+        are faster."""
+        rows = x.shape[0]
+        if not self._unsliced(rows):
+            return None
+        most = PLAIN_SLICED_ROWS_WIDE if self.out_features >= PLAIN_WIDE else PLAIN_SLICED_ROWS
+        if rows > most and lib.skinny_gemm_splits(rows, self.out_features, self.in_features) != 1:
+            return None
+        act = ctx.buffer(out_name, (rows, self.out_features), torch.bfloat16)
+        packed = self.packed is not None
+        lib.gemm_bf16_skinny_act(x, self.packed if packed else self.weight, self.out_features,
+                                 act, packed, kind, bias=self.bias_f32)
         return act
 
     def forward_f32(self, ctx, x: torch.Tensor, out_name: str) -> torch.Tensor:

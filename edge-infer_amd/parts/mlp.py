@@ -117,8 +117,9 @@ class GatedMLP:
 
 class DenseMLP:
     """down(act(up(x))): two matrices and an elementwise activation between them
-    (`spec.activation`: "relu2" = relu(z)^2, "relu", "silu", "gelu_tanh").  The activation
-    kernel sums the float32 slices of a few-rows product while it reads them."""
+    (`spec.activation`: "relu2" = relu(z)^2, "relu", "silu", "gelu_tanh").  For few rows
+    the first product's kernel applies it to its sums; where it does not, the activation kernel
+    sums the float32 slices while it reads them."""
 
     @property
     def capture_safe(self):
@@ -151,11 +152,12 @@ class DenseMLP:
                            bias=params.get("down_proj.bias"))
 
     def forward(self, ctx, x):
-        n = x.shape[0]
-        up = self.up.forward(ctx, x, "mlp.up")
-        act = ctx.buffer("mlp.act", (n, self.spec.intermediate_size))
-        lib.activation(up, act, self.spec.activation)
-        ctx.release(up)
+        act = self.up.forward_activated(ctx, x, "mlp.act", self.spec.activation)
+        if act is None:
+            up = self.up.forward(ctx, x, "mlp.up")
+            act = ctx.buffer("mlp.act", (x.shape[0], self.spec.intermediate_size))
+            lib.activation(up, act, self.spec.activation)
+            ctx.release(up)
         out = self.down.forward(ctx, act, "mlp.down")
         ctx.release(act)
         return out
