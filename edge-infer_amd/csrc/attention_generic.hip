@@ -257,6 +257,175 @@ attn_generic_kernel(const T* __restrict__ q, const T* __restrict__ k_pages,
   }
 }
 
+// Prompts in float32, keys and values of D = 64 or 128 elements: scores and values by float32 matrix
+// instructions.  The kernel above reads two LDS words for every product (3 prompts, 451 tokens together, 16
+// heads of 128 over 8 kv heads: 198 us a layer); here nothing of a key or value goes through LDS: a wave
+// takes every page's 16 keys 16 w .. 16 w + 15 with a softmax of its own, the scores come out as
+// [keys, rows], which is the order in which the second product wants its weights, and the four waves
+// are joined at the end in a fixed order (14.8 us).  Bound by the latency of a page's keys and values,
+// of which a block meets one after the other.  A row's result depends on its own keys alone: where
+// they lie in their page decides which wave adds them up.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+template <int D>
+__global__ void __launch_bounds__(kThreads)
+attn_prompt_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pages,
+                       const float* __restrict__ v_pages, const int32_t* __restrict__ item_seq,
+                       const int32_t* __restrict__ item_row0, const int32_t* __restrict__ item_npos,
+                       const int32_t* __restrict__ row_pos, const int32_t* __restrict__ page_table,
+                       int table_width, float* __restrict__ out, float* __restrict__ part_o,
+                       float* __restrict__ part_ml, int nq, int nkv, int Gb, int head_blocks, int window,
+                       int chunk, const float* __restrict__ slopes, const float* __restrict__ sinks,
+                       float scale, int n_splits, const float* __restrict__ gate, int keep, float cap) {
+  constexpr int S = D / 16, H = D / 64, kWaves = kThreads / EI_WAVE;
+  static_assert(kWaves * 16 == EI_PAGE, "the waves share a page out");
+  __shared__ __attribute__((aligned(16))) float o_lds[kWaves][kRows][D + 4];
+  __shared__ float m_lds[kWaves][kRows], l_lds[kWaves][kRows];
+  const int item = blockIdx.x, split = blockIdx.z;
+  const int g = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks, G = nq / nkv;
+  const int seq = item_seq[item], npos = item_npos[item], row0 = item_row0[item];
+  if (seq < 0 || npos <= 0) return;                 // padding
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / EI_WAVE);
+  const int lane = threadIdx.x % EI_WAVE, r16 = lane & 15, c = lane >> 4;
+  {
+    const int pi = r16 / Gb, in_group = hb * Gb + r16 % Gb;
+    const bool valid = pi < npos && in_group < G;
+    const int row = row0 + min(pi, npos - 1), head = g * G + min(in_group, G - 1);
+    const int pos = valid ? row_pos[row] : -1;
+    const float slope = slopes ? slopes[head] : 0.f;
+    const int own_chunk = chunk > 0 && valid ? pos / chunk : 0;
+    f32x4 qv[S];                                    // element 16 s + 4 c + i of row r16
+    const float* q_row = q + (static_cast<size_t>(row) * nq + head) * D + 4 * c;
+#pragma unroll
+    for (int s = 0; s < S; ++s) qv[s] = *reinterpret_cast<const f32x4*>(q_row + 16 * s) * scale;
+    f32x4 acc[H][4];                                // [h][e][j]: value element 64 h + 16 c + 4 j + e
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[h][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m_r = kLowest, l_r = 0.f;                 // (l: this lane's keys)
+
+    const int hi_key = row_pos[row0 + npos - 1];
+    int lo_key = window > 0 ? max(0, row_pos[row0] - window + 1) : 0;
+    if (chunk > 0) lo_key = max(lo_key, row_pos[row0] / chunk * chunk);
+    const int lo_page = lo_key / EI_PAGE, hi_page = hi_key / EI_PAGE;
+    // pages before the window's that hold kept positions: they come first in the walk
+    const int kept_pages = min(lo_page, (keep + EI_PAGE - 1) / EI_PAGE);
+    const int total_pages = kept_pages + hi_page - lo_page + 1;
+    const int per = (total_pages + n_splits - 1) / n_splits;
+    const int i_end = min((split + 1) * per, total_pages);
+    for (int i = split * per; i < i_end; ++i) {
+      const int p = i < kept_pages ? i : lo_page + i - kept_pages;
+      const int key0 = p * EI_PAGE + 16 * wave;
+      if (key0 > hi_key) continue;
+      if (key0 + 16 <= lo_key && key0 >= keep) continue;      // nothing that any row of the item sees
+      const int phys = page_table[static_cast<size_t>(seq) * table_width + p];
+      if (phys < 0) continue;  // a page the window has released: every key in it is masked
+      const size_t page = (static_cast<size_t>(phys) * nkv + g) * EI_PAGE * D;
+      const float* kp = k_pages + page + static_cast<size_t>(16 * wave + r16) * D + 4 * c;
+      const float* vp = v_pages + page + static_cast<size_t>(16 * wave + 4 * c) * D + 4 * r16;
+      f32x4 kv[S], vv[4][H];
+#pragma unroll
+      for (int s = 0; s < S; ++s) kv[s] = *reinterpret_cast<const f32x4*>(kp + 16 * s);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int h = 0; h < H; ++h) vv[j][h] = *reinterpret_cast<const f32x4*>(vp + j * D + 64 * h);
+      f32x4 even = f32x4{0.f, 0.f, 0.f, 0.f}, odd = even;
+#pragma unroll
+      for (int s = 0; s < S; s += 2)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          even = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[s][e], qv[s][e], even, 0, 0, 0);
+          odd = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[s + 1][e], qv[s + 1][e], odd, 0, 0, 0);
+        }
+      float p_val[4];
+      float row_max = kLowest;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {                 // key 4 c + j of the wave's 16 against row r16
+        const int key = key0 + 4 * c + j;
+        const bool visible = valid && key <= pos &&
+                             (window <= 0 || key > pos - window || key < keep) &&
+                             (chunk <= 0 || key / chunk == own_chunk);
+        float dot = even[j] + odd[j];
+        if (cap > 0.f) dot = cap * tanhf(dot / cap);
+        dot -= slope * static_cast<float>(pos - key);
+        p_val[j] = visible ? dot : -INFINITY;
+        row_max = visible ? fmaxf(row_max, dot) : row_max;
+        if (key > hi_key) {                         // later slots hold stale bytes
+#pragma unroll
+          for (int h = 0; h < H; ++h) vv[j][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+      row_max = fmaxf(row_max, __shfl_xor(row_max, 16, EI_WAVE));
+      row_max = fmaxf(row_max, __shfl_xor(row_max, 32, EI_WAVE));
+      const float m_new = fmaxf(m_r, row_max);
+      const float alpha = expf(m_r - m_new);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) p_val[j] = expf(p_val[j] - m_new);      // -inf -> 0
+      l_r = l_r * alpha + ((p_val[0] + p_val[1]) + (p_val[2] + p_val[3]));
+      m_r = m_new;
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[h][e] *= alpha;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int h = 0; h < H; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            acc[h][e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[j][h][e], p_val[j], acc[h][e], 0, 0, 0);
+    }
+    l_r += __shfl_xor(l_r, 16, EI_WAVE);
+    l_r += __shfl_xor(l_r, 32, EI_WAVE);
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<f32x4*>(&o_lds[wave][r16][64 * h + 16 * c + 4 * j]) =
+            f32x4{acc[h][0][j], acc[h][1][j], acc[h][2][j], acc[h][3][j]};
+    if (c == 0) {
+      m_lds[wave][r16] = m_r;
+      l_lds[wave][r16] = l_r;
+    }
+  }
+  __syncthreads();
+  const int r = threadIdx.x / 16, cc = threadIdx.x % 16;
+  const int pi = r / Gb, in_group = hb * Gb + r % Gb;
+  if (pi >= npos || in_group >= G) return;
+  const int row = row0 + pi, head = g * G + in_group;
+  const bool sink = sinks && split == 0;
+  float m = sink ? sinks[head] : kLowest;           // the sink: one more term of the denominator
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) m = fmaxf(m, m_lds[w][r]);
+  float l = sink ? expf(sinks[head] - m) : 0.f, part[kWaves];
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    part[w] = expf(m_lds[w][r] - m);
+    l += l_lds[w][r] * part[w];
+  }
+  float inv = 1.f;
+  float* dst = part_o + ((static_cast<size_t>(row) * nq + head) * n_splits + split) * D;
+  if (n_splits == 1) {
+    dst = out + (static_cast<size_t>(row) * nq + head) * D;
+    inv = l > 0.f ? 1.f / l : 0.f;
+    if (gate) inv *= 1.0f / (1.0f + expf(-gate[static_cast<size_t>(row) * nq + head]));
+  } else if (cc == 0) {
+    float* ml = part_ml + ((static_cast<size_t>(row) * nq + head) * n_splits + split) * 2;
+    ml[0] = m;
+    ml[1] = l;
+  }
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w)
+      o += *reinterpret_cast<const f32x4*>(&o_lds[w][r][64 * h + 4 * cc]) * part[w];
+    *reinterpret_cast<f32x4*>(dst + 64 * h + 4 * cc) = o * inv;
+  }
+}
+
 // One position an item (decoding), keys and values of D = 64 or 128 elements: the kernel above keeps
 // most of its threads and every load waiting for the few rows there are (3 sequences of 300 tokens, 16
 // heads of 128 in float32: 83 us).  Here 16 lanes share a key, D / 16 elements each, and the keys of
@@ -547,7 +716,26 @@ extern "C" int ei_attention(const void* q, const void* k_pages, const void* v_pa
   const size_t lds =
       sizeof(float) * (static_cast<size_t>(kRows) * DQ + static_cast<size_t>(BC) * (DQ + 1) +
                        static_cast<size_t>(BC) * DV + static_cast<size_t>(kRows) * (BC + 1));
-  if (lds > 64 * 1024 && !few) {      // beyond the default bound of a launch: ask for it, once
+  EI_REQUIRE(static_cast<long long>(nkv) * head_blocks <= 65535, "attention: too many heads");
+  dim3 grid(n_items, nkv * head_blocks, n_splits);
+  // (pooled entries, keys of several heads and values inside keys keep the general kernel, as do
+  // other sizes and bfloat16, whose plain prompts have kernels of their own)
+  const bool prompt_f32 = !few && dtype == EI_F32 && key_heads == 1 && !values_in_keys && pool == 0 &&
+                          D == DV && (D == 64 || D == 128) &&
+                          ((bases | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(part_o)) & 15) == 0;
+  if (prompt_f32) {
+#define EI_PROMPT(DD)                                                                             \
+  attn_prompt_f32_kernel<DD><<<grid, kThreads, 0, stream>>>(                                      \
+      static_cast<const float*>(q), static_cast<const float*>(k_pages),                           \
+      static_cast<const float*>(v_pages), item_seq, item_row0, item_npos, row_pos, page_table,    \
+      table_width, static_cast<float*>(out), part_o, part_ml, nq, nkv, Gb, head_blocks, window,   \
+      chunk, slopes, sinks, scale, n_splits, gate, keep, cap)
+    if (D == 128) EI_PROMPT(128);
+    else EI_PROMPT(64);
+#undef EI_PROMPT
+  }
+  const bool launched = few || prompt_f32;
+  if (lds > 64 * 1024 && !launched) {      // beyond the default bound of a launch: ask for it, once
     static bool raised = false;
     if (!raised) {
       const int most = 160 * 1024;
@@ -562,9 +750,7 @@ extern "C" int ei_attention(const void* q, const void* k_pages, const void* v_pa
     }
   }
   EI_REQUIRE(lds <= 160 * 1024, "attention: head sizes too large for the LDS");
-  EI_REQUIRE(static_cast<long long>(nkv) * head_blocks <= 65535, "attention: too many heads");
-  dim3 grid(n_items, nkv * head_blocks, n_splits);
-  if (few) {
+  if (launched) {
     // (launched above)
   } else if (dtype == EI_F32) {
     attn_generic_kernel<float><<<grid, kThreads, lds, stream>>>(
