@@ -3,7 +3,8 @@
 // storage, float32 arithmetic throughout (scores, running maximum, exponentials,
 // sums and the value accumulation).  One kernel serves prefill (many positions of a
 // sequence) and decode (one position, the key range split over several blocks and
-// merged by a second kernel).
+// merged by a second kernel) for every size and option; two more take what is used most: heads of
+// 64 or 128 elements when decoding, and float32 prompts of such heads.
 //
 // Mathematics of the reference: s_t = (q . k_t) / sqrt(d) for keys t <= p (and
 // t > p - window when a window is set), streaming softmax with a running maximum,

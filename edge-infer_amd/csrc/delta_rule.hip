@@ -26,6 +26,8 @@
 //                old ones)
 //   delta_rule   the recurrence; a thread owns 8 or 16 rows of one column of S, L lanes share a
 //                column; tokens come in tiles through LDS
+//   delta_chunks the recurrence for steps that bring many tokens of a sequence, where a head has
+//                one decay: 64 tokens at a time as float32 matrix products (delta_chunks.h)
 //   delta_out    the read-out's norm and gate
 #include "common.h"
 #include "few_rows.h"

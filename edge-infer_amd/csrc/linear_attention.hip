@@ -6,10 +6,10 @@
 //
 // and then out = rmsnorm(o over all heads) * w * sigmoid(g) in the rows' type.  The state is a
 // float32 table with two versions of every sequence's row ([H][DK][DV]): a step reads the row
-// `seq_in` names and writes the whole row `seq_out` names.  The walk over a sequence's tokens
-// is a true recurrence: tokens are taken in order, one after the other, whatever the step
-// holds (a whole prompt, a portion, one token), so a position's result does not depend on how
-// its sequence was cut.
+// `seq_in` names and writes the whole row `seq_out` names.  `la_scan` walks
+// a sequence's tokens one after the other; `la_chunks` takes them 64 at a time as float32 matrix
+// products (recurrence_chunks.h), for steps that bring many tokens of a sequence.  Both sum in
+// float32, in another order: how a sequence was cut changes a result by float32 rounding alone.
 #include "common.h"
 #include "recurrence_chunks.h"
 

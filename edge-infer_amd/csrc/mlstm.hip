@@ -23,6 +23,8 @@
 // prefix sum and a prefix maximum over the lanes, so nothing but S itself is a chain.
 // The state is read from one row of the table and written, whole, to another (the table has two
 // versions a sequence).
+// `mlstm_chunks`: the same for steps that bring many tokens of a sequence, 64 at a time as float32
+// matrix products (recurrence_chunks.h).
 // `mlstm_out`: a wave a (row, head): RMS norm of the read-out, a weight as wide as all heads,
 // a sigmoid gate from the projection, one rounding.
 #include "common.h"

@@ -13,7 +13,9 @@
 // Per sequence the state row holds S of every head as [head][p][n] and then the last taps - 1
 // inputs of every convolved channel, oldest first.  A step reads the row `seq_in` names and
 // writes the whole row `seq_out` names, so a prompt may come whole, in portions or token by
-// token, and a step that fails changes nothing.
+// token, and a step that fails changes nothing.  `ssm_scan` walks the tokens one after the other;
+// `ssm_chunks` takes them 64 at a time as float32 matrix products (recurrence_chunks.h), for steps
+// that bring many tokens of a sequence.
 #include "common.h"
 #include "recurrence_chunks.h"
 
