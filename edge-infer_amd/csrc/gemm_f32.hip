@@ -221,19 +221,26 @@ gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, f
 // many rows of W for every X where that leaves enough blocks).  Two steps are asked for while
 // two are multiplied: more of them cost waves a SIMD and read slower (622 MB, one row: 2 + 2
 // steps 119 us, 4 + 4 steps 140, 8 + 8 steps 157).
-template <int RT, int CT>
+//
+// Where strips of 16 rows leave units without a block, a block owns ROWS = 8 (the instruction's other
+// rows repeat them and are not stored) and asks for DEEP = 4 steps at a time: what bounds it there is
+// how long a wave's own piece takes to arrive (one row, 2,048 -> 1,024: 9.2 -> 8.0 us, 3,072 -> 1,024:
+// 12.6 -> 10.5; 4 rows a block read no faster, 8 steps at a time neither).
+template <int RT, int CT, int ROWS = 16, int DEEP = 2>
 __global__ void __launch_bounds__(512)
 gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
                     int M, int N, int K, long long lda, long long ldw, long long ldc) {
-  constexpr int kDeep = 2;
+  constexpr int kDeep = DEEP;
+  static_assert(ROWS == 16 || CT == 1, "narrow strips come one a block");
   __shared__ f32x4 parts[kSegs][RT * CT][EI_WAVE];
   const int lane = threadIdx.x % EI_WAVE, wave = threadIdx.x / EI_WAVE;
   const int i16 = lane % 16, g = lane / 16;
-  const int n0 = blockIdx.x * 16 * CT;
+  const int n0 = blockIdx.x * ROWS * CT;
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
   const float* w[CT];
 #pragma unroll
-  for (int j = 0; j < CT; ++j) w[j] = W + static_cast<size_t>(min(n0 + 16 * j + i16, N - 1)) * ldw + 4 * g;
+  for (int j = 0; j < CT; ++j)
+    w[j] = W + static_cast<size_t>(min(n0 + 16 * j + i16 % ROWS, N - 1)) * ldw + 4 * g;
   const float* a[RT];
   bool row_live[RT];
 #pragma unroll
@@ -297,7 +304,7 @@ gemm_f32_few_kernel(const float* __restrict__ A, const float* __restrict__ W, fl
     for (int s = 0; s < kSegs; ++s) c[s] = parts[s][tile][l];
     const f32x4 sum = ((c[0] + c[1]) + (c[2] + c[3])) + ((c[4] + c[5]) + (c[6] + c[7]));
     const int m = 16 * (tile / CT) + l % 16, n = n0 + 16 * (tile % CT) + 4 * (l / 16);
-    if (m >= M) continue;
+    if (m >= M || 4 * (l / 16) >= ROWS) continue;
     float* dst = C + static_cast<size_t>(m) * ldc + n;
     if (quads && n + 4 <= N) {
       *reinterpret_cast<f32x4*>(dst) = sum;
@@ -325,7 +332,18 @@ extern "C" int ei_gemm_f32(const float* A, const float* W, float* C, int M, int 
 #define EI_FEW(RT, CT)                                                                   \
   gemm_f32_few_kernel<RT, CT><<<static_cast<unsigned>((N + 16LL * CT - 1) / (16 * CT)), 512, 0, stream>>>( \
       A, W, C, M, N, K, lda, ldw, ldc)
-    if (M <= 16) {
+    // Up to 16 rows and at most a strip of 8 a unit: strips of 8 (1,024 outputs, K 3,072: 12.6 -> 10.5
+    // us at one row, 15.0 -> 14.3 at 16; K 1,024 and 16 rows: 5.8 against 6.0, left as it was).  Up to
+    // 4 rows and at most a strip of 16 a unit: 4 steps at a time (4,096 outputs, K 1,024: 7.0 -> 6.5 us;
+    // at 16 rows, K 4,096, 20.0 against 21.1; with more strips than units 9.0 against 9.3).
+    const long long units_few = ei_compute_units();
+    if ((N + 7LL) / 8 <= units_few && (M <= 8 || (M <= 16 && K >= 2048))) {
+      gemm_f32_few_kernel<1, 1, 8, 4><<<static_cast<unsigned>((N + 7LL) / 8), 512, 0, stream>>>(
+          A, W, C, M, N, K, lda, ldw, ldc);
+    } else if ((N + 15LL) / 16 <= units_few && M <= 4) {
+      gemm_f32_few_kernel<1, 1, 16, 4><<<static_cast<unsigned>((N + 15LL) / 16), 512, 0, stream>>>(
+          A, W, C, M, N, K, lda, ldw, ldc);
+    } else if (M <= 16) {
       if (wide) EI_FEW(1, 2);
       else EI_FEW(1, 1);
     } else if (M <= 32) {

@@ -25,3 +25,23 @@ def test_products_of_every_number_of_rows_within_the_bound_and_the_same_bits(N, 
         if first is None:
             first = out
         assert torch.equal(out, first[:rows]), rows
+
+
+@pytest.mark.parametrize("N,K", [(7, 2052), (1027, 3072), (2047, 2048), (2048, 2064), (2055, 1024), (4096, 520)])
+def test_narrow_strips_of_few_rows(N, K):
+    """Strips of 8 outputs a block (up to 2,048 outputs) and of 16 with more steps asked for at a
+    time (up to 4,096), at their edges: the bound of the test above, and the same bits as 64 rows."""
+    from edge_infer_amd.csrc import lib
+    g = torch.Generator().manual_seed(N + K)
+    a = torch.randn(64, K, generator=g).to("cuda")
+    w = torch.randn(N, K, generator=g).to("cuda")
+    exact = a.double() @ w.double().T
+    bound = (K + 1) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+    wide = torch.full((64, N), float("nan"), device="cuda")
+    lib.gemm_f32(a, w, wide)
+    for rows in (16, 9, 8, 5, 4, 3, 1):
+        out = torch.full((rows + 1, N), 7.0, device="cuda")
+        lib.gemm_f32(a[:rows].contiguous(), w, out[:rows])
+        assert bool(((out[:rows].double() - exact[:rows]).abs() <= bound[:rows]).all()), rows
+        assert torch.equal(out[:rows], wide[:rows]), rows
+        assert bool((out[rows] == 7.0).all()), rows
