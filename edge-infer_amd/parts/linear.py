@@ -15,8 +15,8 @@ layout and lets the kernel read that.
 
 An optional bias [out] enters the sum before the one rounding, as in the reference
 (operators/src/cuda/execution.cu:307-317 fills the product's accumulator with it): as one
-more float32 slice beside the few-rows kernel's, as the library product's addend, or added
-to the float32 product.
+more float32 slice beside the few-rows kernel's, as what its sums start from where it writes a
+feed-forward's activation itself, as the library product's addend, or added to the float32 product.
 """
 from __future__ import annotations
 
