@@ -29,6 +29,7 @@ namespace ei {
 namespace delta_chunks {
 
 using chunks::chunk_place;
+using chunks::rows_of;
 using chunks::f32x16;
 using chunks::f32x4;
 using chunks::Gates;
@@ -88,10 +89,10 @@ solve_kernel(Rows in, Gates gates, Sequences seqs, float* __restrict__ scratch) 
   __shared__ double log_sums[kTokens];
   __shared__ float betas[kTokens], from_start[kTokens], to_end[kTokens];
   const int head = blockIdx.x, chunk = blockIdx.y, seq = blockIdx.z;
-  const int nt = min(kTokens, seqs.count[seq] - chunk * kTokens);
+  const int nt = min(kTokens, rows_of(seqs, seq) - chunk * kTokens);
   if (nt <= 0) return;
   const int first = seqs.row0[seq] + chunk * kTokens;
-  float* mine = scratch + (chunk_place(seqs.row0[seq], seq, chunk) * gridDim.x + head) * At::floats;
+  float* mine = scratch + (chunk_place(seqs, seq, chunk) * gridDim.x + head) * At::floats;
   const int lane = threadIdx.x % EI_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / EI_WAVE);
   const int i16 = lane % 16, g = lane / 16;
   {
@@ -301,13 +302,13 @@ walk_kernel(State state, Sequences seqs, const float* __restrict__ scratch, floa
   __shared__ __attribute__((aligned(16))) float s_lds[NC * 16 * SS];      // S by columns
   __shared__ __attribute__((aligned(16))) float u_lds[NC * 16 * US];      // U by columns
   const int head = blockIdx.x, seq = blockIdx.y, col0 = blockIdx.z * 16 * NC;
-  const int count = seqs.count[seq];
+  const int count = rows_of(seqs, seq);
   if (count <= 0) return;
   const int n_chunks = (count + kTokens - 1) / kTokens;
   const int lane = threadIdx.x % EI_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / EI_WAVE);
   const int i16 = lane % 16, g = lane / 16;
   const size_t apart = static_cast<size_t>(gridDim.x) * At::floats;
-  const float* base = scratch + (chunk_place(seqs.row0[seq], seq, 0) * gridDim.x + head) * At::floats;
+  const float* base = scratch + (chunk_place(seqs, seq, 0) * gridDim.x + head) * At::floats;
   // S of a head lies in the table by columns, [DV][DK]
   const size_t column = head * state.head_floats + static_cast<size_t>(col0 + i16) * DK;
   const float* in = state.rows + static_cast<size_t>(seqs.in[seq]) * state.row_floats + column;
@@ -345,7 +346,8 @@ walk_kernel(State state, Sequences seqs, const float* __restrict__ scratch, floa
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
   const size_t width = static_cast<size_t>(gridDim.x) * DV;
   auto step = [&](const Operands& in_chunk, int c) __attribute__((always_inline)) {
-    constexpr int kSums = NC == 1 ? 2 : 1;       // chains a sum (with more columns there are enough)
+    constexpr int kSums = 2;       // chains a sum (whatever NC, which depends on the whole step: a row's
+                                   // bits do not)
     f32x4 ws[NC][kSums], qs[NC][kSums];
 #pragma unroll
     for (int n = 0; n < NC; ++n)
@@ -371,7 +373,7 @@ walk_kernel(State state, Sequences seqs, const float* __restrict__ scratch, floa
     }
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
-      const f32x4 seen = kSums == 2 ? ws[n][0] + ws[n][kSums - 1] : ws[n][0];
+      const f32x4 seen = ws[n][0] + ws[n][1];
       *reinterpret_cast<f32x4*>(u_lds + (16 * n + i16) * US + 16 * wave + 4 * g) = in_chunk.u[n] - seen;
     }
     lds_barrier();                               // U is there, and S has been read
@@ -412,7 +414,7 @@ walk_kernel(State state, Sequences seqs, const float* __restrict__ scratch, floa
     float* dst = out + (static_cast<size_t>(seqs.row0[seq]) + t0) * width + head * DV + col0 + i16;
 #pragma unroll
     for (int n = 0; n < NC; ++n) {
-      const f32x4 read = kSums == 2 ? (o[n][0] + o[n][kSums - 1]) + (qs[n][0] + qs[n][kSums - 1]) : o[n][0] + qs[n][0];
+      const f32x4 read = (o[n][0] + o[n][1]) + (qs[n][0] + qs[n][1]);
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         if (t0 + r < count) dst[r * width + 16 * n] = read[r];

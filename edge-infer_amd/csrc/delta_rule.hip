@@ -483,7 +483,7 @@ delta_rule_kernel(const float* __restrict__ conv, int OW, int C, const TI* __res
                   const int32_t* __restrict__ seq_in, const int32_t* __restrict__ seq_out,
                   const int32_t* __restrict__ seq_count,
                   const int32_t* __restrict__ seq_row0, float* __restrict__ o_raw, int H, int G,
-                  int D, int DV, float q_scale, float unit_eps) {
+                  int D, int DV, float q_scale, float unit_eps, int most) {
   constexpr int DP = L * OWN;             // D rounded up to what the lanes of a column hold
   constexpr int CB = kThreads / L;        // columns of S a block holds
   constexpr int TILE = DP >= 256 ? kTile / 2 : kTile;   // (the widest keys: half, to fit 64 KB)
@@ -500,7 +500,7 @@ delta_rule_kernel(const float* __restrict__ conv, int OW, int C, const TI* __res
 
   const int seq = blockIdx.x;
   const int count = seq_count[seq];
-  if (count <= 0) return;                 // padding of a fixed-size batch
+  if (count <= 0 || count > most) return; // padding of a fixed-size batch, or one for the chunks
   const int row0 = seq_row0[seq];
   const int head = blockIdx.y, shared_head = head / (H / G);
   const int tid = threadIdx.x;
@@ -944,7 +944,7 @@ extern "C" int ei_delta_tail(const void* proj, int in_dtype, int nsplit, long lo
 // the beta and decay projections (H columns each) at beta_col and decay_col; key_decay: H D decays
 // follow the channels of a conv row instead (decay_col, a_log and dt_bias are then not read);
 // o_raw [N, H DV] float32.  n_seqs blocks walk
-// seq_count rows each from seq_row0.
+// seq_count rows each from seq_row0; sequences of more than `most` rows are left alone.
 extern "C" int ei_delta_rule(const float* conv, int OW, int key_decay, const void* proj, int in_dtype, int nsplit,
                              long long split_stride, int WP, int beta_col, int decay_col,
                              const float* a_log, const float* dt_bias, float* state,
@@ -952,7 +952,7 @@ extern "C" int ei_delta_rule(const float* conv, int OW, int key_decay, const voi
                              const int32_t* seq_out, const int32_t* seq_count,
                              const int32_t* seq_row0, float* o_raw,
                              int n_seqs, int H, int G, int D, int DV, float q_scale,
-                             float unit_eps, hipStream_t stream) {
+                             float unit_eps, int most, hipStream_t stream) {
   EI_REQUIRE(conv && proj && (key_decay || (a_log && dt_bias)) && state && seq_in && seq_out && seq_count && seq_row0 && o_raw,
              "delta_rule: null pointer");
   EI_REQUIRE(n_seqs > 0 && H > 0 && G > 0 && H % G == 0 && DV > 0, "delta_rule: bad head counts");
@@ -990,7 +990,7 @@ extern "C" int ei_delta_rule(const float* conv, int OW, int key_decay, const voi
   delta_rule_kernel<TI, LL, OO, KK><<<grid, kThreads, 0, stream>>>(                             \
       conv, OW, C, static_cast<const TI*>(proj), nsplit, ss, WP, beta_col, decay_col, a_log,    \
       dt_bias, state, static_cast<size_t>(state_stride), seq_in, seq_out, seq_count, seq_row0,  \
-      o_raw, H, G, D, DV, q_scale, unit_eps)
+      o_raw, H, G, D, DV, q_scale, unit_eps, most)
 #define EI_DELTA_O(TI, LL)                                  \
   do {                                                      \
     if (own == 8 && key_decay) EI_DELTA(TI, LL, 8, true);   \
@@ -1017,11 +1017,10 @@ extern "C" int ei_delta_rule(const float* conv, int OW, int key_decay, const voi
   EI_LAUNCH_CHECK();
 }
 
-// proj: [nsplit] slices of rows WP wide whose gate logits begin at gate_col; sigmoid_gate: the gate
-// is their sigmoid, not their silu.
 // The recurrence with one decay a head over a prompt's rows in chunks (see delta_chunks.h), for
-// heads of 64 or 128 elements.  scratch: `scratch_floats` floats, at least (rows / 64 + n_seqs) * H
-// chunks; longest: the most rows that a sequence brings.
+// heads of 64 or 128 elements.  Sequences of fewer than `least` rows are left to the walk.
+// scratch: `scratch_floats` floats, at least chunk_places chunks of H heads; longest: the most
+// rows that a sequence brings.
 extern "C" int ei_delta_chunk_floats(int D, int DV) { return ei::delta_chunks::chunk_floats(D, DV); }
 
 extern "C" int ei_delta_chunks(const float* conv, int OW, const void* proj, int in_dtype, int nsplit,
@@ -1031,13 +1030,13 @@ extern "C" int ei_delta_chunks(const float* conv, int OW, const void* proj, int 
                                const int32_t* seq_out, const int32_t* seq_count,
                                const int32_t* seq_row0, float* o_raw, float* scratch,
                                long long scratch_floats, int rows, int n_seqs, int H, int G, int D,
-                               int DV, float q_scale, float unit_eps, int longest,
+                               int DV, float q_scale, float unit_eps, int longest, int least,
                                hipStream_t stream) {
   EI_REQUIRE(conv && proj && a_log && dt_bias && state && seq_in && seq_out && seq_count && seq_row0 &&
                  o_raw && scratch,
              "delta_chunks: null pointer");
   EI_REQUIRE(rows > 0 && n_seqs > 0 && H > 0 && G > 0 && H % G == 0 && nsplit >= 1 && longest > 0 &&
-                 longest <= rows,
+                 longest <= rows && least > 0,
              "delta_chunks: bad sizes");
   EI_REQUIRE(ei::delta_chunks::sizes_fit(D, DV), "delta_chunks: heads of 64 or 128 elements");
   EI_REQUIRE(in_dtype == EI_F32 || in_dtype == EI_BF16, "delta_chunks: unknown dtype");
@@ -1047,7 +1046,7 @@ extern "C" int ei_delta_chunks(const float* conv, int OW, const void* proj, int 
              "delta_chunks: rows too narrow or unaligned");
   EI_REQUIRE(H <= 65535 && n_seqs <= 65535 && (longest + 63) / 64 <= 65535,
              "delta_chunks: too many heads, sequences or rows");
-  EI_REQUIRE(scratch_floats >= (rows / 64 + 1LL * n_seqs) * H * ei_delta_chunk_floats(D, DV),
+  EI_REQUIRE(scratch_floats >= ei::chunks::chunk_places(rows, n_seqs, least) * H * ei_delta_chunk_floats(D, DV),
              "delta_chunks: scratch too small");
   namespace dc = ei::delta_chunks;
   const dc::Rows in{conv, static_cast<size_t>(OW), 0, G * D, 2 * G * D, H / G, q_scale, unit_eps};
@@ -1062,7 +1061,7 @@ extern "C" int ei_delta_chunks(const float* conv, int OW, const void* proj, int 
   gates.at = beta_col;
   gates.at2 = decay_col;
   const ei::chunks::State table{state, static_cast<size_t>(state_stride), static_cast<size_t>(D) * DV};
-  const ei::chunks::Sequences seqs{seq_in, seq_out, seq_count, seq_row0};
+  const ei::chunks::Sequences seqs{seq_in, seq_out, seq_count, seq_row0, least};
 #define EI_DC(DK_, DV_) dc::launch<DK_, DV_>(in, gates, table, seqs, scratch, o_raw, n_seqs, H, longest, stream)
   if (D == 128 && DV == 128) EI_DC(128, 128);
   else if (D == 128) EI_DC(128, 64);
@@ -1072,6 +1071,8 @@ extern "C" int ei_delta_chunks(const float* conv, int OW, const void* proj, int 
   EI_LAUNCH_CHECK();
 }
 
+// proj: [nsplit] slices of rows WP wide whose gate logits begin at gate_col; sigmoid_gate: the gate
+// is their sigmoid, not their silu.
 extern "C" int ei_delta_out(const float* o_raw, const void* proj, int in_dtype, int nsplit,
                             long long split_stride, int WP, int gate_col, int sigmoid_gate,
                             const float* norm_w, float eps, const int32_t* row_seq, void* out, int out_dtype, int N,

@@ -21,6 +21,7 @@ from . import build
 F32, BF16 = 0, 1
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16}
 PAGE_TOKENS = 64
+EVERY = 2 ** 31 - 1       # `most` rows of a sequence: sequences of any length
 
 _SIGNATURES = {
     "rowwise": {
@@ -72,12 +73,12 @@ _SIGNATURES = {
                         c_int, c_void_p],
         "ei_ssm_scan": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p,
                         c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p,
-                        c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
+                        c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p],
         "ei_ssm_chunk_floats": [c_int, c_int],
         "ei_ssm_chunks": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p,
                           c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p,
                           c_void_p, c_void_p, c_void_p, c_longlong, c_int, c_int, c_int, c_int,
-                          c_int, c_int, c_int, c_int, c_void_p],
+                          c_int, c_int, c_int, c_int, c_int, c_void_p],
         "ei_ssm_out": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p,
                        c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     },
@@ -99,11 +100,11 @@ _SIGNATURES = {
     "linear_attention": {
         "ei_la_scan": [c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p, c_void_p,
                        c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
-                       c_int, c_int, c_void_p],
+                       c_int, c_int, c_int, c_void_p],
         "ei_la_chunk_floats": [c_int, c_int],
         "ei_la_chunks": [c_void_p, c_longlong, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                          c_void_p, c_void_p, c_void_p, c_longlong, c_int, c_int, c_int, c_int,
-                         c_int, c_int, c_void_p],
+                         c_int, c_int, c_int, c_void_p],
         "ei_la_activate": [c_void_p, c_int, c_int, c_longlong, c_longlong, c_void_p, c_int, c_int,
                            c_void_p],
         "ei_la_out": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_longlong, c_longlong,
@@ -141,12 +142,12 @@ _SIGNATURES = {
         "ei_delta_rule": [c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_longlong, c_int, c_int, c_int,
                           c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p,
                           c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_float, c_float,
-                          c_void_p],
+                          c_int, c_void_p],
         "ei_delta_chunk_floats": [c_int, c_int],
         "ei_delta_chunks": [c_void_p, c_int, c_void_p, c_int, c_int, c_longlong, c_int, c_int, c_int,
                             c_void_p, c_void_p, c_void_p, c_longlong, c_void_p, c_void_p, c_void_p,
                             c_void_p, c_void_p, c_void_p, c_longlong, c_int, c_int, c_int, c_int,
-                            c_int, c_int, c_float, c_float, c_int, c_void_p],
+                            c_int, c_int, c_float, c_float, c_int, c_int, c_void_p],
         "ei_delta_out": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_int, c_int, c_int, c_void_p,
                          c_float, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p],
     },
@@ -195,10 +196,11 @@ _SIGNATURES = {
         "ei_mlstm_chunk_floats": [c_int, c_int],
         "ei_mlstm_chunks": [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p,
                             c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_longlong, c_int,
-                            c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_void_p],
+                            c_int, c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_int,
+                            c_void_p],
         "ei_mlstm_walk": [c_void_p, c_int, c_int, c_longlong, c_void_p, c_void_p, c_void_p,
                           c_longlong, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int,
-                          c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_void_p],
+                          c_int, c_int, c_int, c_float, c_float, c_float, c_int, c_int, c_void_p],
         "ei_mlstm_out": [c_void_p, c_void_p, c_int, c_int, c_longlong, c_void_p, c_float,
                          c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p],
     },
@@ -1081,10 +1083,10 @@ def mlstm_proj_width(heads: int, key_dim: int, value_dim: int) -> int:
 
 
 def mlstm_walk(proj, i_bias, f_bias, state, seq_in, seq_out, seq_count, seq_row0, o_raw, heads,
-               key_dim, value_dim, cap, q_scale, bottom_eps) -> None:
+               key_dim, value_dim, cap, q_scale, bottom_eps, most: int = EVERY) -> None:
     """The matrix memory's walk over the rows of a step (see mlstm.hip): proj [rows, width] or
     float32 slices; state float32 [table rows, state floats]; o_raw float32 [rows, heads *
-    value_dim]."""
+    value_dim]; sequences of more than `most` rows are left alone."""
     lib = library("mlstm")
     n, width, nsplit, stride = _rows_of(proj, "proj")
     if width != mlstm_proj_width(heads, key_dim, value_dim):
@@ -1105,20 +1107,22 @@ def mlstm_walk(proj, i_bias, f_bias, state, seq_in, seq_out, seq_count, seq_row0
         _gpu(seq_in, "seq_in", torch.int32), _gpu(seq_out, "seq_out", torch.int32),
         _gpu(seq_count, "seq_count", torch.int32), _gpu(seq_row0, "seq_row0", torch.int32),
         _gpu(o_raw, "o_raw", torch.float32), n_seqs, heads, key_dim, value_dim, float(cap),
-        float(q_scale), float(bottom_eps), n, _stream())
+        float(q_scale), float(bottom_eps), n, int(most), _stream())
     _check(lib, status, "mlstm_walk")
 
 
-def mlstm_chunk_scratch(rows, seqs, heads, key_dim, value_dim) -> int:
-    """float32 elements of scratch that `mlstm_chunks` wants for a step of so many rows."""
-    return _chunk_scratch("mlstm", "ei_mlstm_chunk_floats", rows, seqs, heads, key_dim, value_dim)
+def mlstm_chunk_scratch(rows, seqs, heads, key_dim, value_dim, least=1) -> int:
+    """float32 elements of scratch that `mlstm_chunks` wants for a step of so many rows and
+    sequences, those of `least` rows or more being its own."""
+    return _chunk_scratch("mlstm", "ei_mlstm_chunk_floats", rows, seqs, least, heads, key_dim, value_dim)
 
 
 def mlstm_chunks(proj, i_bias, f_bias, state, seq_in, seq_out, seq_count, seq_row0, o_raw, scratch,
-                 heads, key_dim, value_dim, cap, q_scale, bottom_eps, longest: int) -> None:
+                 heads, key_dim, value_dim, cap, q_scale, bottom_eps, longest: int,
+                 least: int = 1) -> None:
     """What `mlstm_walk` does, by chunks of 64 tokens: heads of 64 or 128 elements, a projection
     [rows, width] in one piece whose width is a multiple of 4; longest: the most rows that a
-    sequence of the step brings."""
+    sequence of the step brings; sequences of fewer than `least` are left alone."""
     lib = library("mlstm")
     n, width, nsplit, _ = _rows_of(proj, "proj")
     if nsplit != 1 or width != mlstm_proj_width(heads, key_dim, value_dim):
@@ -1139,7 +1143,7 @@ def mlstm_chunks(proj, i_bias, f_bias, state, seq_in, seq_out, seq_count, seq_ro
         _gpu(seq_count, "seq_count", torch.int32), _gpu(seq_row0, "seq_row0", torch.int32),
         _gpu(o_raw, "o_raw", torch.float32), _gpu(scratch, "scratch", torch.float32),
         scratch.numel(), n, n_seqs, heads, key_dim, value_dim, float(cap), float(q_scale),
-        float(bottom_eps), int(longest), _stream())
+        float(bottom_eps), int(longest), int(least), _stream())
     _check(lib, status, "mlstm_chunks")
 
 
@@ -1692,11 +1696,11 @@ def delta_tail(proj, state, shape: DeltaShape, rows, seq_in, seq_out, seq_count,
 
 
 def delta_rule(conv, proj, a_log, dt_bias, state, shape: DeltaShape, seq_in, seq_out, seq_count,
-               seq_row0, o_raw, q_scale: float, unit_eps: float) -> None:
+               seq_row0, o_raw, q_scale: float, unit_eps: float, most: int = EVERY) -> None:
     """The recurrence over every sequence's rows of this step, in order; reads S from row
     seq_in[s] of `state` and writes it to row seq_out[s]; o_raw [rows, heads * value_dim]
     float32 receives S^T q of every row.  With a decay per key channel the decays come with the
-    rows of `conv` (a_log and dt_bias None)."""
+    rows of `conv` (a_log and dt_bias None).  Sequences of more than `most` rows are left alone."""
     lib = library("delta_rule")
     rows = conv.shape[0]
     n_seqs = seq_count.numel()
@@ -1719,20 +1723,23 @@ def delta_rule(conv, proj, a_log, dt_bias, state, shape: DeltaShape, seq_in, seq
                                _gpu(seq_row0, "seq_row0", torch.int32),
                                _gpu(o_raw, "o_raw", torch.float32), n_seqs, shape.n_heads,
                                shape.n_kv_heads, shape.key_dim, shape.value_dim, float(q_scale),
-                               float(unit_eps), _stream())
+                               float(unit_eps), int(most), _stream())
     _check(lib, status, "delta_rule")
 
 
-def delta_chunk_scratch(rows, seqs, shape: DeltaShape) -> int:
-    """float32 elements of scratch that `delta_chunks` wants for a step of so many rows."""
-    return _chunk_scratch("delta_rule", "ei_delta_chunk_floats", rows, seqs, shape.n_heads,
+def delta_chunk_scratch(rows, seqs, shape: DeltaShape, least=1) -> int:
+    """float32 elements of scratch that `delta_chunks` wants for a step of so many rows and
+    sequences, those of `least` rows or more being its own."""
+    return _chunk_scratch("delta_rule", "ei_delta_chunk_floats", rows, seqs, least, shape.n_heads,
                           shape.key_dim, shape.value_dim)
 
 
 def delta_chunks(conv, proj, a_log, dt_bias, state, shape: DeltaShape, seq_in, seq_out, seq_count,
-                 seq_row0, o_raw, q_scale: float, unit_eps: float, scratch, longest: int) -> None:
+                 seq_row0, o_raw, q_scale: float, unit_eps: float, scratch, longest: int,
+                 least: int = 1) -> None:
     """What `delta_rule` does with one decay a head, by chunks of 64 tokens: heads of 64 or 128
-    elements; longest: the most rows that a sequence of the step brings."""
+    elements; longest: the most rows that a
+    sequence of the step brings; sequences of fewer than `least` are left alone."""
     lib = library("delta_rule")
     rows = conv.shape[0]
     n_seqs = seq_count.numel()
@@ -1753,7 +1760,7 @@ def delta_chunks(conv, proj, a_log, dt_bias, state, shape: DeltaShape, seq_in, s
         _gpu(seq_row0, "seq_row0", torch.int32), _gpu(o_raw, "o_raw", torch.float32),
         _gpu(scratch, "scratch", torch.float32), scratch.numel(), rows, n_seqs, shape.n_heads,
         shape.n_kv_heads, shape.key_dim, shape.value_dim, float(q_scale), float(unit_eps),
-        int(longest), _stream())
+        int(longest), int(least), _stream())
     _check(lib, status, "delta_chunks")
 
 
@@ -1846,8 +1853,8 @@ def ssm_conv(proj, conv_w, conv_b, state, shape: SsmShape, row_pos, row_seq, seq
 
 
 def ssm_scan(conv, proj, a_log, dt_bias, d_skip, state, shape: SsmShape, seq_in, seq_out,
-             seq_count, seq_row0, y_raw) -> None:
-    """The recurrence over every sequence's rows: S <- exp(-exp(a_log) dt) S + dt B x^T from row
+             seq_count, seq_row0, y_raw, most: int = EVERY) -> None:
+    """The recurrence over the rows of every sequence of at most `most`: S <- exp(-exp(a_log) dt) S + dt B x^T from row
     `seq_in[s]` of `state`, y = S^T C + d_skip x to `y_raw` [n, inner] float32, the last S to row
     `seq_out[s]`; dt = softplus(proj's dt column + dt_bias)."""
     lib = library("ssm")
@@ -1868,19 +1875,23 @@ def ssm_scan(conv, proj, a_log, dt_bias, d_skip, state, shape: SsmShape, seq_in,
         _ssm_state(state, shape), state.shape[1], _gpu(seq_in, "seq_in", torch.int32),
         _gpu(seq_out, "seq_out", torch.int32), _gpu(seq_count, "seq_count", torch.int32),
         _gpu(seq_row0, "seq_row0", torch.int32), _gpu(y_raw, "y_raw", torch.float32), n_seqs,
-        *shape.sizes, _stream())
+        *shape.sizes, int(most), _stream())
     _check(lib, status, "ssm_scan")
 
 
-def ssm_chunk_scratch(rows, seqs, shape: SsmShape) -> int:
-    """float32 elements of scratch that `ssm_chunks` wants for a step of so many rows."""
-    return _chunk_scratch("ssm", "ei_ssm_chunk_floats", rows, seqs, shape.heads, shape.head_dim, shape.state)
+def ssm_chunk_scratch(rows, seqs, shape: SsmShape, least=1) -> int:
+    """float32 elements of scratch that `ssm_chunks` wants for a step of so many rows and
+    sequences, those of `least` rows or more being its own."""
+    return _chunk_scratch("ssm", "ei_ssm_chunk_floats", rows, seqs, least, shape.heads,
+                          shape.head_dim, shape.state)
 
 
 def ssm_chunks(conv, proj, a_log, dt_bias, d_skip, state, shape: SsmShape, seq_in, seq_out,
-               seq_count, seq_row0, y_raw, scratch, longest: int) -> None:
+               seq_count, seq_row0, y_raw, scratch, longest: int,
+               least: int = 1) -> None:
     """What `ssm_scan` does, by chunks of 64 tokens: states of 64 or 128 rows and columns;
-    longest: the most rows that a sequence of the step brings."""
+    longest: the most rows that a
+    sequence of the step brings; sequences of fewer than `least` are left alone."""
     lib = library("ssm")
     n = y_raw.shape[0]
     nsplit, stride = _ssm_proj(proj, n, shape)
@@ -1900,7 +1911,7 @@ def ssm_chunks(conv, proj, a_log, dt_bias, d_skip, state, shape: SsmShape, seq_i
         _gpu(seq_out, "seq_out", torch.int32), _gpu(seq_count, "seq_count", torch.int32),
         _gpu(seq_row0, "seq_row0", torch.int32), _gpu(y_raw, "y_raw", torch.float32),
         _gpu(scratch, "scratch", torch.float32), scratch.numel(), n, n_seqs, *shape.sizes,
-        int(longest), _stream())
+        int(longest), int(least), _stream())
     _check(lib, status, "ssm_chunks")
 
 
@@ -2075,26 +2086,36 @@ def input_conv(h, weight, state, part: int, parts: int, row_pos, row_seq, seq_in
 
 
 # Recurrences by chunks of a prompt's tokens (csrc/recurrence_chunks.h): the scratch that the
-# chunks' states take, and the head sizes that the kernels know.
+# chunks' states take, and the head sizes that the kernels know.  Which sequences go by chunks is a
+# matter of each sequence's own rows (`least` here, `most` of the token-by-token kernels), so that
+# its results do not depend on what else a step holds.
 CHUNK_TOKENS = 64
 CHUNK_SIZES = (64, 128)
 
 
-def _chunk_scratch(library_name: str, symbol: str, rows: int, seqs: int, heads: int, dk: int,
-                   dv: int) -> int:
-    each = getattr(library(library_name), symbol)(dk, dv)
-    return (rows // CHUNK_TOKENS + seqs) * heads * each
+@functools.lru_cache(maxsize=None)
+def _chunk_floats(library_name: str, symbol: str, dk: int, dv: int) -> int:
+    return getattr(library(library_name), symbol)(dk, dv)
 
 
-def la_chunk_scratch(rows, seqs, heads, key_dim, value_dim) -> int:
-    """float32 elements of scratch that `la_chunks` wants for a step of so many rows."""
-    return _chunk_scratch("linear_attention", "ei_la_chunk_floats", rows, seqs, heads, key_dim, value_dim)
+def _chunk_scratch(library_name: str, symbol: str, rows: int, seqs: int, least: int, heads: int,
+                   dk: int, dv: int) -> int:
+    each = _chunk_floats(library_name, symbol, dk, dv)
+    return (rows // CHUNK_TOKENS + min(rows // least, seqs)) * heads * each
+
+
+def la_chunk_scratch(rows, seqs, heads, key_dim, value_dim, least=1) -> int:
+    """float32 elements of scratch that `la_chunks` wants for a step of so many rows and
+    sequences, those of `least` rows or more being its own."""
+    return _chunk_scratch("linear_attention", "ei_la_chunk_floats", rows, seqs, least, heads, key_dim, value_dim)
 
 
 def la_chunks(act, decay, state, seq_in, seq_out, seq_count, seq_row0, o_raw, scratch, heads,
-              key_dim, value_dim, longest: int) -> None:
+              key_dim, value_dim, longest: int,
+              least: int = 1) -> None:
     """What `la_scan` does with activated rows, by chunks of 64 tokens: heads of 64 or 128
-    elements; longest: the most rows that a sequence of the step brings."""
+    elements; longest: the most rows that a
+    sequence of the step brings; sequences of fewer than `least` are left alone."""
     lib = library("linear_attention")
     n, stride = act.shape
     n_seqs = seq_count.numel()
@@ -2110,7 +2131,7 @@ def la_chunks(act, decay, state, seq_in, seq_out, seq_count, seq_row0, o_raw, sc
         _gpu(seq_out, "seq_out", torch.int32), _gpu(seq_count, "seq_count", torch.int32),
         _gpu(seq_row0, "seq_row0", torch.int32), _gpu(o_raw, "o_raw", torch.float32),
         _gpu(scratch, "scratch", torch.float32), scratch.numel(), n, n_seqs, heads, key_dim,
-        value_dim, int(longest), _stream())
+        value_dim, int(longest), int(least), _stream())
     _check(lib, status, "la_chunks")
 
 
@@ -2134,12 +2155,13 @@ def la_activate(proj, act) -> None:
 
 
 def la_scan(proj, decay, state, seq_in, seq_out, seq_count, seq_row0, o_raw, heads, key_dim,
-            value_dim, activated: bool = False) -> None:
+            value_dim, activated: bool = False, most: int = EVERY) -> None:
     """The recurrence of linear attention with a decay per head over the rows of every
     sequence: proj rows [q | k | v | ...] ([n, g] or float32 slices [s, n, g]), silu on all
     three, S_t = decay_h S_(t-1) + k_t v_t^T, o_raw [n, heads * value_dim] float32 = S_t^T q_t.
     state: float32 rows of heads * key_dim * value_dim, two versions (`seq_in`, `seq_out`).
-    activated: the rows hold q, k and v as `la_activate` left them, and silu is not taken again."""
+    activated: the rows hold q, k and v as `la_activate` left them, and silu is not taken again;
+    sequences of more than `most` rows are left alone."""
     lib = library("linear_attention")
     if activated and proj.dtype != torch.float32:
         raise KernelError("la_scan: activated rows are float32")
@@ -2161,7 +2183,7 @@ def la_scan(proj, decay, state, seq_in, seq_out, seq_count, seq_row0, o_raw, hea
         _gpu(seq_in, "seq_in", torch.int32), _gpu(seq_out, "seq_out", torch.int32),
         _gpu(seq_count, "seq_count", torch.int32), _gpu(seq_row0, "seq_row0", torch.int32),
         _gpu(o_raw, "o_raw", torch.float32), n_seqs, heads, key_dim, value_dim,
-        int(bool(activated)), _stream())
+        int(bool(activated)), int(most), _stream())
     _check(lib, status, "la_scan")
 
 

@@ -41,7 +41,7 @@ la_scan_kernel(const TI* __restrict__ proj, int nsplit, size_t split_stride, siz
                const float* __restrict__ decay, const float* state_in_table, float* state_out_table,
                const int32_t* __restrict__ seq_in, const int32_t* __restrict__ seq_out,
                const int32_t* __restrict__ seq_count, const int32_t* __restrict__ seq_row0,
-               float* __restrict__ o_raw, int H, int DK, int DV) {
+               float* __restrict__ o_raw, int H, int DK, int DV, int most) {
   constexpr int G = kThreads / COLS;
   constexpr int DKP = G * R;
   constexpr int QK_PER = kTile * DKP / kThreads;      // q (and k) values a thread fetches a tile
@@ -52,7 +52,7 @@ la_scan_kernel(const TI* __restrict__ proj, int nsplit, size_t split_stride, siz
   __shared__ float part[kTile][G][COLS];
   const int seq = blockIdx.x, head = blockIdx.y, col0 = blockIdx.z * COLS;
   const int count = seq_count[seq];
-  if (count <= 0) return;                       // a padding sequence
+  if (count <= 0 || count > most) return;       // a padding sequence, or one for the chunks
   const int t = threadIdx.x, c = t % COLS, g = t / COLS;
   const int col = col0 + c;
   const bool col_live = col < DV;
@@ -195,12 +195,12 @@ extern "C" long long ei_la_state_floats(int H, int DK, int DV) {
 }
 
 // proj: [nsplit][N, row_stride] of proj_dtype, rows as above; state: float32 rows of
-// H * DK * DV; o_raw: float32 [N, H * DV].
+// H * DK * DV; o_raw: float32 [N, H * DV]; sequences of more than `most` rows are left alone.
 extern "C" int ei_la_scan(const void* proj, int proj_dtype, int nsplit, long long split_stride,
                           long long row_stride, const float* decay, float* state,
                           const int32_t* seq_in, const int32_t* seq_out, const int32_t* seq_count,
                           const int32_t* seq_row0, float* o_raw, int n_seqs, int H, int DK, int DV,
-                          int activated, hipStream_t stream) {
+                          int activated, int most, hipStream_t stream) {
   EI_REQUIRE(proj && decay && state && seq_in && seq_out && seq_count && seq_row0 && o_raw,
              "la_scan: null pointer");
   EI_REQUIRE(n_seqs > 0 && H > 0 && DK >= 1 && DK <= 256 && DV >= 1 && nsplit >= 1,
@@ -219,11 +219,11 @@ extern "C" int ei_la_scan(const void* proj, int proj_dtype, int nsplit, long lon
     if (activated)                                                                             \
       la_scan_kernel<TI, R, COLS, AHEAD, false><<<grid, kThreads, 0, stream>>>(                \
           static_cast<const TI*>(proj), nsplit, ss, rs, decay, state, state, seq_in, seq_out,  \
-          seq_count, seq_row0, o_raw, H, DK, DV);                                              \
+          seq_count, seq_row0, o_raw, H, DK, DV, most);                                              \
     else                                                                                       \
       la_scan_kernel<TI, R, COLS, AHEAD, true><<<grid, kThreads, 0, stream>>>(                 \
           static_cast<const TI*>(proj), nsplit, ss, rs, decay, state, state, seq_in, seq_out,  \
-          seq_count, seq_row0, o_raw, H, DK, DV);                                              \
+          seq_count, seq_row0, o_raw, H, DK, DV, most);                                              \
   } while (0)
 #define EI_LA_T(TI)                                       \
   do {                                                    \
@@ -286,8 +286,9 @@ extern "C" int ei_la_out(const float* o_raw, const void* proj, int proj_dtype, i
 }
 
 // The recurrence over a prompt's rows in chunks (see recurrence_chunks.h).  act: float32 [N,
-// row_stride] with q, k and v as `ei_la_activate` leaves them; scratch: `scratch_floats` floats, at
-// least (N / 64 + n_seqs) * H chunks; longest: the most rows that a sequence brings.
+// row_stride] with q, k and v as `ei_la_activate` leaves them.  Sequences of fewer than `least` rows are left to the walk.
+// scratch: `scratch_floats` floats, at least chunk_places chunks of H heads; longest: the most
+// rows that a sequence brings.
 extern "C" int ei_la_chunk_floats(int DK, int DV) {
   return static_cast<int>(ei::chunks::chunk_floats(ei::chunks::kFixed, DK, DV));
 }
@@ -296,23 +297,24 @@ extern "C" int ei_la_chunks(const float* act, long long row_stride, const float*
                             const int32_t* seq_in, const int32_t* seq_out, const int32_t* seq_count,
                             const int32_t* seq_row0, float* o_raw, float* scratch,
                             long long scratch_floats, int N, int n_seqs, int H, int DK, int DV,
-                            int longest, hipStream_t stream) {
+                            int longest, int least, hipStream_t stream) {
   EI_REQUIRE(act && decay && state && seq_in && seq_out && seq_count && seq_row0 && o_raw && scratch,
              "la_chunks: null pointer");
-  EI_REQUIRE(N > 0 && n_seqs > 0 && H > 0 && longest > 0 && longest <= N, "la_chunks: sizes must be positive");
+  EI_REQUIRE(N > 0 && n_seqs > 0 && H > 0 && longest > 0 && longest <= N && least > 0,
+             "la_chunks: sizes must be positive");
   EI_REQUIRE(ei::chunks::sizes_fit(DK, DV), "la_chunks: heads of 64 or 128 elements");
   EI_REQUIRE(row_stride >= 2LL * H * DK + 1LL * H * DV && row_stride % 4 == 0 &&
                  (reinterpret_cast<uintptr_t>(act) & 15) == 0 && (reinterpret_cast<uintptr_t>(scratch) & 15) == 0,
              "la_chunks: rows narrower than q, k and v, or unaligned");
   EI_REQUIRE(H <= 65535 && n_seqs <= 65535, "la_chunks: too many heads or sequences");
-  EI_REQUIRE(scratch_floats >= (N / 64 + 1LL * n_seqs) * H * ei_la_chunk_floats(DK, DV),
+  EI_REQUIRE(scratch_floats >= ei::chunks::chunk_places(N, n_seqs, least) * H * ei_la_chunk_floats(DK, DV),
              "la_chunks: scratch too small");
   using namespace ei::chunks;
   const Rows at_row{static_cast<size_t>(row_stride), 0, H * DK, 2 * H * DK, 1};
   Gates gates{};
   gates.c0 = decay;
   const State table{state, static_cast<size_t>(H) * DK * DV, static_cast<size_t>(DK) * DV};
-  const Sequences seqs{seq_in, seq_out, seq_count, seq_row0};
+  const Sequences seqs{seq_in, seq_out, seq_count, seq_row0, least};
   launch_sized<kFixed, float>(DK, DV, act, at_row, gates, table, seqs, scratch, o_raw, n_seqs, H,
                               longest, stream);
   EI_LAUNCH_CHECK();

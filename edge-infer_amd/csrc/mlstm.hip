@@ -99,7 +99,7 @@ mlstm_walk_kernel(const TI* __restrict__ proj, int nsplit, size_t split_stride,
                   const int32_t* __restrict__ seq_in, const int32_t* __restrict__ seq_out,
                   const int32_t* __restrict__ seq_count, const int32_t* __restrict__ seq_row0,
                   float* __restrict__ o_raw, int heads, int dim, int vdim, int L, float cap,
-                  float q_scale, float bottom_eps, int tile_rows) {
+                  float q_scale, float bottom_eps, int tile_rows, int most) {
   // (tile_rows: tokens in LDS at a time, kTile, or 1 where every sequence brings one token: a
   // decode step then needs a sixteenth of the LDS, and many more waves fit a compute unit)
   extern __shared__ float lds[];
@@ -115,7 +115,7 @@ mlstm_walk_kernel(const TI* __restrict__ proj, int nsplit, size_t split_stride,
 
   const int seq = blockIdx.x / heads, a = blockIdx.x % heads;
   const int count = seq_count[seq];
-  if (count <= 0) return;                      // padding of a fixed-size batch
+  if (count <= 0 || count > most) return;      // padding of a fixed-size batch, or one for the chunks
   const int row0 = seq_row0[seq];
   const Columns col_of = columns_of(heads, dim, vdim);
   const int P = col_of.width;
@@ -422,13 +422,14 @@ extern "C" int ei_mlstm_proj_width(int heads, int dim, int vdim) {
 }
 
 // proj: [nsplit][N, width]; state: rows of `state_stride` floats; seq_in / seq_out: the row
-// each sequence's state is read from and written to; o_raw: float32 [N, heads * vdim].
+// each sequence's state is read from and written to; o_raw: float32 [N, heads * vdim]; sequences of
+// more than `most` rows are left alone.
 extern "C" int ei_mlstm_walk(const void* proj, int dtype, int nsplit, long long split_stride,
                              const float* i_bias, const float* f_bias, float* state,
                              long long state_stride, const int32_t* seq_in, const int32_t* seq_out,
                              const int32_t* seq_count, const int32_t* seq_row0, float* o_raw,
                              int n_seqs, int heads, int dim, int vdim, float cap, float q_scale,
-                             float bottom_eps, int rows, hipStream_t stream) {
+                             float bottom_eps, int rows, int most, hipStream_t stream) {
   EI_REQUIRE(n_seqs > 0 && heads > 0 && vdim > 0 && nsplit >= 1 && rows >= 1, "mlstm_walk: bad sizes");
   EI_REQUIRE(dim >= 1 && dim <= 256, "mlstm_walk: the key size must lie in 1..256");
   EI_REQUIRE(cap > 0.f, "mlstm_walk: the cap of the gates must be positive");
@@ -457,7 +458,7 @@ extern "C" int ei_mlstm_walk(const void* proj, int dtype, int nsplit, long long 
   mlstm_walk_kernel<TI, NC><<<grid, kThreads, lds, stream>>>(                                  \
       static_cast<const TI*>(proj), nsplit, ss, i_bias, f_bias, state,                         \
       static_cast<size_t>(state_stride), seq_in, seq_out, seq_count, seq_row0, o_raw, heads,   \
-      dim, vdim, L, cap, q_scale, bottom_eps, tile_rows)
+      dim, vdim, L, cap, q_scale, bottom_eps, tile_rows, most)
 #define EI_WALK_COLS(TI)              \
   do {                                \
     if (nc == 4) EI_WALK(TI, 4);      \
@@ -474,8 +475,9 @@ extern "C" int ei_mlstm_walk(const void* proj, int dtype, int nsplit, long long 
 
 // The walk over a prompt's rows in chunks (see recurrence_chunks.h): what `ei_mlstm_walk` does for
 // heads of 64 or 128 elements and a projection in one piece whose rows are multiples of 4
-// elements.  scratch: `scratch_floats` floats, at least (rows / 64 + n_seqs) * heads chunks;
-// longest: the most rows that a sequence brings.
+// elements.  Sequences of fewer than `least` rows are left to the walk.
+// scratch: `scratch_floats` floats, at least chunk_places chunks of all heads; longest: the most
+// rows that a sequence brings.
 extern "C" int ei_mlstm_chunk_floats(int dim, int vdim) {
   return static_cast<int>(ei::chunks::chunk_floats(ei::chunks::kMatrix, dim, vdim));
 }
@@ -485,9 +487,9 @@ extern "C" int ei_mlstm_chunks(const void* proj, int dtype, const float* i_bias,
                                const int32_t* seq_out, const int32_t* seq_count,
                                const int32_t* seq_row0, float* o_raw, float* scratch,
                                long long scratch_floats, int rows, int n_seqs, int heads, int dim,
-                               int vdim, float cap, float q_scale, float bottom_eps, int longest,
+                               int vdim, float cap, float q_scale, float bottom_eps, int longest, int least,
                                hipStream_t stream) {
-  EI_REQUIRE(n_seqs > 0 && heads > 0 && rows >= 1 && longest >= 1 && longest <= rows, "mlstm_chunks: bad sizes");
+  EI_REQUIRE(n_seqs > 0 && heads > 0 && rows >= 1 && longest >= 1 && longest <= rows && least > 0, "mlstm_chunks: bad sizes");
   EI_REQUIRE(ei::chunks::sizes_fit(dim, vdim), "mlstm_chunks: heads of 64 or 128 elements");
   EI_REQUIRE(cap > 0.f, "mlstm_chunks: the cap of the gates must be positive");
   EI_REQUIRE(proj && i_bias && f_bias && state && seq_in && seq_out && seq_count && seq_row0 && o_raw &&
@@ -500,7 +502,7 @@ extern "C" int ei_mlstm_chunks(const void* proj, int dtype, const float* i_bias,
                  (reinterpret_cast<uintptr_t>(scratch) & 15) == 0,
              "mlstm_chunks: unaligned rows");
   EI_REQUIRE(heads <= 65535 && n_seqs <= 65535, "mlstm_chunks: too many heads or sequences");
-  EI_REQUIRE(scratch_floats >= (rows / 64 + 1LL * n_seqs) * heads * ei_mlstm_chunk_floats(dim, vdim),
+  EI_REQUIRE(scratch_floats >= ei::chunks::chunk_places(rows, n_seqs, least) * heads * ei_mlstm_chunk_floats(dim, vdim),
              "mlstm_chunks: scratch too small");
   using namespace ei::chunks;
   const Rows at_row{static_cast<size_t>(col_of.width), col_of.q, col_of.k, col_of.v, 1};
@@ -517,7 +519,7 @@ extern "C" int ei_mlstm_chunks(const void* proj, int dtype, const float* i_bias,
   gates.q_scale = q_scale;
   gates.bottom_eps = bottom_eps;
   const State table{state, static_cast<size_t>(state_stride), head_state_floats(dim, vdim)};
-  const Sequences seqs{seq_in, seq_out, seq_count, seq_row0};
+  const Sequences seqs{seq_in, seq_out, seq_count, seq_row0, least};
   if (dtype == EI_F32)
     launch_sized<kMatrix, float>(dim, vdim, static_cast<const float*>(proj), at_row, gates, table, seqs,
                                  scratch, o_raw, n_seqs, heads, longest, stream);

@@ -45,9 +45,18 @@ struct Rows {
   int q, k, v, share;
 };
 
+// The step's sequences, one behind the other in its rows.  Those of fewer than `least` rows (at
+// least 1) are not the chunks' to take: what a sequence's rows go through depends on how many they
+// are, not on what else the step holds.
 struct Sequences {
   const int32_t *in, *out, *count, *row0;
+  int least;
 };
+
+__device__ __forceinline__ int rows_of(const Sequences& seqs, int seq) {
+  const int count = seqs.count[seq];
+  return count >= seqs.least ? count : 0;
+}
 
 // What the gates are made of: per-head constants, and columns `at + head` and `at2 + head` of the
 // rows `raw` (float32 slices or one bfloat16 piece), as the kinds need them.
@@ -74,11 +83,16 @@ __host__ __device__ constexpr size_t chunk_floats(int kind, int dk, int dv) {
   return static_cast<size_t>(dk) * dv + (kind == kMatrix ? dk : 0) + kScalars;
 }
 
-// The scratch of chunk c of sequence s of the step: sequences lie one behind the other in the
-// step's rows, so ceil(count / 64) <= floor((row0 + count) / 64) - floor(row0 / 64) + 1 keeps the
-// sequences' parts apart, and rows / 64 + sequences chunks hold all of them.
-__device__ __forceinline__ size_t chunk_place(int row0, int seq, int chunk) {
-  return static_cast<size_t>(row0 / kTokens) + seq + chunk;
+// The scratch of chunk c of sequence s: ceil(count / 64) <= floor((row0 + count) / 64) -
+// floor(row0 / 64) + 1, and from one sequence that is taken to the next both row0 / least and s grow
+// by one or more, so no two sequences' parts meet, and chunk_places hold all of them.
+__device__ __forceinline__ size_t chunk_place(const Sequences& seqs, int seq, int chunk) {
+  const int row0 = seqs.row0[seq];
+  return static_cast<size_t>(row0 / kTokens) + min(row0 / seqs.least, seq) + chunk;
+}
+
+inline long long chunk_places(int rows, int n_seqs, int least) {
+  return rows / kTokens + (rows / least < n_seqs ? rows / least : n_seqs);
 }
 
 __device__ __forceinline__ float gate_column(const Gates& g, size_t row, int column) {
@@ -147,10 +161,10 @@ add_kernel(const T* __restrict__ rows, Rows at_row, Gates gates, Sequences seqs,
   constexpr int MK = KT / (4 / WV) > 0 ? KT / (4 / WV) : 1, MV = VT / WV;   // tiles a wave
   __shared__ float weight[kTokens];
   const int chunk = blockIdx.x, head = blockIdx.y, seq = blockIdx.z;
-  const int nt = min(kTokens, seqs.count[seq] - chunk * kTokens);
+  const int nt = min(kTokens, rows_of(seqs, seq) - chunk * kTokens);
   if (nt <= 0) return;
   const int first = seqs.row0[seq] + chunk * kTokens;
-  float* mine = scratch + (chunk_place(seqs.row0[seq], seq, chunk) * gridDim.y + head) *
+  float* mine = scratch + (chunk_place(seqs, seq, chunk) * gridDim.y + head) *
                               chunk_floats(KIND, DK, DV);
   float* scalars = mine + chunk_floats(KIND, DK, DV) - kScalars;
   const int lane = threadIdx.x % EI_WAVE, wave = threadIdx.x / EI_WAVE;
@@ -237,12 +251,12 @@ __global__ void __launch_bounds__(kThreads)
 carry_kernel(State state, Sequences seqs, float* __restrict__ scratch) {
   constexpr int kBatch = 8;                              // chunks whose sums are asked for at once
   const int head = blockIdx.y, seq = blockIdx.z;
-  const int count = seqs.count[seq];
+  const int count = rows_of(seqs, seq);
   if (count <= 0) return;
   const int chunks = (count + kTokens - 1) / kTokens;
   constexpr size_t kFloats = chunk_floats(KIND, DK, DV);
   const size_t apart = gridDim.y * kFloats;              // from one chunk to the next
-  float* base = scratch + (chunk_place(seqs.row0[seq], seq, 0) * gridDim.y + head) * kFloats;
+  float* base = scratch + (chunk_place(seqs, seq, 0) * gridDim.y + head) * kFloats;
   const float* in = state.rows + static_cast<size_t>(seqs.in[seq]) * state.row_floats + head * state.head_floats;
   float* out = state.rows + static_cast<size_t>(seqs.out[seq]) * state.row_floats + head * state.head_floats;
   const int e0 = 4 * (blockIdx.x * kThreads + threadIdx.x);
@@ -312,10 +326,10 @@ read_kernel(const T* __restrict__ rows, Rows at_row, Gates gates, Sequences seqs
   __shared__ double log_sums[kTokens];
   __shared__ float takes[kTokens], from_state[kTokens], over[kTokens], rowmax[kTokens];
   const int chunk = blockIdx.x, head = blockIdx.y, seq = blockIdx.z;
-  const int nt = min(kTokens, seqs.count[seq] - chunk * kTokens);
+  const int nt = min(kTokens, rows_of(seqs, seq) - chunk * kTokens);
   if (nt <= 0) return;
   const int first = seqs.row0[seq] + chunk * kTokens;
-  const float* mine = scratch + (chunk_place(seqs.row0[seq], seq, chunk) * gridDim.y + head) *
+  const float* mine = scratch + (chunk_place(seqs, seq, chunk) * gridDim.y + head) *
                                     chunk_floats(KIND, DK, DV);
   const int lane = threadIdx.x % EI_WAVE, wave = threadIdx.x / EI_WAVE;
   const int half = lane / 32, l = lane % 32;

@@ -222,11 +222,11 @@ ssm_scan_kernel(const float* __restrict__ conv, const TI* __restrict__ proj, int
                 const float* __restrict__ d_skip, float* __restrict__ state, size_t state_stride,
                 const int32_t* __restrict__ seq_in, const int32_t* __restrict__ seq_out,
                 const int32_t* __restrict__ seq_count, const int32_t* __restrict__ seq_row0,
-                float* __restrict__ y_raw, int heads, int groups, int P, int Nst, int L) {
+                float* __restrict__ y_raw, int heads, int groups, int P, int Nst, int L, int most) {
   extern __shared__ float lds[];
   const int seq = blockIdx.x, head = blockIdx.y;
   const int count = seq_count[seq];
-  if (count <= 0) return;                       // padding: the whole block leaves together
+  if (count <= 0 || count > most) return;       // padding, or one for the chunks: the whole block leaves
   const int cols = kScanThreads / L;            // columns of S this block walks
   const int npad = L * kScanRows;
   const int tid = threadIdx.x;
@@ -509,7 +509,7 @@ extern "C" int ei_ssm_scan(const float* conv, const void* proj, int in_dtype, in
                            const float* dt_bias, const float* d_skip, float* state,
                            long long state_stride, const int32_t* seq_in, const int32_t* seq_out,
                            const int32_t* seq_count, const int32_t* seq_row0, float* y_raw,
-                           int n_seqs, int heads, int groups, int P, int Nst, int taps,
+                           int n_seqs, int heads, int groups, int P, int Nst, int taps, int most,
                            hipStream_t stream) {
   EI_SSM_SHAPE("ssm_scan");
   EI_REQUIRE(conv && proj && a_log && dt_bias && d_skip && state && seq_in && seq_out && seq_count &&
@@ -541,7 +541,7 @@ extern "C" int ei_ssm_scan(const float* conv, const void* proj, int in_dtype, in
     ssm_scan_kernel<TI, AHEAD><<<grid, kScanThreads, lds, stream>>>(                              \
         conv, static_cast<const TI*>(proj), nsplit, ss, rs, dt_col0, a_log, dt_bias, d_skip,      \
         state, static_cast<size_t>(state_stride), seq_in, seq_out, seq_count, seq_row0, y_raw,    \
-        heads, groups, P, Nst, L);                                                                \
+        heads, groups, P, Nst, L, most);                                                          \
   } while (0)
   if (in_dtype == EI_F32) EI_SSM_SCAN(float);
   else if (in_dtype == EI_BF16) EI_SSM_SCAN(bf16_t);
@@ -552,8 +552,9 @@ extern "C" int ei_ssm_scan(const float* conv, const void* proj, int in_dtype, in
 }
 
 // The recurrence over a prompt's rows in chunks (see recurrence_chunks.h): what `ei_ssm_scan` does
-// for states of 64 or 128 rows and heads of 64 or 128 columns.  scratch: `scratch_floats` floats, at
-// least (N / 64 + n_seqs) * heads chunks; longest: the most rows that a sequence brings.
+// for states of 64 or 128 rows and heads of 64 or 128 columns.  Sequences of fewer than `least` rows are left to the walk.
+// scratch: `scratch_floats` floats, at least chunk_places chunks of all heads; longest: the most
+// rows that a sequence brings.
 extern "C" int ei_ssm_chunk_floats(int P, int Nst) {
   return static_cast<int>(ei::chunks::chunk_floats(ei::chunks::kSelective, Nst, P));
 }
@@ -564,18 +565,19 @@ extern "C" int ei_ssm_chunks(const float* conv, const void* proj, int in_dtype, 
                              long long state_stride, const int32_t* seq_in, const int32_t* seq_out,
                              const int32_t* seq_count, const int32_t* seq_row0, float* y_raw,
                              float* scratch, long long scratch_floats, int N, int n_seqs, int heads,
-                             int groups, int P, int Nst, int taps, int longest, hipStream_t stream) {
+                             int groups, int P, int Nst, int taps, int longest, int least,
+                             hipStream_t stream) {
   EI_SSM_SHAPE("ssm_chunks");
   EI_REQUIRE(conv && proj && a_log && dt_bias && d_skip && state && seq_in && seq_out && seq_count &&
                  seq_row0 && y_raw && scratch && n_seqs > 0 && nsplit >= 1 && N > 0 && longest > 0 &&
-                 longest <= N,
+                 longest <= N && least > 0,
              "ssm_chunks: bad arguments");
   EI_REQUIRE(ei::chunks::sizes_fit(Nst, P), "ssm_chunks: states of 64 or 128 rows and columns");
   EI_REQUIRE(in_dtype == EI_F32 || in_dtype == EI_BF16, "ssm_chunks: unknown dtype");
   EI_REQUIRE((reinterpret_cast<uintptr_t>(conv) & 15) == 0 && (reinterpret_cast<uintptr_t>(scratch) & 15) == 0,
              "ssm_chunks: unaligned rows");
   EI_REQUIRE(heads <= 65535 && n_seqs <= 65535, "ssm_chunks: too many heads or sequences");
-  EI_REQUIRE(scratch_floats >= (N / 64 + 1LL * n_seqs) * heads * ei_ssm_chunk_floats(P, Nst),
+  EI_REQUIRE(scratch_floats >= ei::chunks::chunk_places(N, n_seqs, least) * heads * ei_ssm_chunk_floats(P, Nst),
              "ssm_chunks: scratch too small");
   using namespace ei::chunks;
   // C is the query, B the key, x the value
@@ -591,7 +593,7 @@ extern "C" int ei_ssm_chunks(const float* conv, const void* proj, int in_dtype, 
   gates.stride = static_cast<size_t>(row_stride);
   gates.at = inner + C;
   const State table{state, static_cast<size_t>(state_stride), static_cast<size_t>(P) * Nst};
-  const Sequences seqs{seq_in, seq_out, seq_count, seq_row0};
+  const Sequences seqs{seq_in, seq_out, seq_count, seq_row0, least};
   launch_sized<kSelective, float>(Nst, P, conv, at_row, gates, table, seqs, scratch, y_raw, n_seqs,
                                   heads, longest, stream);
   EI_LAUNCH_CHECK();

@@ -21,6 +21,8 @@ from typing import Dict, Optional, Tuple
 
 import torch
 
+from ..csrc import lib
+
 
 @dataclass(frozen=True)
 class KVRequest:
@@ -275,6 +277,18 @@ class StepContext:
         for which in buffers:
             self.workspace.release(which)
 
-    def longest(self) -> int:
-        """The most tokens that a sequence brings in this step (host value)."""
-        return max((seq.count for seq in self.sequences), default=0)
+    def routes(self, chunk_from: int):
+        """(`longest`, `most`) of a recurrence that goes by chunks from `chunk_from` tokens of a
+        sequence on: `longest` the most tokens that a sequence of this step brings, 0 where none
+        goes by chunks; `most` the most tokens of a sequence that goes token by token, None where
+        none does.  Host values."""
+        if self.decode or not self.sequences:
+            return 0, lib.EVERY
+        span = self.notes.get("tokens a sequence")
+        if span is None:
+            counts = [seq.count for seq in self.sequences]
+            span = self.notes["tokens a sequence"] = min(counts), max(counts)
+        shortest, longest = span
+        if longest < chunk_from:
+            return 0, lib.EVERY
+        return longest, None if shortest >= chunk_from else chunk_from - 1

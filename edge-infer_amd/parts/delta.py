@@ -99,10 +99,12 @@ class GatedDelta:
         # (S is a megabyte a layer and sequence at real sizes: two versions instead of copies)
         return StateRequest(shape=(cls.shape_of(spec).state_floats,), two_versions=True)
 
-    # from so many tokens of one sequence on, by chunks and not token by token, where a head has one
-    # decay (16 heads of 128 x 128: 64 tokens of one sequence 25 us by tokens and 33 by chunks, 8 x
-    # 512 298 and 158, 2,048 671 and 129)
-    CHUNK_FROM = 96
+    # From so many tokens of a sequence on, by chunks and not token by token, where a head has one
+    # decay (16 heads of 128 x 128: 2,048 tokens 671 us by tokens and 129 by chunks, 96 tokens 35 and
+    # 28, beside 32 sequences of one token 71 and 62).  A step of so few rows is the host's, which
+    # pays for two launches more (2k Tirurax, whole steps: 128 tokens 1,208 and 1,235 us, 192 tokens
+    # 1,240 and 1,267, beside 8 decoding sequences 1,347 and 1,236, 256 tokens 1,305 and 1,147).
+    CHUNK_FROM = 192
 
     @classmethod
     def kernel_libraries(cls, spec, dtype):
@@ -216,13 +218,15 @@ class GatedDelta:
         o_raw = ctx.buffer("delta.o_raw", (n, shape.v_width), torch.float32)
         rates = (None, None) if shape.low_rank else (self.decay_log_rate, self.decay_bias)
         how = (rows_in, rows_out, meta.seq_count, meta.seq_row0, o_raw, self.q_scale, self.spec.unit_eps)
-        longest = ctx.longest() if self.chunks_fit and not ctx.decode else 0
-        if longest >= self.CHUNK_FROM:
-            scratch = ctx.buffer("delta.chunks", (lib.delta_chunk_scratch(n, ctx.n_seqs, shape),), torch.float32)
-            lib.delta_chunks(conv, proj, *rates, state, shape, *how, scratch, longest)
+        longest, most = ctx.routes(self.CHUNK_FROM) if self.chunks_fit else (0, lib.EVERY)
+        if longest:
+            least = self.CHUNK_FROM
+            scratch = ctx.buffer("delta.chunks", (lib.delta_chunk_scratch(n, ctx.n_seqs, shape, least),),
+                                 torch.float32)
+            lib.delta_chunks(conv, proj, *rates, state, shape, *how, scratch, longest, least)
             ctx.release(scratch)
-        else:
-            lib.delta_rule(conv, proj, *rates, state, shape, *how)
+        if most:
+            lib.delta_rule(conv, proj, *rates, state, shape, *how, most)
         ctx.release(conv)
         gated = ctx.buffer("delta.gated", (n, shape.v_width))
         lib.delta_out(o_raw, proj, self.out_norm, self.spec.out_norm_eps, shape, meta.row_seq,

@@ -27,10 +27,11 @@ from .linear import Linear
 
 class LinearAttention:
     ACTIVATE_ROWS = 64       # from so many rows of a prompt step on, q, k and v are activated aside
-    # from so many tokens of one sequence on, by chunks and not token by token (16 heads of 128 x
-    # 128: 64 tokens of one sequence 20 us by tokens and 30 by chunks, 8 x 512 398 and 131, 2,048
-    # 785 and 77)
-    CHUNK_FROM = 96
+    # From so many tokens of a sequence on, by chunks and not token by token (16 heads of 128 x 128:
+    # 2,048 tokens 785 us by tokens and 77 by chunks, 96 tokens 27 and 30, 160 tokens 42 and 32; whole
+    # steps of the 2k Gopuzen: 128 tokens 2,120 and 2,151 us, 160 tokens 2,214 and 2,206, beside 8
+    # decoding sequences 2,470 and 2,299).
+    CHUNK_FROM = 160
 
     @property
     def capture_safe(self):
@@ -102,13 +103,15 @@ class LinearAttention:
             activated = True
         sequences = (meta.seq_state_in, meta.seq_state_out, meta.seq_count, meta.seq_row0)
         sizes = (spec.n_heads, spec.key_dim, spec.value_dim)
-        longest = ctx.longest() if activated and self.chunks_fit else 0
-        if longest >= self.CHUNK_FROM:
-            scratch = ctx.buffer("la.chunks", (lib.la_chunk_scratch(n, ctx.n_seqs, *sizes),), torch.float32)
-            lib.la_chunks(rows, self.decay, state, *sequences, o_raw, scratch, *sizes, longest)
+        # (what goes by chunks makes a step of at least ACTIVATE_ROWS rows)
+        longest, most = ctx.routes(self.CHUNK_FROM) if self.chunks_fit else (0, lib.EVERY)
+        if longest:
+            least = self.CHUNK_FROM
+            scratch = ctx.buffer("la.chunks", (lib.la_chunk_scratch(n, ctx.n_seqs, *sizes, least),), torch.float32)
+            lib.la_chunks(rows, self.decay, state, *sequences, o_raw, scratch, *sizes, longest, least)
             ctx.release(scratch)
-        else:
-            lib.la_scan(rows, self.decay, state, *sequences, o_raw, *sizes, activated=activated)
+        if most:
+            lib.la_scan(rows, self.decay, state, *sequences, o_raw, *sizes, activated=activated, most=most)
         if activated:
             ctx.release(rows)
         gated = ctx.buffer("la.gated", (n, spec.v_width))

@@ -40,9 +40,8 @@ class MatrixMemory:
     def capture_rows(self):
         return min(self.proj.capture_rows, self.o.capture_rows)
 
-    # from so many tokens of one sequence on, by chunks and not token by token (16 heads of 128 x
-    # 128 in bfloat16: 64 tokens of one sequence 48 us by tokens and 40 by chunks, 8 x 512 495 and
-    # 154, 2,048 1,300 and 92)
+    # From so many tokens of a sequence on, by chunks and not token by token (16 heads of 128 x 128 in
+    # bfloat16: 64 tokens 46 us by tokens and 40 by chunks, 2,048 tokens 1,300 and 92)
     CHUNK_FROM = 64
 
     @classmethod
@@ -107,14 +106,18 @@ class MatrixMemory:
         sequences = (meta.seq_state_in, meta.seq_state_out, meta.seq_count, meta.seq_row0)
         sizes = (spec.n_heads, spec.key_dim, spec.value_dim)
         how = (spec.gate_cap, self.q_scale, spec.bottom_eps)
-        longest = ctx.longest() if self.chunks_fit and not ctx.decode and proj.dim() == 2 else 0
-        if longest >= self.CHUNK_FROM:
-            scratch = ctx.buffer("mlstm.chunks", (lib.mlstm_chunk_scratch(n, ctx.n_seqs, *sizes),), torch.float32)
+        longest, most = (ctx.routes(self.CHUNK_FROM) if self.chunks_fit and proj.dim() == 2
+                         else (0, lib.EVERY))
+        if longest:
+            least = self.CHUNK_FROM
+            scratch = ctx.buffer("mlstm.chunks", (lib.mlstm_chunk_scratch(n, ctx.n_seqs, *sizes, least),),
+                                 torch.float32)
             lib.mlstm_chunks(proj, self.in_bias, self.forget_bias, state, *sequences, o_raw, scratch,
-                             *sizes, *how, longest)
+                             *sizes, *how, longest, least)
             ctx.release(scratch)
-        else:
-            lib.mlstm_walk(proj, self.in_bias, self.forget_bias, state, *sequences, o_raw, *sizes, *how)
+        if most:
+            lib.mlstm_walk(proj, self.in_bias, self.forget_bias, state, *sequences, o_raw, *sizes, *how,
+                           most=most)
         gated = ctx.buffer("mlstm.gated", (n, spec.v_width))
         lib.mlstm_out(o_raw, proj, self.out_norm, spec.out_norm_eps, meta.row_seq, gated,
                       spec.n_heads, spec.key_dim, spec.value_dim)

@@ -57,9 +57,10 @@ class StateSpace:
             "o_proj.weight": ParamSpec((hidden, spec.inner)),
         }
 
-    # from so many tokens of one sequence on, by chunks and not token by token (16 heads of 128
-    # columns, state 128: 64 tokens of one sequence 30 us by tokens and 35 by chunks, 8 x 512 305
-    # and 143, 2,048 790 and 82)
+    # From so many tokens of a sequence on, by chunks and not token by token (16 heads of 128 columns,
+    # state 128: 64 tokens 29 us by tokens and 34 by chunks, 96 tokens 41 and 35, 2,048 tokens 790 and
+    # 82; whole steps of the 2k Vafepel: 64 tokens 1,149 and 1,178 us, 96 tokens 1,258 and 1,248,
+    # beside 32 decoding sequences 1,584 and 1,545)
     CHUNK_FROM = 96
 
     @classmethod
@@ -115,13 +116,14 @@ class StateSpace:
         y_raw = ctx.buffer("ssm.y_raw", (n, shape.inner), torch.float32)
         constants = (self.a_log, self.dt_bias, self.skip)
         sequences = (rows_in, rows_out, meta.seq_count, meta.seq_row0)
-        longest = ctx.longest() if self.chunks_fit and not ctx.decode else 0
-        if longest >= self.CHUNK_FROM:
-            scratch = ctx.buffer("ssm.chunks", (lib.ssm_chunk_scratch(n, ctx.n_seqs, shape),), torch.float32)
-            lib.ssm_chunks(conv, proj, *constants, state, shape, *sequences, y_raw, scratch, longest)
+        longest, most = ctx.routes(self.CHUNK_FROM) if self.chunks_fit else (0, lib.EVERY)
+        if longest:
+            least = self.CHUNK_FROM
+            scratch = ctx.buffer("ssm.chunks", (lib.ssm_chunk_scratch(n, ctx.n_seqs, shape, least),), torch.float32)
+            lib.ssm_chunks(conv, proj, *constants, state, shape, *sequences, y_raw, scratch, longest, least)
             ctx.release(scratch)
-        else:
-            lib.ssm_scan(conv, proj, *constants, state, shape, *sequences, y_raw)
+        if most:
+            lib.ssm_scan(conv, proj, *constants, state, shape, *sequences, y_raw, most)
         ctx.release(conv)
         gated = ctx.buffer("ssm.gated", (n, shape.inner))
         lib.ssm_out(y_raw, proj, self.out_norm, self.spec.norm_eps, shape, self.spec.norm_parts,

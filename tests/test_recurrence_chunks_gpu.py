@@ -247,3 +247,46 @@ def test_a_prompt_whole_and_in_portions(cfg):
         return torch.cat([out[-2][:1], out[-1]])
     whole, cut = logits(200), logits(40)
     assert ((whole - cut).norm() / cut.norm()).item() <= 1e-5
+
+
+@pytest.mark.parametrize("cfg", designs(), ids=lambda c: c["architecture"])
+def test_a_sequence_beside_others_has_the_bits_it_has_alone(cfg):
+    """Which recurrence a prompt goes through, and the order of its sums, are a matter of its own
+    length: a step of long and short prompts (either side of what goes by chunks) gives every
+    float32 logit the bits that a step of that prompt alone gives it."""
+    import edge_infer_amd as ei
+    from edge_infer_amd.config import resolve_architecture
+    model = ei.random_model(resolve_architecture(cfg).config_class.from_dict(cfg), seed=4, dtype="float32")
+    g = torch.Generator().manual_seed(10)
+    ids = [torch.randint(0, 97, (n,), generator=g).tolist() for n in (5, 200, 192, 191, 160, 159, 96, 95, 64, 63, 2)]
+
+    def logits(prompts):
+        session = ei.Session(model, max_tokens=4096, max_seqs=11)
+        slots = [session.begin() for _ in prompts]
+        first = session.step([(s, p, list(range(len(p)))) for s, p in zip(slots, prompts)])
+        return first.clone().split([len(p) for p in prompts])
+    for beside, prompt in zip(logits(ids), ids):
+        assert torch.equal(beside, logits([prompt])[0]), len(prompt)
+
+
+@pytest.mark.parametrize("dk,dv", [(64, 64), (128, 128)])
+def test_the_delta_rule_sums_alike_in_small_and_large_steps(dk, dv):
+    """A step of 70 sequences takes 32 columns a block, one sequence alone 16."""
+    from edge_infer_amd.csrc import lib
+    H, G, n, count = 4, 2, 70, 70
+    shape = lib.DeltaShape(H, G, dk, dv, 4)
+    g = torch.Generator().manual_seed(3)
+    conv = torch.randn(n * count, shape.conv_width, generator=g).to(DEV)
+    proj = torch.randn(n * count, shape.width, generator=g).to(DEV)
+    a_log, bias = torch.rand(H, generator=g).to(DEV), torch.rand(H, generator=g).to(DEV) - 2.0
+    table = torch.randn(3 * n, shape.state_floats, generator=g).to(DEV)
+
+    def outputs(seqs):
+        rows = count * seqs
+        moved, out = table.clone(), torch.empty(rows, H * dv, device=DEV)
+        scratch = torch.empty(lib.delta_chunk_scratch(rows, seqs, shape), device=DEV)
+        lib.delta_chunks(conv[:rows], proj[:rows], a_log, bias, moved, shape, *metadata([count] * seqs), out,
+                         dk ** -0.5, 1e-6, scratch, count)
+        return out[:count], moved[1]
+    for alone, beside in zip(outputs(1), outputs(n)):
+        assert torch.equal(alone, beside)
