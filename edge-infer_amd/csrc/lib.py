@@ -2100,8 +2100,14 @@ def _chunk_floats(library_name: str, symbol: str, dk: int, dv: int) -> int:
 
 def _chunk_scratch(library_name: str, symbol: str, rows: int, seqs: int, least: int, heads: int,
                    dk: int, dv: int) -> int:
-    each = _chunk_floats(library_name, symbol, dk, dv)
-    return (rows // CHUNK_TOKENS + min(rows // least, seqs)) * heads * each
+    return chunk_scratch(_chunk_floats(library_name, symbol, dk, dv), rows, seqs, least, heads)
+
+
+def chunk_scratch(each: int, rows: int, seqs: int, least: int, heads: int) -> int:
+    """Elements for the chunks that a step may hold, rows // 64 + min(rows // least, seqs) of them,
+    `each` elements a head: no less, and exactly linear in rows and sequences (steps of one class
+    share a plan whose sizes are scaled)."""
+    return heads * (rows * -(-each // CHUNK_TOKENS) + min(rows * -(-each // least), seqs * each))
 
 
 def la_chunk_scratch(rows, seqs, heads, key_dim, value_dim, least=1) -> int:

@@ -98,18 +98,21 @@ def _round_up_coarse(count: int) -> int:
 FEW_ROWS = 256
 
 
-def workspace_class(ctx):
+def workspace_class(ctx, chunk_levels=()):
     """(signature, scale) under which a step's buffers are planned.  Decode steps and steps
     of few rows are planned for their exact shape (the few-rows product slices K differently
     for every row count).  Prompt steps of more rows share a plan with every step of about
     their size: rows rounded up by at most an eighth, sequences and wanted rows to a power of
     two (wanted rows that are all rows follow the rows); the recorded sizes are scaled to the
     largest step of the class, which is safe because every buffer of such a step is at most
-    linear in rows, sequences and wanted rows."""
+    linear in rows, sequences and wanted rows.  `chunk_levels`: the lengths from which the model's
+    recurrences take a sequence by chunks; they ask for a buffer more then, so steps that do and
+    steps that do not are different classes."""
     rows, seqs, want = ctx.n_rows, ctx.n_seqs, ctx.meta.n_want
     bound = ctx.context_bound if ctx.fixed_shape else None
+    route = sum(1 for level in chunk_levels if ctx.routes(level)[0])
     if ctx.decode or rows <= FEW_ROWS:
-        return (rows, seqs, want, ctx.decode, bound), 1.0
+        return (rows, seqs, want, ctx.decode, bound, route), 1.0
     rows_up, seqs_up = _round_up_fine(rows), _round_up_coarse(seqs)
     if want == rows:
         want_up, want_key = rows_up, "all"
@@ -118,7 +121,7 @@ def workspace_class(ctx):
     else:
         want_up = want_key = _round_up_coarse(want)
     scale = max(rows_up / rows, seqs_up / seqs, want_up / max(1, want))
-    return (rows_up, seqs_up, want_key, False, bound), scale
+    return (rows_up, seqs_up, want_key, False, bound, route), scale
 
 
 def members_of(block):
@@ -130,6 +133,14 @@ def members_of(block):
         return tuple(block.members())
     return tuple(part for part in vars(block).values()
                  if hasattr(part, "forward") or hasattr(part, "add_norm"))
+
+
+def parts_below(block):
+    """The parts a block holds and, where these hold parts themselves, those too."""
+    for part in members_of(block):
+        yield part
+        if hasattr(part, "members"):
+            yield from parts_below(part)
 
 
 class DecoderModel:
@@ -234,6 +245,15 @@ class DecoderModel:
             self._planner_list = found
         return found
 
+    def _chunk_levels(self):
+        """The lengths of a sequence from which some part takes it by chunks."""
+        found = getattr(self, "_chunk_level_list", None)
+        if found is None:
+            found = self._chunk_level_list = sorted(
+                {part.CHUNK_FROM for layer in self.layers for part in parts_below(layer)
+                 if getattr(part, "chunks_fit", False)})
+        return found
+
     def plan_step(self, plan) -> None:
         """Let the parts add the metadata sections they plan for themselves (work items of
         their kernels and the like) to the step plan; the engine only carries them."""
@@ -298,7 +318,7 @@ class DecoderModel:
         workspace = ctx.workspace
         ctx.notes.clear()      # what the parts note lives for one pass (a step that is captured
         #                        runs two passes over one context: eagerly, then recorded)
-        workspace.start(*workspace_class(ctx))
+        workspace.start(*workspace_class(ctx, self._chunk_levels()))
         try:
             logits = self._forward(ctx)
         except BaseException:

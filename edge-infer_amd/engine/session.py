@@ -153,9 +153,10 @@ class Session:
 
     def workspace_report(self) -> dict:
         """Bytes of the step workspaces: what is held, and for every planned shape of step
-        (rows, sequences, wanted rows, decode, context bound) the arena it needs, what its
-        values would need without sharing, and what sharing saves (the reference reports
-        the same of its decode plan, runtime/include/qwen3.hpp:60-63)."""
+        (rows, sequences, wanted rows, decode, context bound, how many of the recurrences' lengths
+        for chunks it reaches) the arena it needs, what its values would need without sharing, and
+        what sharing saves (the reference reports the same of its decode plan,
+        runtime/include/qwen3.hpp:60-63)."""
         def plans(workspace):
             return {signature: {"arena_bytes": layout.arena.arena_bytes,
                                 "bytes_without_sharing": layout.arena.bytes_without_sharing(),

@@ -290,3 +290,31 @@ def test_the_delta_rule_sums_alike_in_small_and_large_steps(dk, dv):
         return out[:count], moved[1]
     for alone, beside in zip(outputs(1), outputs(n)):
         assert torch.equal(alone, beside)
+
+
+@pytest.mark.parametrize("cfg", designs(), ids=lambda c: c["architecture"])
+def test_steps_with_and_without_chunks_keep_their_plans(cfg, monkeypatch):
+    """Two shapes of step of 512 rows and 8 sequences, one of whose prompts go by chunks, and steps
+    of a few rows more or less, in turn: each runs from the plan that its class has."""
+    import edge_infer_amd as ei
+    from edge_infer_amd.config import resolve_architecture
+    from edge_infer_amd.parts.base import Workspace
+    model = ei.random_model(resolve_architecture(cfg).config_class.from_dict(cfg), seed=4, dtype="float32")
+    session = ei.Session(model, max_tokens=2048, max_seqs=8)
+
+    def step(counts):
+        slots = [session.begin() for _ in counts]
+        session.step([(s, [7] * n, [n - 1]) for s, n in zip(slots, counts)])
+        for slot in slots:
+            session.end(slot)
+    shapes = [[63] * 8, [400] + [16] * 7, [399] + [14] * 7, [61] * 8]
+    for counts in shapes:
+        step(counts)
+    plans = set(session.workspace_report()["plans"])
+
+    def diverged(self):
+        raise AssertionError("a step left its plan")
+    monkeypatch.setattr(Workspace, "_diverged", diverged)
+    for counts in shapes + shapes:
+        step(counts)
+    assert set(session.workspace_report()["plans"]) == plans and len(plans) == 2

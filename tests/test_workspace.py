@@ -145,3 +145,63 @@ def test_old_plans_are_dropped_and_planned_again_when_needed():
     assert "broken" not in ws._plans
     run_step(ws, "broken")
     assert "broken" in ws._plans
+
+
+class Step:
+    """What `workspace_class` asks of a step's context."""
+    decode, fixed_shape, context_bound = False, False, 0
+
+    def __init__(self, counts, want):
+        from edge_infer_amd.parts.base import StepContext
+        self.n_rows, self.n_seqs = sum(counts), len(counts)
+        self.meta = type("Meta", (), {"n_want": want})
+        self.sequences = [type("Seq", (), {"count": count}) for count in counts]
+        self.notes = {}
+        self.routes = lambda level: StepContext.routes(self, level)
+
+
+def test_steps_that_go_by_chunks_are_a_class_of_their_own():
+    from edge_infer_amd.engine.model import workspace_class
+    one, other = Step([64] * 8, 8), Step([400] + [16] * 7, 8)
+    assert workspace_class(one)[0] == workspace_class(other)[0]        # nothing by chunks in the model
+    assert workspace_class(one, [96])[0] != workspace_class(other, [96])[0]
+    assert workspace_class(one, [96])[0] == workspace_class(Step([95] + [59] * 7, 8), [96])[0]
+    levels = [64, 96, 192]       # where two steps differ, they lie on different sides of a level
+    keys = [workspace_class(Step([n] + [40] * 7, 8), levels)[0][-1] for n in (40, 64, 95, 96, 191, 192, 500)]
+    assert keys == [0, 1, 1, 2, 2, 3, 3]
+    few = [workspace_class(Step([n, 200 - n], 1), [96])[0] for n in (100, 120)]
+    assert few[0] == few[1] != workspace_class(Step([95, 95, 10], 1), [96])[0]
+
+
+def test_a_class_has_room_for_the_chunks_of_its_largest_step():
+    """Every step of a class is served from the plan that any other step of it recorded."""
+    import random
+    from edge_infer_amd.csrc import lib
+    from edge_infer_amd.engine.model import workspace_class
+    rng = random.Random(5)
+    cases = [([319], [320]), ([300, 5, 5, 5], [305, 5, 5, 5]), ([257], [288])]
+    for _ in range(300):
+        seqs = rng.randint(1, 20)
+        make = lambda: [rng.choice([1, 5, 63, 64, 97, 200, 300]) for _ in range(seqs)]  # noqa: E731
+        cases.append((make(), make()))
+    met = 0
+    for first, second in cases:
+        for each, least, heads in ((16388, 96, 1), (36868, 192, 3), (4100, 64, 2)):
+            steps = [Step(first, 0), Step(second, 0)]
+            (key, scale), (other, _) = [workspace_class(step, [least]) for step in steps]
+            longest = [step.routes(least)[0] for step in steps]
+            if key != other or not all(longest) or steps[0].n_rows <= 256:
+                continue
+            met += 1
+            workspace = Workspace("cpu")
+            for step, served in zip(steps, (False, True)):
+                workspace.start(key, scale)
+                pieces = lib.chunk_scratch(each, step.n_rows, step.n_seqs, least, heads)
+                # what the kernels ask for
+                assert pieces >= (step.n_rows // 64 + min(step.n_rows // least, step.n_seqs)) * heads * each
+                workspace.get("rows", (step.n_rows, 8), torch.float32)
+                scratch = workspace.get("chunks", (pieces,), torch.float32)
+                workspace.release(scratch)
+                assert (workspace._layout is not None) == served, (first, second, each)
+                workspace.finish()
+    assert met > 50
