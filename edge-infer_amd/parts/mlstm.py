@@ -41,7 +41,9 @@ class MatrixMemory:
         return min(self.proj.capture_rows, self.o.capture_rows)
 
     # From so many tokens of a sequence on, by chunks and not token by token (16 heads of 128 x 128 in
-    # bfloat16: 64 tokens 46 us by tokens and 40 by chunks, 2,048 tokens 1,300 and 92)
+    # bfloat16: 64 tokens 46 us by tokens and 40 by chunks, 2,048 tokens 1,300 and 92; whole steps of
+    # the 2k Zadenex in bfloat16, slices added up included: 64 tokens 1,511 and 1,264 us, 256 tokens
+    # 4,190 and 1,598, 64 tokens beside 32 decoding sequences 2,572 and 1,501)
     CHUNK_FROM = 64
 
     @classmethod
@@ -106,8 +108,14 @@ class MatrixMemory:
         sequences = (meta.seq_state_in, meta.seq_state_out, meta.seq_count, meta.seq_row0)
         sizes = (spec.n_heads, spec.key_dim, spec.value_dim)
         how = (spec.gate_cap, self.q_scale, spec.bottom_eps)
-        longest, most = (ctx.routes(self.CHUNK_FROM) if self.chunks_fit and proj.dim() == 2
-                         else (0, lib.EVERY))
+        longest, most = ctx.routes(self.CHUNK_FROM) if self.chunks_fit else (0, lib.EVERY)
+        if longest and proj.dim() == 3:
+            # (the chunks' kernels read a row several times: its slices are added up once)
+            slices, proj = proj, proj[0]
+            if len(slices) > 1:
+                proj = ctx.buffer("mlstm.rows", slices.shape[1:], torch.float32)
+                lib.sum_slices(slices, proj)
+                ctx.release(slices)
         if longest:
             least = self.CHUNK_FROM
             scratch = ctx.buffer("mlstm.chunks", (lib.mlstm_chunk_scratch(n, ctx.n_seqs, *sizes, least),),

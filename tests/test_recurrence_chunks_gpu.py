@@ -318,3 +318,37 @@ def test_steps_with_and_without_chunks_keep_their_plans(cfg, monkeypatch):
     for counts in shapes + shapes:
         step(counts)
     assert set(session.workspace_report()["plans"]) == plans and len(plans) == 2
+
+
+@pytest.mark.parametrize("width", [64, 1024])
+def test_the_matrix_memory_goes_by_chunks_in_steps_of_few_rows(width, monkeypatch):
+    """In bfloat16 steps of at most 256 rows have float32 slices of the input product (one at a width
+    of 64, several at 1,024): a prompt of 100 tokens beside one of 20 goes by chunks all the same.
+    The logits differ from those token by token by what a bfloat16 rounding of the mixer's rows
+    that falls the other way moves them (2^-8 of a few of them)."""
+    import edge_infer_amd as ei
+    from edge_infer_amd.config import resolve_architecture
+    from edge_infer_amd.csrc import lib
+    from edge_infer_amd.parts.mlstm import MatrixMemory
+    cfg = next(c for c in designs() if c["architecture"] == "Zadenex") | {"width": width}
+    model = ei.random_model(resolve_architecture(cfg).config_class.from_dict(cfg), seed=4, dtype="bfloat16")
+    g = torch.Generator().manual_seed(9)
+    ids = [torch.randint(0, 97, (n,), generator=g).tolist() for n in (100, 20)]
+    calls = []
+    for name in ("mlstm_chunks", "mlstm_walk", "sum_slices"):
+        def counted(*args, _call=getattr(lib, name), _name=name, **kw):
+            calls.append(_name)
+            return _call(*args, **kw)
+        monkeypatch.setattr(lib, name, counted)
+
+    def logits(prompts):
+        calls.clear()
+        session = ei.Session(model, max_tokens=1024, max_seqs=2)
+        return session.step([(session.begin(), p, list(range(len(p)))) for p in prompts]).clone()
+    got = logits(ids)
+    assert calls.count("mlstm_chunks") == calls.count("mlstm_walk") == 1
+    assert (calls.count("sum_slices") > 0) == (width > 64)
+    monkeypatch.setattr(MatrixMemory, "CHUNK_FROM", 10 ** 6)
+    walked = logits(ids)
+    assert calls.count("mlstm_chunks") == 0
+    assert ((got - walked).norm() / walked.norm()).item() <= 2.0 ** -8
