@@ -19,6 +19,10 @@
 // 4 g + r: a sum can be multiplied on without leaving its registers, the A operand's lane then
 // bringing four neighbouring k values.
 //
+// Causality holds for values that are not finite too: where the system's right sides or U hold such a
+// one, the products with matrices that are zero above the diagonal are taken term by term (zero
+// times infinity is not zero).
+//
 // What bounds it: the walk is a chain over chunks of 112 products (of 32 cycles) a wave, two barriers
 // and 116 KB of operands a block, 2.9 us a chunk of one sequence.  2,048 tokens of 16 heads of 128 x
 // 128: 671 us token by token, 129 by chunks (solve 34, walk 93); 8 x 512: 298 and 158.
@@ -28,6 +32,7 @@
 namespace ei {
 namespace delta_chunks {
 
+using chunks::any_not_finite;
 using chunks::chunk_place;
 using chunks::rows_of;
 using chunks::f32x16;
@@ -276,6 +281,23 @@ solve_kernel(Rows in, Gates gates, Sequences seqs, float* __restrict__ scratch) 
 #pragma unroll
       for (int c = 0; c < kMine; ++c)
         solved[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(inv[r], x[b][c][r], solved[c], 0, 0, 0);
+    float met = 0.f;
+#pragma unroll
+    for (int c = 0; c < kMine; ++c) met += solved[c][0] * 0.f;
+    if (any_not_finite(met)) {
+#pragma unroll
+      for (int c = 0; c < kMine; ++c) {
+        f32x4 sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {
+          const float xm = __shfl(x[b][c][m % 4], m / 4 * 16 + i16, EI_WAVE);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (m <= 4 * g + r) sum[r] += t_lds[(16 * b + 4 * g + r) * TS + m] * xm;
+        }
+        solved[c] = sum;
+      }
+    }
 #pragma unroll
     for (int c = 0; c < kMine; ++c) {
       x[b][c] = solved[c];
@@ -292,9 +314,10 @@ solve_kernel(Rows in, Gates gates, Sequences seqs, float* __restrict__ scratch) 
 }
 
 // A block a (head, sequence, 16 NC columns of S), wave w having rows 16 (DK / 64) w on of S and tokens
-// 16 w .. 16 w + 15 of a chunk.  A chunk's operands are asked for a chunk ahead.
+// 16 w .. 16 w + 15 of a chunk.  A chunk's operands are asked for a chunk ahead.  (Keys of 64 and 32
+// columns: bound to the registers that let a SIMD hold two waves.)
 template <int DK, int DV, int NC>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, DK == 64 && NC == 2 ? 2 : 1)
 walk_kernel(State state, Sequences seqs, const float* __restrict__ scratch, float* __restrict__ out) {
   typedef Scratch<DK, DV> At;
   constexpr int KT = DK / 64;                    // tiles of 16 rows of S a wave
@@ -402,6 +425,25 @@ walk_kernel(State state, Sequences seqs, const float* __restrict__ scratch, floa
             add[n][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(in_chunk.k[i][b][r], ub[b][n][r], add[n][i], 0, 0, 0);
           o[n][r % kSums] = __builtin_amdgcn_mfma_f32_16x16x4f32(in_chunk.p[b][r], ub[b][n][r], o[n][r % kSums], 0, 0, 0);
         }
+    }
+    float met = 0.f;
+#pragma unroll
+    for (int n = 0; n < NC; ++n) met += o[n][0][0] * 0.f + o[n][1][0] * 0.f;
+    if (any_not_finite(met)) {
+      const float* weights = base + c * apart + At::p;
+#pragma unroll
+      for (int n = 0; n < NC; ++n) {
+        o[n][0] = o[n][1] = zero;
+#pragma unroll 1
+        for (int s = 0; s < 16 * (wave + 1); ++s) {
+          const float u = u_lds[(16 * n + i16) * US + s];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int t = 16 * wave + 4 * g + r;
+            if (s <= t) o[n][0][r] += weights[operand_at(t, s, kTokens)] * u;
+          }
+        }
+      }
     }
 #pragma unroll
     for (int n = 0; n < NC; ++n)

@@ -20,8 +20,12 @@
 // 2,048 tokens of 16 heads of 128 x 128 at the instruction's rate, and the chunks' states, written
 // once, carried and read, are 130 MB.
 //
-// Rows of a chunk beyond its sequence's end are its last row again, with weight zero.  A row that
-// is not finite makes its whole chunk's outputs not finite (the walk only those from it on).
+// Rows of a chunk beyond its sequence's end are its last row again, with weight zero.
+//
+// Causality holds for values that are not finite too: the products with the weights below the
+// diagonal multiply zeros above it, and zero times infinity is none, so a tile of values that holds
+// such a one takes its sum term by term, without the places above the diagonal.  (Every row of a
+// product meets every value of its column, so one row of the result tells.)
 #pragma once
 #include "common.h"
 
@@ -145,6 +149,9 @@ __device__ __forceinline__ void lane_gates(const Gates& g, int head, size_t row,
     log_sum = each;
   }
 }
+
+// Whether some lane of the wave has a value that is not finite.
+__device__ __forceinline__ bool any_not_finite(float value) { return __any(value * 0.f != 0.f); }
 
 __device__ __forceinline__ float at(const float* p) { return *p; }
 __device__ __forceinline__ float at(const bf16_t* p) { return bf16_to_f32(*p); }
@@ -492,7 +499,21 @@ read_kernel(const T* __restrict__ rows, Rows at_row, Gates gates, Sequences seqs
         }
       }
     }
-    acc += (sums[0] + sums[1]) + (sums[2] + sums[3]);
+    f32x16 own = (sums[0] + sums[1]) + (sums[2] + sums[3]);
+    if (any_not_finite(own[0])) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) own[e] = 0.f;
+#pragma unroll 1
+      for (int s = 0; s < min(nt, 32 * (rt + 1)); ++s) {
+        const float v = at(v_at + static_cast<size_t>(first + s) * at_row.stride);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int t = rt * 32 + e % 4 + 8 * (e / 4) + 4 * half;
+          if (s <= t) own[e] += p_lds[t * PS + s] * v;
+        }
+      }
+    }
+    acc += own;
     const size_t width = static_cast<size_t>(gridDim.y) * DV;
     const float skip = KIND == kSelective ? gates.c2[head] : 0.f;
 #pragma unroll
