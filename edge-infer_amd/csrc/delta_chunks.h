@@ -121,7 +121,7 @@ solve_kernel(Rows in, Gates gates, Sequences seqs, float* __restrict__ scratch) 
         beta = 1.0f / (1.0f + expf(-chunks::gate_column(gates, row, gates.at + head)));
         const float z = chunks::gate_column(gates, row, gates.at2 + head) + gates.c1[head];
         const float soft = z > 30.f ? z : log1pf(expf(z));
-        each = -static_cast<double>(expf(gates.c0[head])) * soft;
+        each = chunks::bounded_log(-static_cast<double>(expf(gates.c0[head])) * soft);
       }
 #pragma unroll
       for (int step = 1; step < kTokens; step *= 2) {

@@ -108,6 +108,12 @@ __device__ __forceinline__ float gate_column(const Gates& g, size_t row, int col
   return v;
 }
 
+// The logarithm of a decay, so low a one that one step of it leaves nothing of a float32 (the least
+// is e^-103.98) as e^-128: a sum of logarithms then stays below 2^13, where float64 has 13 digits
+// behind the point, however low they are and even if they are minus infinity (the difference of two of
+// those would be no number).
+__device__ __forceinline__ double bounded_log(double each) { return each < -128.0 ? -128.0 : each; }
+
 // A chunk's gates, lane t having token t: `log_sum` the sum of the log decays up to t (float64),
 // `take` the input weight b_t (kMatrix: its logarithm).  Tokens beyond the chunk's end do not
 // decay and bring nothing.
@@ -116,9 +122,7 @@ __device__ __forceinline__ void lane_gates(const Gates& g, int head, size_t row,
                                            double& log_sum, float& take) {
   if constexpr (KIND == kFixed) {
     const float d = g.c0[head];
-    // (a decay of zero: a logarithm so low that every power but the zeroth vanishes; a power of two,
-    // so that its multiples are exact and differences of equal ones are zero)
-    const double each = d > 0.f ? log(static_cast<double>(d)) : -0x1p997;
+    const double each = bounded_log(log(static_cast<double>(d)));
     log_sum = each * (min(t, nt - 1) + 1);
     take = t < nt ? 1.f : 0.f;
   } else {
@@ -128,7 +132,7 @@ __device__ __forceinline__ void lane_gates(const Gates& g, int head, size_t row,
       if (t < nt) {
         const float z = gate_column(g, row, g.at + head) + g.c1[head];
         const float dt = z > 20.f ? z : log1pf(expf(z));
-        each = -static_cast<double>(expf(g.c0[head])) * dt;
+        each = bounded_log(-static_cast<double>(expf(g.c0[head])) * dt);
         take = dt;
       }
     } else {

@@ -356,11 +356,12 @@ def test_the_matrix_memory_goes_by_chunks_in_steps_of_few_rows(width, monkeypatc
 
 def both_ways(kind, counts, d, poison):
     """(by chunks, token by token): the outputs and last states of one recurrence on inputs that
-    `poison` has changed.  `poison(rows)` gets {"q", "k", "v", "gate"} as views [rows, columns]."""
+    `poison` has changed.  `poison(rows)` gets {"q", "k", "v", "gate"} as views [rows, columns] and, a value a head,
+    {"rates", "bias"}."""
     from edge_infer_amd.csrc import lib
     H, rows, longest = 2, sum(counts), max(counts)
     g = torch.Generator().manual_seed(21)
-    per_head = [torch.randn(H, generator=g).to(DEV) for _ in range(3)]
+    per_head = [torch.randn(H, generator=g) for _ in range(3)]
     meta, results = metadata(counts), []
     if kind == "fixed":
         act = torch.randn(rows, 3 * H * d, generator=g)
@@ -384,8 +385,8 @@ def both_ways(kind, counts, d, poison):
         views["gate"] = proj[:, shape.beta_col:shape.beta_col + 2 * H]
         inputs, floats = [conv, proj], shape.state_floats
     table = torch.randn(3 * len(counts), floats, generator=g)
-    poison(views)
-    inputs = [x.to(DEV) for x in inputs]
+    poison(views | {"rates": per_head[0], "bias": per_head[1]})
+    inputs, per_head = [x.to(DEV) for x in inputs], [x.to(DEV) for x in per_head]
     for chunks in (True, False):
         moved, out = table.to(DEV), torch.zeros(rows, H * d, device=DEV)
         if kind == "fixed":
@@ -441,3 +442,19 @@ def test_what_is_not_finite_spoils_nothing_before_it(kind, d, what, value):
         assert not finite[130 + row].all() or (kind, what) in (("matrix", "gate"), ("delta", "gate"),
                                                                ("selective", "gate"))
         check_ways(results, 1e-4)
+
+
+@pytest.mark.parametrize("kind", ["selective", "delta"])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("rate", [28.0, 100.0])
+def test_rates_of_any_size(kind, d, rate):
+    """Rates of e^28, where a step decays by e^-7e12 or, 40 below, by e^-6e-6 of what there is, and of
+    e^100, which float32 does not hold: a decay of nothing, as token by token.  (Float32 sums of up to
+    some 200 products in two orders: 1e-5 of the row's largest.)"""
+    def poison(views):
+        views["rates"][0], views["bias"][:] = rate, 0.0
+        gate = views["gate"][:, -2:]                     # the decays' logits, a column a head
+        gate[:, 0] = torch.where(torch.arange(len(gate)) % 7 == 3, 5.0, -40.0)
+    results = both_ways(kind, [130, 130, 70], d, poison)
+    assert all(part.isfinite().all() for part in results[1])
+    check_ways(results, 1e-5)
