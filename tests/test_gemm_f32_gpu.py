@@ -45,3 +45,23 @@ def test_narrow_strips_of_few_rows(N, K):
         assert bool(((out[:rows].double() - exact[:rows]).abs() <= bound[:rows]).all()), rows
         assert torch.equal(out[:rows], wide[:rows]), rows
         assert bool((out[rows] == 7.0).all()), rows
+
+
+@pytest.mark.parametrize("N,K", [(17, 20), (100, 1028), (4099, 68), (1000, 3072)])
+def test_where_the_operands_lie_does_not_change_the_bits(N, K):
+    """Rows that begin at any float give the bits of rows that begin at a multiple of four."""
+    from edge_infer_amd.csrc import lib
+    g = torch.Generator().manual_seed(N + K)
+    a, w = torch.randn(130, K, generator=g).to("cuda"), torch.randn(N, K, generator=g).to("cuda")
+
+    def moved(x, by):
+        room = torch.empty(x.numel() + 4, device="cuda")
+        view = room[by:by + x.numel()].view(x.shape)
+        return view.copy_(x)
+    for rows in (130, 65, 40, 17, 8, 1):
+        want = torch.empty(rows, N, device="cuda")
+        lib.gemm_f32(a[:rows], w, want)
+        for by_a, by_w in ((1, 0), (0, 1), (2, 3)):
+            out = torch.empty(rows, N, device="cuda")
+            lib.gemm_f32(moved(a[:rows], by_a), moved(w, by_w), out)
+            assert torch.equal(out, want), (rows, by_a, by_w)
