@@ -5,7 +5,7 @@
 //
 // The order of an output's sum depends on K alone, so a row's result does not depend on which other
 // rows are in the batch, on where the operands lie, nor on which of the kernels below computed it:
-// matrix-core kernels for K in fours (few rows, many rows), and one of plain multiply-adds, k in
+// matrix-core kernels for K in fours (few rows, many rows, very many outputs), and one of plain multiply-adds, k in
 // ascending order, for every other size.
 #include "common.h"
 
@@ -72,8 +72,8 @@ gemm_f32_kernel(const float* __restrict__ A, const float* __restrict__ W, float*
 //
 // The sum of an output is cut into kSegs pieces of K, each a chain of products from zero, added as
 // a tree, ((c0 + c1) + (c2 + c3)) + ((c4 + c5) + (c6 + c7)).  The pieces depend on K alone and
-// both kernels below add them the same way, so a row gives the same bits in either kernel,
-// whatever other rows there are; the waves of a block take the pieces side by side.
+// the kernels below add them the same way, so a row gives the same bits in each of them, whatever
+// other rows there are.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 // four neighbouring floats that begin anywhere: one load all the same (global loads of 16 bytes want
 // 4-byte alignment), slower only by the cache lines it touches
@@ -135,9 +135,11 @@ __device__ __forceinline__ void chain(const float* const (&a)[RT], const float* 
 
 // Many rows: a block of four waves makes 16 RT x 16 CT outputs, every wave all of them for two
 // neighbouring pieces of K, the first of which waits in LDS for the second.  No operand goes
-// through LDS: a wave's step reads 1 KB a tile row or column for 4 RT CT products of 32 cycles, 4
-// bytes a cycle and SIMD at 4 x 4 tiles.  Two blocks fit a compute unit, so one's first loads and
-// last sums lie under the other's products.
+// through LDS: a wave's step reads 1 KB a tile row or column for 4 RT CT products of 32 cycles.  What
+// bounds it are those loads, whose neighbouring lanes are different rows: 16 bytes a cycle and unit,
+// as long as the products of the four waves take.  4 x 4 tiles take 292 registers, a block a unit;
+// bound to 256, two blocks fit, but read over each other's cache lines (2,048 rows, 4,096 x 4,096: 665 us
+// against 770; 451 rows, 6,144 x 1,024: 76 against 99).
 template <int RT, int CT>
 __global__ void __launch_bounds__(256)
 gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
@@ -146,8 +148,8 @@ gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, f
   const int lane = threadIdx.x % EI_WAVE, wave = threadIdx.x / EI_WAVE;
   const int i16 = lane % 16, g = lane / 16;
   // Blocks go to the eight dies in turn.  Of few row tiles, those that share a column tile follow
-  // each other on one die, whose L2 then serves W to all but the first (100 x 151,936 x 1,024:
-  // 564 -> 524 us); of many, the column tiles come first, which keeps a die's share of both
+  // each other on one die, whose L2 then serves W to all but the first (192 x 16,000 x 1,024:
+  // 80.8 -> 77.0 us); of many, the column tiles come first, which keeps a die's share of both
   // operands small.
   const int row_tiles = (M + 16 * RT - 1) / (16 * RT);
   int row_tile, col_tile;
@@ -214,6 +216,134 @@ gemm_f32_tile_kernel(const float* __restrict__ A, const float* __restrict__ W, f
 #pragma unroll
         for (int e = 0; e < 4; ++e)
           if (n + e < N) dst[e] = sum[i][j][e];
+      }
+    }
+  }
+}
+
+// Very many outputs: a block of eight waves makes 128 x 128 of them, a wave 64 x 32, and the operands
+// come through LDS, 32 values of K at a time, so a row is read from the caches once for 128 outputs and
+// not once for 64, 128 bytes at a time.  A wave goes through all of K; what the pieces of K leave is
+// added up as the tree wants it as soon as two neighbours are there (`fold`), so three sums wait at
+// most and two waves fit a SIMD (224 registers).  2,048 rows, 151,936 outputs, K 1,024: 5.58 ms, 114
+// TFLOP/s (147 the instruction's own rate); the kernel above 8.58, plain multiply-adds from LDS 7.2.
+constexpr int kTile = 128, kStage = 2 * kStep, kRowFloats = kStage + 4;   // (LDS rows: no bank twice)
+constexpr int kTileThreads = 512;
+
+__global__ void __launch_bounds__(kTileThreads, 2)
+gemm_f32_lds_kernel(const float* __restrict__ A, const float* __restrict__ W, float* __restrict__ C,
+                    int M, int N, int K, long long lda, long long ldw, long long ldc, int row_tiles,
+                    int col_tiles) {
+  constexpr int RT = 4, CT = 2;                          // tiles of 16 x 16 a wave
+  constexpr int kLoads = kTile * kStage / 4 / kTileThreads;
+  __shared__ __attribute__((aligned(16))) float a_lds[2][kTile * kRowFloats];
+  __shared__ __attribute__((aligned(16))) float w_lds[2][kTile * kRowFloats];
+  // blocks go to the eight dies in turn: those of a die share a column tile, row tile by row tile
+  const int die = blockIdx.x % 8, there = blockIdx.x / 8;
+  const int row_tile = there % row_tiles, col_tile = there / row_tiles * 8 + die;
+  if (col_tile >= col_tiles) return;
+  const int m0 = row_tile * kTile, n0 = col_tile * kTile;
+  const int lane = threadIdx.x % EI_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / EI_WAVE);
+  const int i16 = lane % 16, g = lane / 16;
+  const int wm = wave / 4 * 64, wn = wave % 4 * 32;      // the wave's part of the block's tile
+  const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
+  // thread -> piece f = t + 512 u of a stage: row f / 8, floats 4 (f % 8) .. + 3
+  const int piece = threadIdx.x % 8 * 4;
+  const float* a_row[kLoads];
+  const float* w_row[kLoads];
+  int at_lds[kLoads];
+#pragma unroll
+  for (int u = 0; u < kLoads; ++u) {
+    const int row = threadIdx.x / 8 + u * (kTileThreads / 8);
+    a_row[u] = A + static_cast<size_t>(min(m0 + row, M - 1)) * lda + piece;
+    w_row[u] = W + static_cast<size_t>(min(n0 + row, N - 1)) * ldw + piece;
+    at_lds[u] = row * kRowFloats + piece;
+  }
+  f32x4 a_next[kLoads], w_next[kLoads];
+  auto fetch = [&](int k0) __attribute__((always_inline)) {
+    const bool live = k0 + piece < K;
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      a_next[u] = live ? *reinterpret_cast<const f32x4_any*>(a_row[u] + k0) : zero;
+      w_next[u] = live ? *reinterpret_cast<const f32x4_any*>(w_row[u] + k0) : zero;
+    }
+  };
+  f32x4 acc[RT][CT], one[RT][CT], two[RT][CT], four[RT][CT];   // sums of that many pieces of K
+  auto each = [&](auto&& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int j = 0; j < CT; ++j) f(i, j);
+  };
+  each([&](int i, int j) { acc[i][j] = one[i][j] = two[i][j] = four[i][j] = zero; });
+  // piece `seg` is there: it, and what it completes, joins its neighbour
+  auto fold = [&](int seg) __attribute__((always_inline)) {
+    if (seg % 2 == 0) {
+      each([&](int i, int j) { one[i][j] = acc[i][j]; });
+    } else {
+      each([&](int i, int j) { acc[i][j] = one[i][j] + acc[i][j]; });
+      if (seg % 4 == 1) {
+        each([&](int i, int j) { two[i][j] = acc[i][j]; });
+      } else {
+        each([&](int i, int j) { acc[i][j] = two[i][j] + acc[i][j]; });
+        if (seg % 8 == 3) each([&](int i, int j) { four[i][j] = acc[i][j]; });
+        else each([&](int i, int j) { four[i][j] = four[i][j] + acc[i][j]; });
+      }
+    }
+    each([&](int i, int j) { acc[i][j] = zero; });
+  };
+  const int steps = (K + kStep - 1) / kStep, per = steps_a_segment(K), stages = (steps + 1) / 2;
+  fetch(0);
+  int seg = 0, left = per;                               // the piece of K, and the steps left of it
+  for (int stage = 0; stage < stages; ++stage) {
+    float* a_now = a_lds[stage % 2];
+    float* w_now = w_lds[stage % 2];
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      *reinterpret_cast<f32x4*>(a_now + at_lds[u]) = a_next[u];
+      *reinterpret_cast<f32x4*>(w_now + at_lds[u]) = w_next[u];
+    }
+    // (the other half is read no more: every wave has passed the last barrier behind its reads)
+    __syncthreads();
+    if (stage + 1 < stages) fetch((stage + 1) * kStage);
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      if (2 * stage + half < steps) {
+        f32x4 ad[RT], wd[CT];
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+          ad[i] = *reinterpret_cast<const f32x4*>(a_now + (wm + 16 * i + i16) * kRowFloats + kStep * half + 4 * g);
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+          wd[j] = *reinterpret_cast<const f32x4*>(w_now + (wn + 16 * j + i16) * kRowFloats + kStep * half + 4 * g);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          each([&](int i, int j) {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wd[j][s], ad[i][s], acc[i][j], 0, 0, 0);
+          });
+        if (--left == 0) {
+          fold(seg++);
+          left = per;
+        }
+      }
+    }
+  }
+  for (; seg < kSegs; ++seg) fold(seg);                  // (pieces cut short, and those without a step)
+  const bool quads = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    const int m = m0 + wm + 16 * i + i16;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      const int n = n0 + wn + 16 * j + 4 * g;
+      float* dst = C + static_cast<size_t>(m) * ldc + n;
+      if (quads && n + 4 <= N) {
+        *reinterpret_cast<f32x4*>(dst) = four[i][j];
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < N) dst[e] = four[i][j][e];
       }
     }
   }
@@ -358,7 +488,6 @@ extern "C" int ei_gemm_f32(const float* A, const float* W, float* C, int M, int 
     EI_LAUNCH_CHECK();
   }
   if (fours) {
-    // the largest tile that leaves no compute unit without a block
     const long long units = ei_compute_units();
     auto blocks_of = [&](int rt, int ct) {
       return ((M + 16LL * rt - 1) / (16 * rt)) * ((N + 16LL * ct - 1) / (16 * ct));
@@ -367,8 +496,18 @@ extern "C" int ei_gemm_f32(const float* A, const float* W, float* C, int M, int 
       const long long rows = (M + 16LL * rt - 1) / (16 * rt), cols = (N + 16LL * ct - 1) / (16 * ct);
       return rows * (rows <= kFewRowTiles ? (cols + 7) / 8 * 8 : cols);
     };
-    EI_REQUIRE(grid_of(2, 2) <= 0x7fffffff || blocks_of(4, 4) <= 0x7ffffff0,
-               "gemm_f32: too many outputs for one launch");
+    // From a block of 128 x 128 for every unit on, those (1,024 rows, 4,096 outputs, K 1,024: 99 -> 78 us,
+    // 512 rows, 6,144 outputs, three quarters of the units: 76 both; 2,048 rows over a vocabulary of
+    // 151,936: 8,575 -> 5,581, 100 rows 522 -> 380).
+    const long long big_rows = (M + kTile - 1LL) / kTile, big_cols = (N + kTile - 1LL) / kTile;
+    const long long big = big_rows * ((big_cols + 7) / 8 * 8);
+    if (big_rows * big_cols >= units) {
+      EI_REQUIRE(big <= 0x7fffffff, "gemm_f32: too many outputs for one launch");
+      gemm_f32_lds_kernel<<<static_cast<unsigned>(big), kTileThreads, 0, stream>>>(
+          A, W, C, M, N, K, lda, ldw, ldc, static_cast<int>(big_rows), static_cast<int>(big_cols));
+      EI_LAUNCH_CHECK();
+    }
+    // else the largest tile that leaves no compute unit without a block
 #define EI_TILE(RT, CT)                                                                     \
   gemm_f32_tile_kernel<RT, CT><<<static_cast<unsigned>(grid_of(RT, CT)), 256, 0, stream>>>( \
       A, W, C, M, N, K, lda, ldw, ldc, (N + 16 * CT - 1) / (16 * CT))

@@ -6,9 +6,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("N,K", [(1, 4), (17, 20), (64, 128), (100, 1028), (130, 2052), (4099, 68),
-                                 (65600, 36)])
+                                 (65600, 36), (16500, 1028), (16411, 2052), (33000, 4)])
 def test_products_of_every_number_of_rows_within_the_bound_and_the_same_bits(N, K):
-    """Rows 1 .. 64 take the kernel of few rows, more the tiles of 32 x 32, 32 x 64 and 64 x 64.
+    """Rows 1 .. 64 take the kernel of few rows, more the tiles of 32 x 32, 32 x 64 and 64 x 64 or,
+    from 256 tiles of 128 x 128 on, those.
     A sum of K float32 products in any order is within K u sum |a w| of the exact one (u = 2^-24,
     and one more u for a product's own rounding); a row has the same bits in every kernel."""
     from edge_infer_amd.csrc import lib
