@@ -25,7 +25,7 @@
 //
 // What bounds it: the walk is a chain over chunks of 112 products (of 32 cycles) a wave, two barriers
 // and 116 KB of operands a block, 2.9 us a chunk of one sequence.  2,048 tokens of 16 heads of 128 x
-// 128: 671 us token by token, 129 by chunks (solve 34, walk 93); 8 x 512: 298 and 158.
+// 128: 671 us token by token, 128 by chunks (solve 34, walk 93); 8 x 512: 298 and 151.
 #pragma once
 #include "recurrence_chunks.h"
 
@@ -488,13 +488,19 @@ inline int chunk_floats(int dk, int dv) { return kTokens * (3 * dk + kTokens + d
 
 template <int DK, int DV>
 inline void launch(const Rows& in, const Gates& gates, const State& state, const Sequences& seqs,
-                   float* scratch, float* out, int n_seqs, int heads, int longest, hipStream_t stream) {
+                   float* scratch, float* out, int rows, int n_seqs, int heads, int longest,
+                   hipStream_t stream) {
   static_assert(Scratch<DK, DV>::floats == kTokens * (3 * DK + kTokens + DV) + 4, "what the host allots");
   solve_kernel<DK, DV><<<dim3(heads, (longest + kTokens - 1) / kTokens, n_seqs), kSolvers, 0, stream>>>(
       in, gates, seqs, scratch);
-  // 16 columns a block while that makes at most two blocks a compute unit: the shortest chain; else
-  // 32, which read every operand half as often (8 x 512 tokens, 1,024 blocks: 115 -> 90 us)
-  if (static_cast<long long>(heads) * n_seqs * (DV / 16) <= 2LL * ei_compute_units())
+  // 16 columns a block, the shortest chain, while that makes at most a block for every compute unit: keys
+  // of 128 take the registers of one (16 heads of 128 x 128, 2 sequences of 1,024 tokens, 256 blocks: 85 us
+  // against 110 by 32 columns; 3 sequences 150 against 128, 4 sequences 163 against 142), and keys of 64,
+  // of which two fit, gain no more by the second (384 blocks: 88 us either way, 512: 96); 32 columns
+  // read every operand half as often.  Sequences count by their share of the longest one, whose chain the
+  // walk lasts as long as: those of a token are not the chunks' anyway
+  const long long chains = min(n_seqs, (rows + longest - 1) / longest);
+  if (heads * chains * (DV / 16) <= ei_compute_units())
     walk_kernel<DK, DV, 1><<<dim3(heads, n_seqs, DV / 16), kThreads, 0, stream>>>(state, seqs, scratch, out);
   else
     walk_kernel<DK, DV, 2><<<dim3(heads, n_seqs, DV / 32), kThreads, 0, stream>>>(state, seqs, scratch, out);

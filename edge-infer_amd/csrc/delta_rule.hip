@@ -1062,7 +1062,7 @@ extern "C" int ei_delta_chunks(const float* conv, int OW, const void* proj, int 
   gates.at2 = decay_col;
   const ei::chunks::State table{state, static_cast<size_t>(state_stride), static_cast<size_t>(D) * DV};
   const ei::chunks::Sequences seqs{seq_in, seq_out, seq_count, seq_row0, least};
-#define EI_DC(DK_, DV_) dc::launch<DK_, DV_>(in, gates, table, seqs, scratch, o_raw, n_seqs, H, longest, stream)
+#define EI_DC(DK_, DV_) dc::launch<DK_, DV_>(in, gates, table, seqs, scratch, o_raw, rows, n_seqs, H, longest, stream)
   if (D == 128 && DV == 128) EI_DC(128, 128);
   else if (D == 128) EI_DC(128, 64);
   else if (DV == 128) EI_DC(64, 128);
