@@ -2473,6 +2473,7 @@ def has_skinny_gemm() -> bool:
 _SKINNY_MAX_SPLITS = int(os.environ.get("EDGE_INFER_SKINNY_MAX_SPLITS", "0"))   # 0: no cap
 
 
+@functools.lru_cache(maxsize=8192)      # (a prompt's host time: 6 us a call, two or three a layer)
 def skinny_gemm_splits(rows: int, n: int, k: int) -> int:
     """K slices the weight-streaming product uses for [rows, k] x [n, k]^T."""
     return library("gemm_bf16").ei_skinny_gemm_splits(rows, n, k, _SKINNY_MAX_SPLITS)
