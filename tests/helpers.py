@@ -116,3 +116,51 @@ def assert_close_long(dtype, actual, expected, what=""):
     """For the long-context models with raised q/k norm weights."""
     assert_close(dtype, actual, expected, what, rms_rel=BF16_LONG_RMS_REL,
                  max_rel=BF16_LONG_MAX_REL)
+
+
+def paged_attention(q, k_pages, v_pages, table, row_seq, row_pos, heads, kv_heads, scale, window=None,
+                    keep_first=0, chunk=None, slopes=None, sinks=None, softcap=None, gate=None, pool=0,
+                    pool_only=False, pool_k=None, pool_v=None, pool_table=None):
+    """Causal attention over paged keys and values in float64, written from its definition: (output
+    [rows, heads, D], logarithm of the sum of exponentials [rows, heads]); rows with row_seq < 0 are
+    zero.  pool_only: over the pooled entries alone (a row that sees none: zero and minus infinity)."""
+    import torch
+    rows, D = q.shape[0], q.shape[1] // heads
+    q = q.double().view(rows, heads, D)
+    out = torch.zeros(rows, heads, D, dtype=torch.float64)
+    logs = torch.full((rows, heads), float("-inf"), dtype=torch.float64)
+    for r in range(rows):
+        seq, p = row_seq[r], row_pos[r]
+        if seq < 0:
+            continue
+        seen = [t for t in range(p + 1)
+                if (not window or t > p - window or t < keep_first) and (not chunk or t // chunk == p // chunk)]
+        blocks = max(0, (p - window + 1) // pool) if pool else 0
+        for h in range(heads):
+            g = h // (heads // kv_heads)
+            scores, values = [], []
+            if not pool_only:
+                at = [(int(table[seq][t // 64]), t % 64) for t in seen]
+                keys = torch.stack([k_pages[page, g, slot] for page, slot in at]).double()
+                s = keys @ q[r, h] * scale
+                s = softcap * torch.tanh(s / softcap) if softcap else s
+                if slopes is not None:
+                    s = s - slopes[h].double() * (p - torch.tensor(seen, dtype=torch.float64))
+                scores.append(s)
+                values.append(torch.stack([v_pages[page, g, slot] for page, slot in at]).double())
+            if blocks:
+                at = [(int(pool_table[seq][b // 64]), b % 64) for b in range(blocks)]
+                s = torch.stack([pool_k[page, g, slot] for page, slot in at]).double() @ q[r, h] * scale
+                scores.append(softcap * torch.tanh(s / softcap) if softcap else s)
+                values.append(torch.stack([pool_v[page, g, slot] for page, slot in at]).double())
+            if not scores:
+                continue
+            s, v = torch.cat(scores), torch.cat(values)
+            if sinks is not None and not pool_only:
+                s = torch.cat([s, sinks[h].double()[None]])
+                v = torch.cat([v, torch.zeros(1, D, dtype=torch.float64)])
+            logs[r, h] = torch.logsumexp(s, 0)
+            out[r, h] = torch.softmax(s, 0) @ v
+            if gate is not None:
+                out[r, h] *= torch.sigmoid(gate[r, h].double())
+    return out, logs

@@ -1,7 +1,9 @@
 """Float32 prompts through the matrix-instruction kernel against the general kernel, which takes
-queries that are not 16-byte aligned, and a row alone against the same row among others."""
+queries that are not 16-byte aligned, against attention in float64, and a row alone against the same
+row among others."""
 import pytest
 import torch
+from helpers import paged_attention
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -69,5 +71,14 @@ def test_prompts(option, D, heads, kv_heads):
     assert not bool(torch.isnan(fast).any())
     assert (general - fast).abs().max().item() <= 2e-6 * general.abs().max().clamp(min=1.0).item()
     assert torch.equal(general[-1], fast[-1])                   # padding is not written
+    # against float64 (see the decode kernel's test for the bound): every seventh row, and the last
+    some = sorted({*range(0, rows - 1, 7), rows - 2})
+    host = {n: x.cpu() if isinstance(x, torch.Tensor) else x for n, x in more.items()}
+    if "gate" in host:
+        host["gate"] = host["gate"][some]
+    want, _ = paged_attention(q[some].cpu(), k, v, table, [row_seq[r] for r in some], [row_pos[r] for r in some],
+                              heads, kv_heads, D ** -0.5, **host)
+    got = fast[some].double().view(len(some), heads, D)
+    assert (got - want).abs().max().item() <= 4e-6 * want.abs().max().clamp(min=1.0).item()
     alone = run(q, [(s, first + i, 1) for s, first, npos in items for i in range(npos)])
     assert torch.equal(alone, fast)

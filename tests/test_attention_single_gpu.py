@@ -1,6 +1,8 @@
-"""Decoding through the generic kernels: one position an item against the kernel of many rows."""
+"""Decoding through the generic kernels: one position an item against the kernel of many rows, and
+against attention in float64."""
 import pytest
 import torch
+from helpers import paged_attention
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -72,3 +74,19 @@ def test_one_position_an_item(option, D, heads, kv_heads, dtype, splits):
     bound = 2e-6 * slow.abs().max().clamp(min=1.0) + (2.0 ** -7 * slow.abs() if dtype == torch.bfloat16 else 0.0)
     assert bool(((slow - fast).abs() <= bound).all())
     assert torch.equal(slow[-1], fast[-1])                      # padding is not written
+    # Against float64: scores of a few units are sums of D products (some 1e-6 off), and a weight is
+    # off by what its score is; the sums over keys and their join add a few roundings
+    host = {n: x.cpu() if isinstance(x, torch.Tensor) else x for n, x in more.items()}
+    want, logs = paged_attention(q.cpu(), k, v, table, [0, 1, 2, 3, 4, -1], [n - 1 for n in contexts] + [0], heads,
+                                 kv_heads, D ** -0.5, **host)
+    if how.get("pool_only"):
+        sums, top, total = fast[:, :, :D], fast[:, :, D], fast[:, :, D + 1]
+        live = logs[:-1].isfinite()
+        assert torch.equal(total[:-1] > 0, live)
+        assert ((top + total.log())[:-1][live] - logs[:-1][live]).abs().max().item() <= 4e-6
+        got, want = (sums / total[:, :, None])[:-1][live].double(), want[:-1][live]
+        assert ((got - want).abs() <= 4e-6 * want.abs().max().clamp(min=1.0)).all()
+        return
+    got, want = fast.double().view(rows, heads, D)[:-1], want[:-1]
+    bound = 4e-6 * want.abs().max().clamp(min=1.0) + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0.0)
+    assert ((got - want).abs() <= bound).all()
