@@ -1738,8 +1738,8 @@ def delta_chunks(conv, proj, a_log, dt_bias, state, shape: DeltaShape, seq_in, s
                  seq_row0, o_raw, q_scale: float, unit_eps: float, scratch, longest: int,
                  least: int = 1) -> None:
     """What `delta_rule` does with one decay a head, by chunks of 64 tokens: heads of 64 or 128
-    elements; longest: the most rows that a
-    sequence of the step brings; sequences of fewer than `least` are left alone."""
+    elements; longest: the most rows that a sequence of the step brings; sequences of fewer than
+    `least` are left alone."""
     lib = library("delta_rule")
     rows = conv.shape[0]
     n_seqs = seq_count.numel()
@@ -1854,9 +1854,9 @@ def ssm_conv(proj, conv_w, conv_b, state, shape: SsmShape, row_pos, row_seq, seq
 
 def ssm_scan(conv, proj, a_log, dt_bias, d_skip, state, shape: SsmShape, seq_in, seq_out,
              seq_count, seq_row0, y_raw, most: int = EVERY) -> None:
-    """The recurrence over the rows of every sequence of at most `most`: S <- exp(-exp(a_log) dt) S + dt B x^T from row
-    `seq_in[s]` of `state`, y = S^T C + d_skip x to `y_raw` [n, inner] float32, the last S to row
-    `seq_out[s]`; dt = softplus(proj's dt column + dt_bias)."""
+    """The recurrence over the rows of every sequence of at most `most`: S <- exp(-exp(a_log) dt) S +
+    dt B x^T from row `seq_in[s]` of `state`, y = S^T C + d_skip x to `y_raw` [n, inner] float32, the
+    last S to row `seq_out[s]`; dt = softplus(proj's dt column + dt_bias)."""
     lib = library("ssm")
     n = y_raw.shape[0]
     nsplit, stride = _ssm_proj(proj, n, shape)
@@ -1887,11 +1887,10 @@ def ssm_chunk_scratch(rows, seqs, shape: SsmShape, least=1) -> int:
 
 
 def ssm_chunks(conv, proj, a_log, dt_bias, d_skip, state, shape: SsmShape, seq_in, seq_out,
-               seq_count, seq_row0, y_raw, scratch, longest: int,
-               least: int = 1) -> None:
+               seq_count, seq_row0, y_raw, scratch, longest: int, least: int = 1) -> None:
     """What `ssm_scan` does, by chunks of 64 tokens: states of 64 or 128 rows and columns;
-    longest: the most rows that a
-    sequence of the step brings; sequences of fewer than `least` are left alone."""
+    longest: the most rows that a sequence of the step brings; sequences of fewer than `least` are
+    left alone."""
     lib = library("ssm")
     n = y_raw.shape[0]
     nsplit, stride = _ssm_proj(proj, n, shape)
@@ -2117,11 +2116,10 @@ def la_chunk_scratch(rows, seqs, heads, key_dim, value_dim, least=1) -> int:
 
 
 def la_chunks(act, decay, state, seq_in, seq_out, seq_count, seq_row0, o_raw, scratch, heads,
-              key_dim, value_dim, longest: int,
-              least: int = 1) -> None:
+              key_dim, value_dim, longest: int, least: int = 1) -> None:
     """What `la_scan` does with activated rows, by chunks of 64 tokens: heads of 64 or 128
-    elements; longest: the most rows that a
-    sequence of the step brings; sequences of fewer than `least` are left alone."""
+    elements; longest: the most rows that a sequence of the step brings; sequences of fewer than
+    `least` are left alone."""
     lib = library("linear_attention")
     n, stride = act.shape
     n_seqs = seq_count.numel()

@@ -286,7 +286,8 @@ extern "C" int ei_la_out(const float* o_raw, const void* proj, int proj_dtype, i
 }
 
 // The recurrence over a prompt's rows in chunks (see recurrence_chunks.h).  act: float32 [N,
-// row_stride] with q, k and v as `ei_la_activate` leaves them.  Sequences of fewer than `least` rows are left to the walk.
+// row_stride] with q, k and v as `ei_la_activate` leaves them.  Sequences of fewer than `least` rows are left
+// to the walk.
 // scratch: `scratch_floats` floats, at least chunk_places chunks of H heads; longest: the most
 // rows that a sequence brings.
 extern "C" int ei_la_chunk_floats(int DK, int DV) {

@@ -489,7 +489,8 @@ extern "C" int ei_mlstm_chunks(const void* proj, int dtype, const float* i_bias,
                                long long scratch_floats, int rows, int n_seqs, int heads, int dim,
                                int vdim, float cap, float q_scale, float bottom_eps, int longest, int least,
                                hipStream_t stream) {
-  EI_REQUIRE(n_seqs > 0 && heads > 0 && rows >= 1 && longest >= 1 && longest <= rows && least > 0, "mlstm_chunks: bad sizes");
+  EI_REQUIRE(n_seqs > 0 && heads > 0 && rows >= 1 && longest >= 1 && longest <= rows && least > 0,
+             "mlstm_chunks: bad sizes");
   EI_REQUIRE(ei::chunks::sizes_fit(dim, vdim), "mlstm_chunks: heads of 64 or 128 elements");
   EI_REQUIRE(cap > 0.f, "mlstm_chunks: the cap of the gates must be positive");
   EI_REQUIRE(proj && i_bias && f_bias && state && seq_in && seq_out && seq_count && seq_row0 && o_raw &&

@@ -552,7 +552,8 @@ extern "C" int ei_ssm_scan(const float* conv, const void* proj, int in_dtype, in
 }
 
 // The recurrence over a prompt's rows in chunks (see recurrence_chunks.h): what `ei_ssm_scan` does
-// for states of 64 or 128 rows and heads of 64 or 128 columns.  Sequences of fewer than `least` rows are left to the walk.
+// for states of 64 or 128 rows and heads of 64 or 128 columns.  Sequences of fewer than `least` rows are
+// left to the walk.
 // scratch: `scratch_floats` floats, at least chunk_places chunks of all heads; longest: the most
 // rows that a sequence brings.
 extern "C" int ei_ssm_chunk_floats(int P, int Nst) {

@@ -126,9 +126,9 @@ def test_swiglu_with_gate_and_up_in_strips(lib, dtype, I, strip):
 @pytest.mark.parametrize("shape", [(1, 381, 96), (5, 64, 200), (70, 130, 33), (130, 257, 512),
                                    (8, 100, 1000), (40, 4100, 1028), (6, 77, 260), (200, 300, 264)])
 def test_gemm_f32(lib, shape):
-    """Few rows take the weight-streaming kernel (K in fours), many the tiled one; both sum
-    every output over k in ascending order, so a row gives the same bits alone, among up to
-    8 rows and among many."""
+    """K in fours: few rows take one matrix-core kernel, many another, and both sum an output in
+    eight pieces of K joined by one tree; any other K takes one kernel that sums in ascending
+    order.  So a row gives the same bits alone, among up to 8 rows and among many."""
     M, N, K = shape
     a = torch.randn(M, K, device=DEV)
     w = torch.randn(N, K, device=DEV)
@@ -889,8 +889,9 @@ def test_gemm_f32_at_the_widths_of_real_checkpoints(lib, shape, which):
         out = torch.full((M, N), float("nan"), device=DEV)
         lib.gemm_f32(x[:M], w, out)
         err = (out.double() - expected[:M]).abs().max().item()
-        # every output is one thread's sum over k in ascending order: K roundings of 2^-24 of
-        # partial sums that grow like sqrt(k) add up to about 2^-24 K / 2.4 (one sigma)
+        # every output is eight chains of K / 8 products joined by a tree: a chain's roundings, 2^-24
+        # at most of partial sums that grow like sqrt(k), add up to about 2^-24 (K / 8) / 2.4 (one
+        # sigma), eight of them to 2^-24 K / 6.9, and the seven sums of the tree to 2^-24 sqrt(K)
         assert err <= 6 * 2.0 ** -24 * K, f"{shape} {which} {M} rows: max error {err:.3e}"
     del expected
     torch.cuda.empty_cache()
