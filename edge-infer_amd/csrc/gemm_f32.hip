@@ -496,17 +496,24 @@ extern "C" int ei_gemm_f32(const float* A, const float* W, float* C, int M, int 
       const long long rows = (M + 16LL * rt - 1) / (16 * rt), cols = (N + 16LL * ct - 1) / (16 * ct);
       return rows * (rows <= kFewRowTiles ? (cols + 7) / 8 * 8 : cols);
     };
-    // From a block of 128 x 128 for every unit on, those (1,024 rows, 4,096 outputs, K 1,024: 99 -> 78 us,
-    // 512 rows, 6,144 outputs, three quarters of the units: 76 both; 2,048 rows over a vocabulary of
-    // 151,936: 8,575 -> 5,581, 100 rows 522 -> 380).
+    // Blocks of 128 x 128 where they are done sooner: a unit holds one at a time, and a round of them over
+    // the chip lasts as long as three rounds of 64 x 64 tiles (K 1,024: 75 to 78 us against 25 to 29).  Rows x
+    // outputs x K, us by 128 x 128 and by 64 x 64: taken 1,024 x 4,096 x 1,024 78 and 100, 513 x 6,144 x 2,048
+    // 150 and 179, 100 x 151,936 x 1,024 380 and 525, 2,048 x 24,576 x 4,096 3,520 and 4,650; left, a last round
+    // being nearly empty, 261 x 11,264 x 2,048 290 and 181, 800 x 6,144 x 4,096 583 and 421.  Over 220 products of
+    // 65 to 3,554 rows the choice is within 3 % of the better of the two.
     const long long big_rows = (M + kTile - 1LL) / kTile, big_cols = (N + kTile - 1LL) / kTile;
     const long long big = big_rows * ((big_cols + 7) / 8 * 8);
-    if (big_rows * big_cols >= units) {
+    const long long big_rounds = (big_rows * big_cols + units - 1) / units;
+    const long long small_rounds = (blocks_of(4, 4) + units - 1) / units;
+    if (3 * big_rounds < small_rounds) {
       EI_REQUIRE(big <= 0x7fffffff, "gemm_f32: too many outputs for one launch");
       gemm_f32_lds_kernel<<<static_cast<unsigned>(big), kTileThreads, 0, stream>>>(
           A, W, C, M, N, K, lda, ldw, ldc, static_cast<int>(big_rows), static_cast<int>(big_cols));
       EI_LAUNCH_CHECK();
     }
+    EI_REQUIRE(grid_of(2, 2) <= 0x7fffffff || blocks_of(4, 4) <= 0x7ffffff0,
+               "gemm_f32: too many outputs for one launch");
     // else the largest tile that leaves no compute unit without a block
 #define EI_TILE(RT, CT)                                                                     \
   gemm_f32_tile_kernel<RT, CT><<<static_cast<unsigned>(grid_of(RT, CT)), 256, 0, stream>>>( \

@@ -6,10 +6,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("N,K", [(1, 4), (17, 20), (64, 128), (100, 1028), (130, 2052), (4099, 68),
-                                 (65600, 36), (16500, 1028), (16411, 2052), (33000, 4)])
+                                 (65600, 36), (10500, 1028), (10411, 2052), (49411, 4)])
 def test_products_of_every_number_of_rows_within_the_bound_and_the_same_bits(N, K):
-    """Rows 1 .. 64 take the kernel of few rows, more the tiles of 32 x 32, 32 x 64 and 64 x 64 or,
-    from 256 tiles of 128 x 128 on, those.
+    """Rows 1 .. 64 take the kernel of few rows, more the tiles of 32 x 32, 32 x 64 and 64 x 64 or those
+    of 128 x 128 (257 and 300 rows of the outputs above 10,000, 65 and 100 of 49,411 too).
     A sum of K float32 products in any order is within K u sum |a w| of the exact one (u = 2^-24,
     and one more u for a product's own rounding); a row has the same bits in every kernel."""
     from edge_infer_amd.csrc import lib
