@@ -101,10 +101,12 @@ class GatedDelta:
 
     # From so many tokens of a sequence on, by chunks and not token by token, where a head has one
     # decay (16 heads of 128 x 128: 2,048 tokens 671 us by tokens and 129 by chunks, 96 tokens 35 and
-    # 28, beside 32 sequences of one token 71 and 62).  A step of so few rows is the host's, which
-    # pays for two launches more (2k Tirurax, whole steps: 128 tokens 1,208 and 1,235 us, 192 tokens
-    # 1,240 and 1,267, beside 8 decoding sequences 1,347 and 1,236, 256 tokens 1,305 and 1,147).
-    CHUNK_FROM = 192
+    # 28, beside 32 sequences of one token 71 and 62).  Whole steps of the 2k Tirurax, by tokens and by
+    # chunks, us: in float32 one prompt of 63 tokens 2,101 and 2,128, 95 the same, 127 2,321 and 2,260,
+    # 191 3,385 and 3,255; in bfloat16, where a lone short prompt is the host's, 95 tokens 1,154 and
+    # 1,174, 127 1,163 and 1,190, 191 1,252 and 1,208, 8 of 150 2,442 and 2,404, 16 of 128 3,262 and
+    # 3,149, 16 of 8 to 193 3,122 and, from 192, 160, 96 and 16 on, 3,150, 3,112, 2,881 and 2,849.
+    CHUNK_FROM = 96
 
     @classmethod
     def kernel_libraries(cls, spec, dtype):

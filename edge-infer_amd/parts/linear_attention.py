@@ -29,9 +29,9 @@ class LinearAttention:
     ACTIVATE_ROWS = 64       # from so many rows of a prompt step on, q, k and v are activated aside
     # From so many tokens of a sequence on, by chunks and not token by token (16 heads of 128 x 128:
     # 2,048 tokens 785 us by tokens and 77 by chunks, 96 tokens 27 and 30, 160 tokens 42 and 32; whole
-    # steps of the 2k Gopuzen: 128 tokens 2,120 and 2,151 us, 160 tokens 2,214 and 2,206, beside 8
-    # decoding sequences 2,470 and 2,299).
-    CHUNK_FROM = 160
+    # steps of the 2k Gopuzen: 128 tokens 2,085 and 2,120 us, 8 of 100 3,342 and 3,256, 8 of 150 4,088
+    # and 3,774, 16 of 128 5,023 and 4,915).
+    CHUNK_FROM = 96
 
     @property
     def capture_safe(self):

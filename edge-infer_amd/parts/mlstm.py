@@ -41,10 +41,13 @@ class MatrixMemory:
         return min(self.proj.capture_rows, self.o.capture_rows)
 
     # From so many tokens of a sequence on, by chunks and not token by token (16 heads of 128 x 128 in
-    # bfloat16: 64 tokens 46 us by tokens and 40 by chunks, 2,048 tokens 1,300 and 92; whole steps of
-    # the 2k Zadenex in bfloat16, slices added up included: 64 tokens 1,511 and 1,264 us, 256 tokens
-    # 4,190 and 1,598, 64 tokens beside 32 decoding sequences 2,572 and 1,501)
-    CHUNK_FROM = 64
+    # bfloat16: 64 tokens 46 us by tokens and 40 by chunks, 2,048 tokens 1,300 and 92).  Whole steps of
+    # the 2k Zadenex, by tokens and by chunks, us: in bfloat16, slices added up included, one prompt of
+    # 24 tokens 1,194 and 1,232, 40 1,235 and 1,242, 63 1,522 and 1,242, 256 4,190 and 1,598, 8 of 40
+    # 2,063 and 2,102, 64 beside 32 decoding sequences 2,572 and 1,501; in float32 24 tokens 2,031 and
+    # 1,985, 40 2,835 and 2,682, 63 3,591 and 3,331, four of 28 to 137 8,410 and, from 64 and from 32
+    # on, 8,040 and 7,833.
+    CHUNK_FROM = 32
 
     @classmethod
     def parameters(cls, spec, hidden):

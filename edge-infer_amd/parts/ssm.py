@@ -59,8 +59,8 @@ class StateSpace:
 
     # From so many tokens of a sequence on, by chunks and not token by token (16 heads of 128 columns,
     # state 128: 64 tokens 29 us by tokens and 34 by chunks, 96 tokens 41 and 35, 2,048 tokens 790 and
-    # 82; whole steps of the 2k Vafepel: 64 tokens 1,149 and 1,178 us, 96 tokens 1,258 and 1,248,
-    # beside 32 decoding sequences 1,584 and 1,545)
+    # 82; whole steps of the 2k Vafepel: 63 tokens 1,183 and 1,209 us, 95 tokens 1,298 and 1,292, 127
+    # 1,407 and 1,361, 96 beside 32 decoding sequences 1,584 and 1,545)
     CHUNK_FROM = 96
 
     @classmethod
