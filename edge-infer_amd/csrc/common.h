@@ -193,15 +193,20 @@ __device__ __forceinline__ float rows_sum(float x) {
   return __uint_as_float(r.x) + __uint_as_float(r.y);
 }
 
-// Sum over the 64 lanes, every lane getting it.  The steps inside a row of 16 lanes are DPP
-// operand modifiers of vector adds (quad permutes, then mirrors of half rows and rows), the
-// two across rows are gfx950's row swaps; no step goes through LDS as a shuffle would.
-__device__ __forceinline__ float wave_sum(float v) {
+// Sum over the 16 lanes of a row, every lane getting it: DPP operand modifiers of vector adds
+// (quad permutes, then mirrors of half rows and rows).
+__device__ __forceinline__ float row16_sum(float v) {
   v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xb1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
   v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4e, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
   v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, false));  // row_half_mirror
   v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xf, 0xf, false));  // row_mirror
-  return rows_sum(v);
+  return v;
+}
+
+// Sum over the 64 lanes, every lane getting it: inside rows as above, the two steps across rows are
+// gfx950's row swaps; no step goes through LDS as a shuffle would.
+__device__ __forceinline__ float wave_sum(float v) {
+  return rows_sum(row16_sum(v));
 }
 
 __device__ __forceinline__ float wave_max(float v) {

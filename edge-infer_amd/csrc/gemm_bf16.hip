@@ -19,17 +19,18 @@
 // (operators/src/cuda/execution.cu:319-323); the sums stay float32 and the consumer rounds
 // once when it stores in the storage type.
 #include "common.h"
+#include "gemm_whole.h"
 
 #include <type_traits>
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
+using ei::bf16x8;
+using ei::f32x4;
+using ei::kPackedTile;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
 constexpr int kSums = 0, kGated = 1, kGatedBias = 2, kPlain = 3;    // see skinny_gemm_kernel
-constexpr int kPackedTile = 16 * 32;      // elements of one packed tile: 16 rows x 32 k, 1 KB
 
 // MB * 16 rows of X per workgroup, any K range.  A workgroup is WAVES waves, each owning
 // STRIPS strips of 16 rows of W; X travels through LDS one K-tile (KT: 256, or 128 where two
@@ -50,14 +51,16 @@ constexpr int kPackedTile = 16 * 32;      // elements of one packed tile: 16 row
 // the form with 128 rows and two strips has no registers to spare).  kPlain: every strip stands
 // for itself, `gated_out` [M, N] takes ei::activate(sum), with sums that start at `bias` unless
 // it is null.
+// STATS (kSums, packed W, at most 16 rows): the rows of X still have to be divided by their root mean
+// square, see ei::RowNorm.
 // The next kernel then reads one bfloat16 matrix; the alternative writes float32 sums and reads
 // them again in a launch of its own, 3.4 to 5 us a layer of a decode step.
-template <int MB, int WAVES, bool PACKED, int END, int STRIPS, int KT>
+template <int MB, int WAVES, bool PACKED, int END, int STRIPS, int KT, bool STATS = false>
 __global__ void __launch_bounds__(WAVES * EI_WAVE)
 skinny_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X,
                    float* __restrict__ out, bf16_t* __restrict__ gated_out, int M, int N, int K,
                    int k_per_split, int row_groups, ei::GateAct act,
-                   const float* __restrict__ bias) {
+                   const float* __restrict__ bias, const float* __restrict__ stats, float eps) {
   constexpr bool GATED = END == kGated || END == kGatedBias;
   constexpr int JN = KT / 32;             // MFMA steps per K-tile
   static_assert(KT == 256 || (KT == 128 && PACKED), "K-tiles of 256, or 128 with packed weights");
@@ -103,6 +106,10 @@ skinny_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X,
   for (int s = 0; s < STRIPS; ++s)
     w_lane[s] = (static_cast<unsigned>(min(strip + s, n_strips - 1)) * kPackedTile + lane * 8) * 2u;
   const size_t tile_stride = static_cast<size_t>(n_strips) * kPackedTile;
+
+  static_assert(!STATS || (PACKED && STRIPS == 1 && MB == 1 && END == kSums), "see ei::RowNorm");
+  ei::RowFactors<1> factors;
+  if constexpr (STATS) factors.ask(stats, M, K, t);
 
   f32x4 acc[MB][STRIPS];
 #pragma unroll
@@ -348,6 +355,13 @@ skinny_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X,
     }
   }
 
+  if constexpr (STATS) {
+    __shared__ float factor[16];
+    factors.finish(factor, K, eps, t);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[0][0][r] *= factor[r16];
+  }
   if constexpr (END == kPlain) {
 #pragma unroll
     for (int s = 0; s < STRIPS; ++s) {
@@ -537,10 +551,10 @@ extern "C" int ei_skinny_gemm_splits(int M, int N, int K, int max_splits) {
 
 namespace {
 
-template <int MB, bool PACKED, int END, int STRIPS, int KT = 256>
+template <int MB, bool PACKED, int END, int STRIPS, int KT = 256, bool STATS = false>
 void launch_tile_kernel(const bf16_t* w, const bf16_t* x, float* out, bf16_t* gated_out, int M,
                         int N, int K, int k_per_split, int splits, const ei::GateAct& act,
-                        const float* bias, hipStream_t stream) {
+                        const float* bias, const ei::RowNorm& rs, hipStream_t stream) {
   const int n_strips = ((N + 15) / 16 + STRIPS - 1) / STRIPS;     // what a wave owns
   const int row_groups = (M + MB * 16 - 1) / (MB * 16);
   const int waves = tile_kernel_waves(n_strips, splits, row_groups,
@@ -549,20 +563,20 @@ void launch_tile_kernel(const bf16_t* w, const bf16_t* x, float* out, bf16_t* ga
   if (row_groups > 1) strip_blocks = (strip_blocks + 7) / 8 * 8;   // whole rounds of the dies
   dim3 grid(strip_blocks * row_groups, splits);
   if (waves == 4)
-    skinny_gemm_kernel<MB, 4, PACKED, END, STRIPS, KT><<<grid, 4 * EI_WAVE, 0, stream>>>(
-        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias);
+    skinny_gemm_kernel<MB, 4, PACKED, END, STRIPS, KT, STATS><<<grid, 4 * EI_WAVE, 0, stream>>>(
+        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias, rs.squares, rs.eps);
   else if (waves == 6)
-    skinny_gemm_kernel<MB, 6, PACKED, END, STRIPS, KT><<<grid, 6 * EI_WAVE, 0, stream>>>(
-        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias);
+    skinny_gemm_kernel<MB, 6, PACKED, END, STRIPS, KT, STATS><<<grid, 6 * EI_WAVE, 0, stream>>>(
+        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias, rs.squares, rs.eps);
   else
-    skinny_gemm_kernel<MB, 8, PACKED, END, STRIPS, KT><<<grid, 8 * EI_WAVE, 0, stream>>>(
-        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias);
+    skinny_gemm_kernel<MB, 8, PACKED, END, STRIPS, KT, STATS><<<grid, 8 * EI_WAVE, 0, stream>>>(
+        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias, rs.squares, rs.eps);
 }
 
 template <bool PACKED, int END>
 int launch_skinny(const void* X, const void* W, float* out, void* gated_out, int M, int N, int K,
                   int splits, hipStream_t stream, const ei::GateAct& act = ei::GateAct{0, 0.f, 1.f},
-                  const float* bias = nullptr) {
+                  const float* bias = nullptr, const ei::RowNorm& rs = ei::RowNorm{nullptr, 0.f}) {
   EI_REQUIRE(act.kind >= 0 && act.kind <= (END == kPlain ? 3 : 2),
              "gemm_bf16_skinny_gated: unknown activation");
   EI_REQUIRE(M >= 1 && M <= kMaxRows, "gemm_bf16_skinny: rows must lie in 1..256");
@@ -587,22 +601,48 @@ int launch_skinny(const void* X, const void* W, float* out, void* gated_out, int
   const bf16_t* x = static_cast<const bf16_t*>(X);
   const bf16_t* w = static_cast<const bf16_t*>(W);
   bf16_t* g = static_cast<bf16_t*>(gated_out);
+  EI_REQUIRE(!rs.squares || (PACKED && (END == kSums || END == kGated) && M <= ei::kWholeRows && K % 64 == 0 &&
+                             K <= ei::kStatsWidth && rs.eps > 0.f &&
+                             (reinterpret_cast<uintptr_t>(rs.squares) & 15) == 0),
+             "gemm_bf16_skinny: a norm is finished for at most 16 rows of at most 4096 columns, a multiple of 64");
+  if constexpr (PACKED && (END == kGated || END == kGatedBias || END == kPlain)) {
+    // (a plain activation of 9 to 16 rows: 2048 -> 8192 takes 10.6 us that way, 10.1 with X in LDS)
+    if (M <= (END == kPlain ? 8 : ei::kWholeRows)) {
+      constexpr int how = END == kPlain ? ei::kActivatedRows : ei::kGatedRows;
+      if (rs.squares) {
+        if constexpr (END == kGated)
+          ei::launch_whole_product<how, true, false>(w, x, M, N, K, nullptr, nullptr, g, const_cast<float*>(rs.squares), rs.eps, act, stream);
+      } else if (END != kGated && bias) {
+        if constexpr (END != kGated)
+          ei::launch_whole_product<how, false, true>(w, x, M, N, K, nullptr, bias, g, nullptr, 0.f, act, stream);
+      } else {
+        ei::launch_whole_product<how, false, false>(w, x, M, N, K, nullptr, nullptr, g, nullptr, 0.f, act, stream);
+      }
+      EI_LAUNCH_CHECK();
+    }
+  }
+  if (rs.squares) {
+    if constexpr (PACKED && END == kSums)
+      launch_tile_kernel<1, true, END, 1, 256, true>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, rs, stream);
+    EI_LAUNCH_CHECK();
+  }
   if (mode.strips == 2) {
     if constexpr (PACKED) {
       if (MB == 4)
-        launch_tile_kernel<4, PACKED, END, 2, 128>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
+        launch_tile_kernel<4, PACKED, END, 2, 128>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, rs, stream);
       else
-        launch_tile_kernel<8, PACKED, END, 2, 128>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
+        launch_tile_kernel<8, PACKED, END, 2, 128>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, rs, stream);
     }
   } else if (MB == 1) {
-    launch_tile_kernel<1, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
+    if constexpr (!PACKED || END == kSums || END == kPlain)
+      launch_tile_kernel<1, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, rs, stream);
   } else if (MB == 2) {
-    launch_tile_kernel<2, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
+    launch_tile_kernel<2, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, rs, stream);
   } else if (MB == 4) {
-    launch_tile_kernel<4, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
+    launch_tile_kernel<4, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, rs, stream);
   } else {
     if constexpr (PACKED)
-      launch_tile_kernel<8, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, stream);
+      launch_tile_kernel<8, PACKED, END, 1>(w, x, out, g, M, N, K, k_per_split, splits, act, bias, rs, stream);
   }
   EI_LAUNCH_CHECK();
 }
@@ -624,9 +664,12 @@ extern "C" int ei_gemm_bf16_skinny(const void* X, const void* W, float* out, int
 // order in which a wave's lanes hold an MFMA operand.  A wave's load is then one contiguous
 // kilobyte and the waves that run together read neighbouring kilobytes, which keeps every
 // memory channel busy; rows of W that are 2^n bytes apart do not.
+// `stats` (or null): the rows of X still have to be divided by their root mean square, see ei::RowNorm.
 extern "C" int ei_gemm_bf16_skinny_packed(const void* X, const void* Wp, float* out, int M, int N,
-                                          int K, int splits, hipStream_t stream) {
-  return launch_skinny<true, kSums>(X, Wp, out, nullptr, M, N, K, splits, stream);
+                                          int K, int splits, const float* stats, float eps,
+                                          hipStream_t stream) {
+  return launch_skinny<true, kSums>(X, Wp, out, nullptr, M, N, K, splits, stream,
+                                    ei::GateAct{0, 0.f, 1.f}, nullptr, ei::RowNorm{stats, eps});
 }
 
 // Gated feed-forward in one pass: W [N, K] holds, in strips of 16 rows, the gate rows of 16
@@ -636,11 +679,15 @@ extern "C" int ei_gemm_bf16_skinny_packed(const void* X, const void* Wp, float* 
 // of K in one slice.  `packed`: W is in the streaming layout of ei_gemm_bf16_skinny_packed.
 extern "C" int ei_gemm_bf16_skinny_gated(const void* X, const void* W, void* act, int M, int N,
                                          int K, int packed, int kind, float limit, float alpha,
-                                         const float* bias, hipStream_t stream) {
+                                         const float* bias, const float* stats, float eps,
+                                         hipStream_t stream) {
   const ei::GateAct how{kind, limit, alpha};
+  EI_REQUIRE(!stats || (packed && !bias), "gemm_bf16_skinny_gated: sums of squares go with packed weights and no bias");
   if (packed && bias)
     return launch_skinny<true, kGatedBias>(X, W, nullptr, act, M, N, K, 1, stream, how, bias);
-  if (packed) return launch_skinny<true, kGated>(X, W, nullptr, act, M, N, K, 1, stream, how);
+  if (packed)
+    return launch_skinny<true, kGated>(X, W, nullptr, act, M, N, K, 1, stream, how, nullptr,
+                                       ei::RowNorm{stats, eps});
   if (bias)
     return launch_skinny<false, kGatedBias>(X, W, nullptr, act, M, N, K, 1, stream, how, bias);
   return launch_skinny<false, kGated>(X, W, nullptr, act, M, N, K, 1, stream, how);
@@ -653,4 +700,23 @@ extern "C" int ei_gemm_bf16_skinny_act(const void* X, const void* W, void* out, 
   const ei::GateAct how{kind, 0.f, 1.f};
   if (packed) return launch_skinny<true, kPlain>(X, W, nullptr, out, M, N, K, 1, stream, how, bias);
   return launch_skinny<false, kPlain>(X, W, nullptr, out, M, N, K, 1, stream, how, bias);
+}
+
+// residual [M, N] float32 += X [M, K] bfloat16 . W^T in place, for at most 16 rows and W in the
+// streaming layout; rows [M, N] bfloat16 and squares [M, N / 16] float32 are what a norm of the
+// residual with this weight (float32 [N]) leaves to the products that read it (ei::kAddRows).
+extern "C" int ei_gemm_bf16_add(const void* X, const void* Wp, float* residual, const float* weight,
+                                void* rows, float* squares, int M, int N, int K, hipStream_t stream) {
+  EI_REQUIRE(X && Wp && residual && weight && rows && squares, "gemm_bf16_add: null pointer");
+  EI_REQUIRE(M >= 1 && M <= ei::kWholeRows, "gemm_bf16_add: rows must lie in 1..16");
+  EI_REQUIRE(N >= 16 && N % 16 == 0 && K >= 8 && K % 8 == 0,
+             "gemm_bf16_add: N must be a multiple of 16, K of 8");
+  EI_REQUIRE(((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Wp) |
+               reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(weight) |
+               reinterpret_cast<uintptr_t>(rows)) & 15) == 0,
+             "gemm_bf16_add: pointers must be 16-byte aligned");
+  ei::launch_whole_product<ei::kAddRows, false, false>(
+      static_cast<const bf16_t*>(Wp), static_cast<const bf16_t*>(X), M, N, K, residual, weight,
+      static_cast<bf16_t*>(rows), squares, 0.f, ei::GateAct{0, 0.f, 1.f}, stream);
+  EI_LAUNCH_CHECK();
 }

@@ -252,9 +252,11 @@ _SIGNATURES = {
         "ei_gemm_bf16_skinny": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                 c_void_p],
         "ei_gemm_bf16_skinny_packed": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
-                                       c_void_p],
+                                       c_void_p, c_float, c_void_p],
         "ei_gemm_bf16_skinny_gated": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
-                                      c_int, c_float, c_float, c_void_p, c_void_p],
+                                      c_int, c_float, c_float, c_void_p, c_void_p, c_float, c_void_p],
+        "ei_gemm_bf16_add": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
+                             c_int, c_void_p],
         "ei_gemm_bf16_skinny_act": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                     c_int, c_void_p, c_void_p],
     },
@@ -2190,7 +2192,6 @@ def la_scan(proj, decay, state, seq_in, seq_out, seq_count, seq_row0, o_raw, hea
         int(bool(activated)), int(most), _stream())
     _check(lib, status, "la_scan")
 
-
 def la_out(o_raw, proj, gate_column: int, norm_w, eps: float, row_seq, out) -> None:
     """out [n, v] = rmsnorm(o_raw) * norm_w * sigmoid(g), g the columns gate_column ..
     gate_column + v - 1 of proj's rows (summed over slices)."""
@@ -2519,9 +2520,47 @@ def pack_weight(w: torch.Tensor) -> torch.Tensor:
     return w.view(strips, 16, tiles, 4, 8).permute(2, 0, 3, 1, 4).contiguous()
 
 
+STATS_WIDTH = 4096      # widest rows whose norm a product finishes (`stats` of the products below)
+WHOLE_ROWS = 16         # most rows of the products whose sums are whole inside a block
+
+
+def _row_stats(stats, m: int, k: int, what: str):
+    """(pointer, eps) of `stats`: None, or (sums of squares [m, k / 16], eps) of rows x that still have
+    to be divided by their root mean square, see `gemm_bf16_add`."""
+    if stats is None:
+        return None, 0.0
+    sums, eps = stats
+    if m > WHOLE_ROWS or k > STATS_WIDTH or k % 64 or tuple(sums.shape) != (m, k // 16):
+        raise KernelError(f"{what}: sums of squares {list(sums.shape)} do not belong to rows [{m}, {k}]")
+    return _gpu(sums, "stats", torch.float32), float(eps)
+
+
+def gemm_bf16_add(x: torch.Tensor, packed: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
+                  rows: torch.Tensor, stats: torch.Tensor) -> None:
+    """residual [m, n] (float32) += x . w^T for at most `WHOLE_ROWS` rows, with the weight given as
+    `pack_weight(w)`; rows [m, n] = the new residual times `weight` [n], rounded to bfloat16, and
+    stats [m, n / 16] = the sums of the new residual's squares, 16 columns each: what the products
+    that read a norm of the residual need of it."""
+    lib = library("gemm_bf16")
+    m, k = x.shape
+    n = residual.shape[1]
+    if (tuple(residual.shape) != (m, n) or tuple(rows.shape) != (m, n) or tuple(weight.shape) != (n,)
+            or n % 16 or tuple(stats.shape) != (m, n // 16)
+            or tuple(packed.shape) != (8 * ((k + 255) // 256), n // 16, 4, 16, 8)):
+        raise KernelError(f"gemm_bf16_add: {list(x.shape)} x packed {list(packed.shape)} -> "
+                          f"{list(residual.shape)}, {list(rows.shape)}, {list(stats.shape)} do not agree")
+    status = lib.ei_gemm_bf16_add(_gpu(x, "x", torch.bfloat16), _gpu(packed, "packed", torch.bfloat16),
+                                  _gpu(residual, "residual", torch.float32),
+                                  _gpu(weight, "weight", torch.float32),
+                                  _gpu(rows, "rows", torch.bfloat16),
+                                  _gpu(stats, "stats", torch.float32), m, n, k, _stream())
+    _check(lib, status, "gemm_bf16_add")
+
+
 def gemm_bf16_skinny_packed(x: torch.Tensor, packed: torch.Tensor, n: int,
-                            out: torch.Tensor) -> None:
-    """`gemm_bf16_skinny` with the weight given as `pack_weight(w)` of a matrix [n, k]."""
+                            out: torch.Tensor, stats=None) -> None:
+    """`gemm_bf16_skinny` with the weight given as `pack_weight(w)` of a matrix [n, k].  `stats`: (sums
+    of squares, eps) of rows that `gemm_bf16_add` wrote; the product is then that of the norm's rows."""
     lib = library("gemm_bf16")
     m, k = x.shape
     if (out.dim() != 3 or tuple(out.shape[1:]) != (m, n) or packed.dim() != 5
@@ -2531,7 +2570,8 @@ def gemm_bf16_skinny_packed(x: torch.Tensor, packed: torch.Tensor, n: int,
     status = lib.ei_gemm_bf16_skinny_packed(_gpu(x, "x", torch.bfloat16),
                                             _gpu(packed, "packed", torch.bfloat16),
                                             _gpu(out, "out", torch.float32), m, n, k,
-                                            out.shape[0], _stream())
+                                            out.shape[0], *_row_stats(stats, m, k, "gemm_bf16_skinny_packed"),
+                                            _stream())
     _check(lib, status, "gemm_bf16_skinny_packed")
 
 
@@ -2548,12 +2588,13 @@ def _fused_weight(w, n: int, k: int, packed: bool, bias, what: str) -> None:
 
 def gemm_bf16_skinny_gated(x: torch.Tensor, w: torch.Tensor, n: int, act: torch.Tensor,
                            packed: bool, activation: str = "silu", limit: float = 0.0,
-                           alpha: float = 1.0, bias: Optional[torch.Tensor] = None) -> None:
+                           alpha: float = 1.0, bias: Optional[torch.Tensor] = None,
+                           stats=None) -> None:
     """act[m, i] = silu(x[m] . gate_i) * (x[m] . up_i) (or another `activation` of `swiglu`) for a weight [n, k] whose rows are, in
     strips of 16, the gate rows of 16 outputs followed by their up rows; `w` is that matrix or
     (packed) its `pack_weight` copy; `bias` (float32 [n], in the order of the rows) is what the
     sums start from.  For at most 256 rows; K is not sliced, so it pays where
-    `skinny_gemm_splits` is 1."""
+    `skinny_gemm_splits` is 1.  `stats` as for `gemm_bf16_skinny_packed` (packed, without a bias)."""
     lib = library("gemm_bf16")
     m, k = x.shape
     if activation not in GATE_ACTIVATIONS:
@@ -2566,7 +2607,7 @@ def gemm_bf16_skinny_gated(x: torch.Tensor, w: torch.Tensor, n: int, act: torch.
                                            _gpu(act, "act", torch.bfloat16), m, n, k, int(packed),
                                            GATE_ACTIVATIONS[activation], float(limit), float(alpha),
                                            None if bias is None else _gpu(bias, "bias", torch.float32),
-                                           _stream())
+                                           *_row_stats(stats, m, k, "gemm_bf16_skinny_gated"), _stream())
     _check(lib, status, "gemm_bf16_skinny_gated")
 
 

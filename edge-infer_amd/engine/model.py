@@ -361,6 +361,10 @@ class DecoderModel:
             turn = self._pass_starts.get(run)
             if turn is not None:
                 pending = self.enter_pass(ctx, residual, pending, embedded, turn)
+            after = run + 1
+            ctx.following = (self.layers[self.spec.schedule[after].layer]
+                             if after < len(self.spec.schedule) and after not in self._pass_starts
+                             else None)
             pending = self.layers[entry.layer].forward(ctx, residual, pending, entry)
         if isinstance(pending, PendingNorm):
             pending.settle(ctx, residual)

@@ -551,8 +551,14 @@ class Attention:
 
     bias_later = True      # forward(..., bias_later=True) hands the last product's bias on
 
-    def forward(self, ctx, x, entry, bias_later=False, projected=None):
-        """The mixer's rows; with `bias_later`, (rows, float32 bias of the output projection
+    def reads_norm_rows(self, rows):
+        return self.qkv.reads_norm_rows(rows)
+
+    def can_add(self, rows):
+        return self.o.can_add(rows)
+
+    def forward(self, ctx, x, entry, bias_later=False, projected=None, add_to=None):
+        """The mixer's rows (with `add_to`, where `can_add`: see `Linear.forward_add`); with `bias_later`, (rows, float32 bias of the output projection
         that is still to be added, or None), for a caller whose next kernel adds it.  `projected`:
         the input product's rows, made by the caller."""
         spec = self.spec
@@ -715,6 +721,9 @@ class Attention:
             lib.gate_rows(qkv, self.gate_column, out)
         ctx.release(None if projected is not None else qkv, None if isinstance(q, lib.DecodeProjection) else q, part_o, part_ml, gate,
                     aside.get("pool_o"), aside.get("pool_ml"))
-        delta = self.o.forward(ctx, out, "attn.o", bias_later=bias_later)
+        if add_to is not None:
+            delta = self.o.forward_add(ctx, out, add_to)
+        else:
+            delta = self.o.forward(ctx, out, "attn.o", bias_later=bias_later)
         ctx.release(out)
         return delta

@@ -264,6 +264,7 @@ class StepContext:
         self.context_bound = max_context if context_bound is None else context_bound
         self.fixed_shape = fixed_shape
         self.sequences = ()             # engine.batch.SeqStep of every live sequence (host)
+        self.following = None           # the block that reads the stream next, if one does
         self.notes = {}                 # what parts work out once a step and share between layers
 
     def buffer(self, name, shape, dtype=None):
@@ -275,7 +276,8 @@ class StepContext:
         never released lives to the end of the step; None and tensors that are not the
         workspace's are ignored."""
         for which in buffers:
-            self.workspace.release(which)
+            for buffer in getattr(which, "held", (which,)):
+                self.workspace.release(buffer)
 
     def routes(self, chunk_from: int):
         """(`longest`, `most`) of a recurrence that goes by chunks from `chunk_from` tokens of a

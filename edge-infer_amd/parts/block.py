@@ -6,6 +6,8 @@ import torch
 from ..csrc import lib
 from ..weights.loader import ParamSpec
 from .base import StateRequest
+from .linear import AddTo, NormRows
+from .norm import RMSNorm
 from .registry import lookup
 
 
@@ -13,7 +15,9 @@ class PreNormBlock:
     """x += mixer(norm1(x)); x += feed_forward(norm2(x)).
     runtime/include/execution/decoder.hpp:119-168 of the reference.  The second
     addition is left pending: the next block's first norm (or the model's final
-    norm) performs it while reading the row.  A layer may have no feed-forward (then it has
+    norm) performs it while reading the row.  For few rows a sublayer's last product adds to the
+    stream itself and the product that reads the norm finishes it (`Linear.forward_add`), where the
+    sublayers' products can; the norms then have no kernel of their own.  A layer may have no feed-forward (then it has
     no second norm either, and the mixer's output is what is left pending)."""
 
     parts = ("norm1", "mixer", "norm2", "ffn")
@@ -78,16 +82,44 @@ class PreNormBlock:
             self.norm2 = norm_cls(layer_spec.norm, hidden, sub("norm2"), dtype, device)
             self.ffn = ffn_cls(layer_spec.feed_forward, hidden, sub("ffn"), dtype, device)
 
+    def joins(self, rows):
+        """The norm that this block reads the stream through, where it takes its `NormRows`."""
+        return self._joins(self.norm1, self.mixer, rows)
+
+    @staticmethod
+    def _joins(norm, reader, rows):
+        reads = getattr(reader, "reads_norm_rows", None)
+        return norm if type(norm) is RMSNorm and reads is not None and reads(rows) else None
+
+    @staticmethod
+    def _add_to(sublayer, norm, residual, name):
+        """`add_to` for a sublayer whose rows are read through `norm` next."""
+        can = getattr(sublayer, "can_add", None)
+        if norm is None or can is None or not can(residual.shape[0]):
+            return {}
+        return {"add_to": AddTo(residual, norm, name)}
+
     def forward(self, ctx, residual, pending, entry):
-        h = self.norm1.add_norm(ctx, residual, pending, "block.h")
-        ctx.release(pending)             # added into the residual: its storage is free
-        a = self.mixer.forward(ctx, h, entry)
+        rows = residual.shape[0]
+        if isinstance(pending, NormRows):
+            h = pending
+        else:
+            h = self.norm1.add_norm(ctx, residual, pending, "block.h")
+            ctx.release(pending)             # added into the residual: its storage is free
+        after = {} if self.ffn is None else self._add_to(
+            self.mixer, self._joins(self.norm2, self.ffn, rows), residual, "block.h2")
+        a = self.mixer.forward(ctx, h, entry, **after)
         ctx.release(h)
         if self.ffn is None:
             return a
-        h2 = self.norm2.add_norm(ctx, residual, a, "block.h")
-        ctx.release(a)
-        out = self.ffn.forward(ctx, h2)
+        if after:
+            h2 = a
+        else:
+            h2 = self.norm2.add_norm(ctx, residual, a, "block.h")
+            ctx.release(a)
+        joins = getattr(ctx.following, "joins", None)
+        out = self.ffn.forward(ctx, h2, **({} if joins is None else self._add_to(
+            self.ffn, joins(rows), residual, "block.h1")))
         ctx.release(h2)
         return out
 

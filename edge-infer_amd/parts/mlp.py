@@ -105,12 +105,21 @@ class GatedMLP:
 
     bias_later = True      # forward(..., bias_later=True) hands the last product's bias on
 
-    def forward(self, ctx, x, bias_later=False):
-        """The feed-forward's rows; with `bias_later`, (rows, float32 bias of the down
+    def reads_norm_rows(self, rows):
+        return self.gate_up.reads_norm_rows(rows)
+
+    def can_add(self, rows):
+        return self.down.can_add(rows)
+
+    def forward(self, ctx, x, bias_later=False, add_to=None):
+        """The feed-forward's rows (with `add_to`, where `can_add`: see `Linear.forward_add`); with `bias_later`, (rows, float32 bias of the down
         projection that is still to be added, or None): a caller whose next kernel reads the
         rows anyway adds it there and saves a launch."""
         act = self._activated(ctx, x)
-        out = self.down.forward(ctx, act, "mlp.down", bias_later=bias_later)
+        if add_to is not None:
+            out = self.down.forward_add(ctx, act, add_to)
+        else:
+            out = self.down.forward(ctx, act, "mlp.down", bias_later=bias_later)
         ctx.release(act)
         return out
 

@@ -101,7 +101,13 @@ class StateSpace:
         self.skip = f32(params["skip"])
         self.out_norm = f32(params["out_norm.weight"])
 
-    def forward(self, ctx, x, entry):
+    def reads_norm_rows(self, rows):
+        return self.proj.reads_norm_rows(rows)
+
+    def can_add(self, rows):
+        return self.o.can_add(rows)
+
+    def forward(self, ctx, x, entry, add_to=None):
         if not entry.writes_cache:
             raise ValueError("mamba2: a run that only reads another run's state is not "
                              "implemented")
@@ -129,6 +135,7 @@ class StateSpace:
         lib.ssm_out(y_raw, proj, self.out_norm, self.spec.norm_eps, shape, self.spec.norm_parts,
                     meta.row_seq, gated)
         ctx.release(y_raw, proj)
-        delta = self.o.forward(ctx, gated, "ssm.o")
+        delta = (self.o.forward(ctx, gated, "ssm.o") if add_to is None
+                 else self.o.forward_add(ctx, gated, add_to))
         ctx.release(gated)
         return delta
