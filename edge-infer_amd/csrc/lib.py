@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import os
+from array import array
 from ctypes import c_float, c_int, c_longlong, c_ulonglong, c_void_p
 from typing import Dict, Optional
 
@@ -267,6 +268,8 @@ _SIGNATURES = {
         "ei_argmax_static_prepare": [],
         "ei_sample": [c_void_p, c_int, c_int, c_float, c_float, c_int, c_ulonglong, c_void_p,
                       c_void_p, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p],
+        "ei_sample_given": [c_void_p, c_int, c_int, c_float, c_float, c_int, c_ulonglong, c_void_p,
+                            c_void_p, c_void_p, c_void_p, c_void_p, c_longlong, c_void_p],
         "ei_sample_scratch_size": [c_int, c_int],
     },
     "peaks": {
@@ -356,6 +359,15 @@ def _gpu(tensor: torch.Tensor, name: str, dtype=None) -> int:
         raise KernelError(f"{name} must be contiguous")
     if dtype is not None and tensor.dtype != dtype:
         raise KernelError(f"{name} must be {dtype}, got {tensor.dtype}")
+    return tensor.data_ptr()
+
+
+def _written(tensor: torch.Tensor, name: str, dtype) -> int:
+    """A small result: on the GPU, or in pinned host memory, which the kernel then writes itself."""
+    if tensor.is_cuda or not tensor.is_pinned():
+        return _gpu(tensor, name, dtype)
+    if not tensor.is_contiguous() or tensor.dtype != dtype:
+        raise KernelError(f"{name} must be contiguous and {dtype}")
     return tensor.data_ptr()
 
 
@@ -2412,7 +2424,7 @@ def argmax(logits: torch.Tensor, tokens: torch.Tensor, probabilities=None, parti
     if tokens.numel() < rows:
         raise KernelError("argmax: tokens shorter than the rows")
     status = lib.ei_argmax(_gpu(logits, "logits", torch.float32), rows, vocab,
-                           _gpu(tokens, "tokens", torch.int32),
+                           _written(tokens, "tokens", torch.int32),
                            None if probabilities is None
                            else _gpu(probabilities, "probabilities", torch.float32),
                            None if partial is None else _gpu(partial, "partial", torch.float32),
@@ -2444,23 +2456,36 @@ def sample_scratch_size(rows: int, vocab: int) -> int:
     return library("sampling").ei_sample_scratch_size(rows, vocab)
 
 
+SAMPLE_GIVEN_ROWS = 64
+
+
 def sample(logits, temperature, top_p, top_k, seed, streams, counters, tokens,
            probabilities=None, scratch=None) -> None:
     """`scratch` (int32, zero before its first use, see `sample_scratch_size`) lets a wide
-    vocabulary be searched by many blocks a row; the tokens are the same without it."""
+    vocabulary be searched by many blocks a row; the tokens are the same without it.
+    `streams` and `counters`: int32 tensors on the GPU, or two `array('i')` of at most
+    `SAMPLE_GIVEN_ROWS` rows, which go with the launch."""
     lib = library("sampling")
     rows, vocab = logits.shape
-    if tokens.numel() < rows or streams.numel() < rows or counters.numel() < rows:
+    given = isinstance(streams, array)
+    if given:
+        if len(streams) < rows or len(counters) < rows:
+            raise KernelError("sample: per-row arrays shorter than the rows")
+        keys = (streams.buffer_info()[0], counters.buffer_info()[0])
+    else:
+        if streams.numel() < rows or counters.numel() < rows:
+            raise KernelError("sample: per-row arrays shorter than the rows")
+        keys = (_gpu(streams, "streams", torch.int32), _gpu(counters, "counters", torch.int32))
+    if tokens.numel() < rows:
         raise KernelError("sample: per-row arrays shorter than the rows")
-    status = lib.ei_sample(_gpu(logits, "logits", torch.float32), rows, vocab, float(temperature),
-                           float(top_p), int(top_k), int(seed) & (2**64 - 1),
-                           _gpu(streams, "streams", torch.int32),
-                           _gpu(counters, "counters", torch.int32),
-                           _gpu(tokens, "tokens", torch.int32),
-                           None if probabilities is None
-                           else _gpu(probabilities, "probabilities", torch.float32),
-                           None if scratch is None else _gpu(scratch, "scratch", torch.int32),
-                           0 if scratch is None else scratch.numel(), _stream())
+    status = (lib.ei_sample_given if given else lib.ei_sample)(
+        _gpu(logits, "logits", torch.float32), rows, vocab, float(temperature),
+        float(top_p), int(top_k), int(seed) & (2**64 - 1), *keys,
+        _written(tokens, "tokens", torch.int32),
+        None if probabilities is None
+        else _gpu(probabilities, "probabilities", torch.float32),
+        None if scratch is None else _gpu(scratch, "scratch", torch.int32),
+        0 if scratch is None else scratch.numel(), _stream())
     _check(lib, status, "sample")
 
 
