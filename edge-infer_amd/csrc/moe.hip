@@ -587,10 +587,11 @@ moe_gemm_kernel(const bf16_t* __restrict__ a, const int32_t* __restrict__ sorted
 }
 
 // The experts of up to MB * 16 rows: a block an expert and STRIPS strips of 16 rows of its matrix
-// (GATED: of its gate and of its up matrix).  The block finds the pairs that chose its expert
+// (GATED: of its gate and of its up matrix).  Every wave finds the pairs that chose its expert
 // itself, in the order of the pairs (padding rows left out); KS waves share a strip's K out and
-// meet in LDS.  Both operands come from memory straight into operand registers, U steps of 32 at a
-// time.  GATED: the
+// meet in LDS.  Both operands come from memory straight into operand registers, U steps of 32 on
+// their way at once: all loads are unconditional (clamped), since one under a condition is waited for
+// where its branch ends.  GATED: the
 // gated products go to out_act [pairs, N] at the pairs' own places; else the products times the
 // pairs' weights go to out_sum [top, rows, N], slice = the choice; the blocks of "expert" E, where
 // there are such, write the identity experts' slices, weight times the row itself.
@@ -602,8 +603,7 @@ moe_few_kernel(const bf16_t* __restrict__ a, const int32_t* __restrict__ expert,
                bf16_t* __restrict__ out_act, float* __restrict__ out_sum, int rows, int N, int K,
                int top, int E, const bf16_t* __restrict__ x, ei::GateAct how) {
   constexpr int G = GATED ? 2 : 1, WAVES = STRIPS * KS;
-  __shared__ int places[MB * 16];
-  __shared__ int wave_counts[WAVES];
+  __shared__ int places[WAVES][MB * 16];        // every wave its own
   __shared__ float red[WAVES][MB][G][4][EI_WAVE];
   const int e = blockIdx.y, n0 = blockIdx.x * (STRIPS * 16), pairs = rows * top;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / EI_WAVE), lane = threadIdx.x % EI_WAVE;
@@ -617,66 +617,87 @@ moe_few_kernel(const bf16_t* __restrict__ a, const int32_t* __restrict__ expert,
     return;
   }
   const int n_strip = wave / KS, slice = wave % KS;
-  const size_t strip = (static_cast<size_t>(e) * (N / 16) + n0 / 16 + n_strip) * (K / 32);
+  const int steps = K / 32, per = (steps + KS - 1) / KS;
+  const size_t strip = (static_cast<size_t>(e) * (N / 16) + n0 / 16 + n_strip) * steps;
   const bf16_t* w1_strip = w1 + strip * 512 + lane * 8;
   const bf16_t* w2_strip = GATED ? w2 + strip * 512 + lane * 8 : nullptr;
-  const int steps = K / 32, per = (steps + KS - 1) / KS;
-  const int s_begin = slice * per, s_end = min(steps, (slice + 1) * per);
+  const int s_begin = slice * per, s_end = min(steps, (slice + 1) * per);     // (may be none)
+  moe_bf16x8 wa[U], wb[GATED ? U : 1], xf[U][MB];
+  auto load_w = [&](int u, int s0) {            // step s0 + u, or the last one of all
+    const int s = min(s0 + u, steps - 1);
+    wa[u] = __builtin_nontemporal_load(reinterpret_cast<const moe_bf16x8*>(w1_strip + s * 512));
+    if (GATED) wb[u] = __builtin_nontemporal_load(reinterpret_cast<const moe_bf16x8*>(w2_strip + s * 512));
+  };
+  constexpr int Q = 4;                          // 64 pairs each
   int count = 0;
-  for (int base = 0; base < pairs; base += WAVES * EI_WAVE) {
-    const int p = base + threadIdx.x;
-    const bool mine = p < pairs && expert[p] == e && !(row_seq && row_seq[p / top] < 0);
-    const unsigned long long mask = __ballot(mine);
-    if (lane == 0) wave_counts[wave] = __popcll(mask);
-    __syncthreads();
-    int before = count, total = 0;
+  for (int base = 0; base < pairs; base += Q * EI_WAVE) {
+    int32_t chosen[Q], seq[Q];
 #pragma unroll
-    for (int w = 0; w < WAVES; ++w) {
-      if (w < wave) before += wave_counts[w];
-      total += wave_counts[w];
-    }
-    const int at = before + __popcll(mask & ((1ull << lane) - 1ull));
-    if (mine && at < MB * 16) places[at] = p;    // (a row chooses an expert once at most)
-    count += total;
-    __syncthreads();
+    for (int q = 0; q < Q; ++q)
+      if (base + q * EI_WAVE < pairs) {
+        const int p = min(base + q * EI_WAVE + lane, pairs - 1);
+        chosen[q] = expert[p];
+        seq[q] = row_seq ? row_seq[p / top] : 0;
+      }
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      if (base + q * EI_WAVE < pairs) {
+        const int p = base + q * EI_WAVE + lane;
+        const bool mine = p < pairs && chosen[q] == e && seq[q] >= 0;
+        const unsigned long long mask = __ballot(mine);
+        const int at = count + __popcll(mask & ((1ull << lane) - 1ull));
+        if (mine && at < MB * 16) places[wave][at] = p;    // (a row chooses an expert once at most)
+        count += __popcll(mask);
+      }
   }
   count = min(__builtin_amdgcn_readfirstlane(count), MB * 16);
-  if (count == 0) return;
+  if (count == 0) return;                       // (the same for every wave)
+  wave_lds_fence();
   const int r16 = lane % 16, quarter = lane / 16;
   const bf16_t* x_row[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
-    const int p = places[min(mb * 16 + r16, count - 1)];      // (clamped: such rows are not stored)
+    const int p = places[wave][min(mb * 16 + r16, count - 1)];      // (clamped: such rows are not stored)
     x_row[mb] = a + static_cast<size_t>(GATED ? p / top : p) * K + quarter * 8;
   }
+  auto load_x = [&](int u, int s0) {
+    const int s = min(s0 + u, steps - 1);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+      if (mb == 0 || mb * 16 < count) xf[u][mb] = *reinterpret_cast<const moe_bf16x8*>(x_row[mb] + s * 32);
+  };
   moe_f32x4 acc[MB][G];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int g = 0; g < G; ++g) acc[mb][g] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int s0 = s_begin; s0 < s_end; s0 += U) {
-    moe_bf16x8 wa[U], wb[GATED ? U : 1], xf[U][MB];
+  auto multiply = [&](int u) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (s0 + u < s_end) {
-        wa[u] = *reinterpret_cast<const moe_bf16x8*>(w1_strip + (s0 + u) * 512);
-        if (GATED) wb[u] = *reinterpret_cast<const moe_bf16x8*>(w2_strip + (s0 + u) * 512);
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-          if (mb * 16 < count) xf[u][mb] = *reinterpret_cast<const moe_bf16x8*>(x_row[mb] + (s0 + u) * 32);
+    for (int mb = 0; mb < MB; ++mb)
+      if (mb == 0 || mb * 16 < count) {
+        acc[mb][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u], xf[u][mb], acc[mb][0], 0, 0, 0);
+        if (GATED)
+          acc[mb][G - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[u], xf[u][mb], acc[mb][G - 1], 0, 0, 0);
       }
+  };
 #pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (s0 + u < s_end) {
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-          if (mb * 16 < count) {
-            acc[mb][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[u], xf[u][mb], acc[mb][0], 0, 0, 0);
-            if (GATED)
-              acc[mb][G - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[u], xf[u][mb], acc[mb][G - 1], 0, 0, 0);
-          }
-      }
+  for (int u = 0; u < U; ++u) {
+    load_w(u, s_begin);
+    load_x(u, s_begin);
   }
+  __builtin_amdgcn_sched_barrier(0);
+  int s0 = s_begin;
+  for (; s0 + U < s_end; s0 += U) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      multiply(u);
+      load_w(u, s0 + U);
+      load_x(u, s0 + U);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (s0 + u < s_end) multiply(u);
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
@@ -695,7 +716,7 @@ moe_few_kernel(const bf16_t* __restrict__ a, const int32_t* __restrict__ expert,
 #pragma unroll
       for (int w = 0; w < KS; ++w) sum[g] += red[first + w][mb][g][i][from];
     }
-    const int p = places[index];
+    const int p = places[wave][index];
     if (GATED)
       out_act[static_cast<size_t>(p) * N + n0 + n] =
           ei::f32_to_bf16(ei::gated_product<bf16_t>(sum[0], sum[G - 1], how));
@@ -1050,16 +1071,39 @@ extern "C" int ei_moe_experts_few(const void* x, const void* w_gate, const void*
   moe_few_kernel<MB, GATED, STRIPS, KS, U>                                                     \
       <<<dim3(ROWS / (STRIPS * 16), EXPERTS), STRIPS * KS * EI_WAVE, 0, stream>>>(             \
           A, expert, weight, row_seq, W1, W2, ACT, OUT, N, ROWS, COLS, top, E, xb, how)
+  // The second product: waves that share a strip's K out, so that a wave has up to 22 steps, but more
+  // of them while the experts in use (at most `pairs`) leave the chip short of waves.  Measured over
+  // the products' own sizes, a row of W being 2,048 wide: 16 experts of 704 at 16 rows 10.0 us with
+  // one wave a strip, 10.5 with two, 11.4 with four, 20.7 with eight and more steps on their way than
+  // they have; 8 of 2,816 at two rows 12.0, 11.7, 8.5, 9.4.
+  const long long in_use = static_cast<long long>(N) * top < E ? N * top : E;
+  int share = F <= 704 ? 1 : F <= 1408 ? 2 : 4;
+  while (share < 4 && in_use * (W / 16) * share < 2048) share *= 2;
+#define EI_FEW_DOWN(MB, U)                                                                     \
+  do {                                                                                         \
+    if (share == 1) EI_FEW(MB, false, 4, 1, U, down_experts, ab, d, nullptr, nullptr, out, W, F); \
+    else if (share == 2) EI_FEW(MB, false, 2, 2, U, down_experts, ab, d, nullptr, nullptr, out, W, F); \
+    else if (F < 1408) EI_FEW(MB, false, 1, 4, 6, down_experts, ab, d, nullptr, nullptr, out, W, F); \
+    else EI_FEW(MB, false, 1, 4, U, down_experts, ab, d, nullptr, nullptr, out, W, F);         \
+  } while (0)
+  // the first product: eight waves a strip where four would leave the chip with under six a unit
+#define EI_FEW_UP(MB)                                                                          \
+  do {                                                                                         \
+    if (in_use * (F / 16) < 384) EI_FEW(MB, true, 1, 8, 4, E, xb, g, u, ab, nullptr, F, W);    \
+    else EI_FEW(MB, true, 1, 4, 8, E, xb, g, u, ab, nullptr, F, W);                            \
+  } while (0)
   if (N <= 16) {
-    EI_FEW(1, true, 1, 8, 8, E, xb, g, u, ab, nullptr, F, W);
-    EI_FEW(1, false, 1, 8, 8, down_experts, ab, d, nullptr, nullptr, out, W, F);
+    EI_FEW_UP(1);
+    EI_FEW_DOWN(1, 11);
   } else if (N <= 32) {
-    EI_FEW(2, true, 1, 8, 8, E, xb, g, u, ab, nullptr, F, W);
-    EI_FEW(2, false, 1, 8, 8, down_experts, ab, d, nullptr, nullptr, out, W, F);
+    EI_FEW_UP(2);
+    EI_FEW_DOWN(2, 8);
   } else {
     EI_FEW(4, true, 1, 8, 4, E, xb, g, u, ab, nullptr, F, W);
     EI_FEW(4, false, 4, 2, 6, down_experts, ab, d, nullptr, nullptr, out, W, F);
   }
+#undef EI_FEW_UP
+#undef EI_FEW_DOWN
 #undef EI_FEW
   EI_LAUNCH_CHECK();
 }
