@@ -116,13 +116,13 @@ struct DecodePrep {
 // its tile takes them from LDS, since the store of another block may not have landed).
 template <int D, int GB, int W, bool PREP, int EXT>
 __global__ void __launch_bounds__(W * EI_WAVE)
-attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages,
-                   const bf16_t* __restrict__ v_pages, const int32_t* __restrict__ row_pos,
-                   const int32_t* __restrict__ row_seq, const int32_t* __restrict__ page_table,
-                   int table_width, bf16_t* __restrict__ out, float* __restrict__ part_o,
-                   float* __restrict__ part_ml, int nq, int nkv, int head_blocks, int window,
-                   float scale, int n_splits, const int32_t* __restrict__ longest,
-                   DecodePrep prep, AttnExtra extra) {
+attn_decode_kernel(const int32_t* __restrict__ row_pos, const int32_t* __restrict__ row_seq,
+                   const int32_t* __restrict__ page_table, const int32_t* __restrict__ longest,
+                   const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
+                   int table_width, const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
+                   float* __restrict__ part_o, float* __restrict__ part_ml, int nq, int nkv,
+                   int G, int head_blocks, float head_blocks_inv, int window, float scale, int n_splits,
+                   int equal_shares, DecodePrep prep, AttnExtra extra) {
   constexpr int DJ = D / 32;            // MFMA steps over the head dimension
   constexpr int LPR = D / 8;            // lanes that cover one value row with 16-byte loads
   constexpr int KPI = EI_WAVE / LPR;    // value rows per load instruction
@@ -136,115 +136,89 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pa
   const float to_cap = CAP ? 2.f * 1.4426950408889634f * scale / extra.cap : 0.f;
 
   const int row = blockIdx.x;                      // packed row = sequence index in decode
-  const int g = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks;
-  const int split = blockIdx.z;
-  const int seq = row_seq[row];
-  if (seq < 0) return;                             // padding row
-  const int G = nq / nkv;
-  const int t = threadIdx.x, wave = t / EI_WAVE, lane = t % EI_WAVE;
+  const int t = threadIdx.x, lane = t % EI_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(t / EI_WAVE);
   const int r16 = lane & 15, c = lane >> 4;
-  const int pos = row_pos[row];
+  // The kernel is a chain of trips to memory, so each asks for all it can: (1) the row's sequence and
+  // position, and the projection or the queries; (2) the page of the wave's first tile, the angles;
+  // (3) that tile's keys and values, which travel while the heads are normed and rotated (the empty
+  // asm statements keep loads ahead of the branches that their uses stand behind; none is under a
+  // condition, since the waits after it would then be for all that is on its way).  A padding row
+  // goes along as position 0 of sequence 0 and writes nothing.  Beside the trips it is bound by the
+  // instructions that the waves of a block issue: a wave without a head or a tile skips them, and the
+  // divisions by the head counts are the host's.
+  // 16 heads, one sequence of 24 to 55 tokens: 6.7 -> 6.1 us, of which 1.6 are the launch; long walks
+  // (8 sequences of 270 tokens, 32 of up to 2,064) take what they did.
+  const int named = row_seq[row], placed = row_pos[row];
+  const int most_tokens = *longest;                // (not looked at where shares are equal)
+  if constexpr (PREP)                              // (the arguments that do not come with the launch,
+    // all of them on the same trip as the two above)
+    asm volatile("" ::"s"(prep.qkv), "s"(prep.nsplit), "s"(prep.split_stride), "s"(prep.q_norm_w),
+                 "s"(prep.k_norm_w), "s"(prep.eps), "s"(prep.rope_table), "s"(prep.rot_dim),
+                 "s"(prep.k_store), "s"(prep.v_store), "s"(nq), "s"(nkv), "s"(G), "s"(head_blocks),
+                 "s"(head_blocks_inv), "s"(window),
+                 "s"(scale), "s"(n_splits), "s"(equal_shares), "s"(out), "s"(named), "s"(placed),
+                 "s"(most_tokens));
+  __builtin_amdgcn_sched_barrier(0);
+  // (the quotient of two numbers below 2^16: the rounding of the float product is far less than half
+  // a step of it)
+  const int g = static_cast<int>((static_cast<float>(blockIdx.y) + 0.5f) * head_blocks_inv);
+  const int hb = blockIdx.y - g * head_blocks, split = blockIdx.z;
   const int head0 = g * G + hb * GB;               // first query head of this block
   const int heads_here = min(GB, G - hb * GB);
+  const bool padding = named < 0;
+  const int seq = padding ? 0 : named, pos = padding ? 0 : placed;
 
   // PREP: rows 0..GB-1 the block's query heads, row GB the new key, row GB+1 the new value,
-  // normed, rotated and rounded.  A wave takes a head at a time, a lane the pair (i, i + D/2):
-  // every load of a head is on its way before the first is used, and nothing but the final
-  // rows goes through LDS.
+  // normed, rotated and rounded.  A wave takes a head at a time, a lane the pair (i, i + D/2);
+  // nothing but the final rows goes through LDS.
   constexpr int PR = PREP ? GB + 2 : 1, FS = PREP ? D + 8 : 8;
   __shared__ __attribute__((aligned(16))) bf16_t fin_lds[PR][FS];
   const bool own_key = PREP && prep.k_store != nullptr;
-  if constexpr (PREP) {
-    constexpr int half = D / 2;
-    static_assert(half <= EI_WAVE, "a lane holds one pair");
-    const size_t width = static_cast<size_t>(nq + 2 * nkv) * D;
-    const float* src = prep.qkv + static_cast<size_t>(row) * width;
-    const int page_now = own_key
-        ? page_table[static_cast<size_t>(seq) * table_width + pos / EI_PAGE] : -1;
-    const bool active = lane < half;
-    // the lane's pair: elements (i, i2), rotated if it lies within the rotated width
-    const int rhalf = prep.rope_table != nullptr ? prep.rot_dim / 2 : half;
-    const int pair = active ? lane : 0;
-    const bool turned = pair < rhalf;
-    const int i = turned ? pair : pair + rhalf;
-    const int i2 = turned ? pair + rhalf : pair + half;
-    for (int h = wave; h < heads_here + (own_key ? 2 : 0); h += W) {
-      const int kind = h < heads_here ? 0 : (h == heads_here ? 1 : 2);   // query, key, value
-      const int slot = kind == 0 ? h : GB + kind - 1;
-      const int column = kind == 0 ? (head0 + h) * D
-                                   : (kind == 1 ? (nq + g) * D : (nq + nkv + g) * D);
-      const float* norm_w = kind == 0 ? prep.q_norm_w : (kind == 1 ? prep.k_norm_w : nullptr);
-      const bool rotate = kind != 2 && prep.rope_table != nullptr && turned;
-      float wx = 1.f, wy = 1.f, cs = 1.f, sn = 0.f;
-      if (norm_w != nullptr) {
-        wx = norm_w[i];
-        wy = norm_w[i2];
-      }
-      if (rotate) {
-        const float* trig = prep.rope_table + static_cast<size_t>(pos) * (2 * rhalf);
-        cs = trig[pair];
-        sn = trig[pair + rhalf];
-      }
-      float x = 0.f, y = 0.f;
-      const float* p = src + column;
-      for (int s0 = 0; s0 < prep.nsplit; s0 += 8) {       // slices in slice order, 8 per trip
-        float xa[8], ya[8];
+  constexpr int half = D / 2;
+  static_assert(half <= EI_WAVE, "a lane holds one pair");
+  constexpr int kAsked = 4;                        // slices of the first head asked for at once
+  const bool active = lane < half;
+  const int prep_heads = heads_here + (own_key ? 2 : 0);
+  // the lane's pair: elements (i, i2), rotated if it lies within the rotated width
+  const int rhalf = PREP && prep.rope_table != nullptr ? prep.rot_dim / 2 : half;
+  const int pair = active ? lane : 0;
+  const bool turned = pair < rhalf;
+  const int i1 = turned ? pair : pair + rhalf;
+  const int i2 = turned ? pair + rhalf : pair + half;
+  const float* prep_src = PREP ? prep.qkv + static_cast<size_t>(row) * (static_cast<size_t>(nq + 2 * nkv) * D) : nullptr;
+  auto kind_of = [&](int h) { return h < heads_here ? 0 : (h == heads_here ? 1 : 2); };   // query, key, value
+  auto column_of = [&](int h) {
+    const int kind = kind_of(h);
+    return kind == 0 ? (head0 + h) * D : (kind == 1 ? (nq + g) * D : (nq + nkv + g) * D);
+  };
+  auto norm_of = [&](int h) {
+    const int kind = kind_of(h);
+    return kind == 0 ? prep.q_norm_w : (kind == 1 ? prep.k_norm_w : nullptr);
+  };
+  float xa[kAsked], ya[kAsked], wx = 1.f, wy = 1.f, cs = 1.f, sn = 0.f;
+  auto ask_head = [&](int h) {
+    const float* p = prep_src + column_of(h);
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (s0 + u < prep.nsplit) {
-            xa[u] = p[(s0 + u) * prep.split_stride + i];
-            ya[u] = p[(s0 + u) * prep.split_stride + i2];
-          }
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-          if (s0 + u < prep.nsplit) {
-            x += xa[u];
-            y += ya[u];
-          }
-      }
-      if (!active) x = y = 0.f;
-      float a = x, b = y;
-      if (norm_w != nullptr) {
-        const float sum = ei::wave_sum(x * x + y * y);
-        const float inv = rsqrtf(sum / static_cast<float>(D) + prep.eps);
-        a = (a * inv) * wx;
-        b = (b * inv) * wy;
-      }
-      if (rotate) {
-        const float ra = a * cs - b * sn;
-        const float rb = a * sn + b * cs;
-        a = ra;
-        b = rb;
-      }
-      if (active) {
-        const bf16_t a16 = ei::from_f32<bf16_t>(a), b16 = ei::from_f32<bf16_t>(b);
-        fin_lds[slot][i] = a16;
-        fin_lds[slot][i2] = b16;
-        if (kind != 0 && hb == 0 && split == 0 && page_now >= 0) {
-          bf16_t* dst = (kind == 1 ? prep.k_store : prep.v_store) +
-                        ((static_cast<size_t>(page_now) * nkv + g) * EI_PAGE + pos % EI_PAGE) * D;
-          dst[i] = a16;
-          dst[i2] = b16;
-        }
-      }
+    for (int u = 0; u < kAsked; ++u) {
+      const float* slice = p + min(u, prep.nsplit - 1) * prep.split_stride;
+      xa[u] = slice[static_cast<unsigned>(i1)];
+      ya[u] = slice[static_cast<unsigned>(i2)];
     }
-    __syncthreads();
-  }
-
-  // query heads as the B operand: lane (n = r16, c) holds q[head n][j*32 + c*8 .. +8]
-  bf16x8 q_reg[DJ];
+    const float* norm_w = norm_of(h);              // (null: anything readable)
+    const float* from = norm_w != nullptr ? norm_w : p;
+    wx = from[static_cast<unsigned>(i1)];
+    wy = from[static_cast<unsigned>(i2)];
+  };
+  if constexpr (PREP) ask_head(min(wave, prep_heads - 1));
+  bf16x8 q_reg[DJ];                                // (without PREP) as below
+  if constexpr (!PREP) {
 #pragma unroll
-  for (int j = 0; j < DJ; ++j) {
-    uint4 z = uint4{0u, 0u, 0u, 0u};
-    if (r16 < heads_here) {
-      if constexpr (PREP)
-        z = *reinterpret_cast<const uint4*>(&fin_lds[r16][j * 32 + c * 8]);
-      else
-        z = *reinterpret_cast<const uint4*>(q + (static_cast<size_t>(row) * nq + head0 + r16) * D +
-                                            j * 32 + c * 8);
-    }
-    q_reg[j] = *reinterpret_cast<bf16x8*>(&z);
+    for (int j = 0; j < DJ; ++j)
+      q_reg[j] = *reinterpret_cast<const bf16x8*>(
+          q + (static_cast<size_t>(row) * nq + head0 + min(r16, heads_here - 1)) * D + j * 32 + c * 8);
   }
+  asm volatile("" ::: "memory");
 
   int lo_key_of = window > 0 ? max(0, pos - window + 1) : 0;
   if constexpr (OPT)
@@ -260,9 +234,10 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pa
   // step follows it).  Sequences of unequal lengths then give blocks of about equal work, and
   // the later slices of a short sequence are empty.  Without it (or with a window, where the
   // ranges start at different pages) every sequence is cut into n_splits equal parts.
-  int per = (pages + n_splits - 1) / n_splits;
-  if (longest != nullptr && window <= 0 && !(OPT && extra.chunk > 0)) {
-    const int most_pages = (*longest + EI_PAGE - 1) / EI_PAGE;
+  int per = pages;
+  if (n_splits > 1) {                              // (a division is 20 instructions)
+    const bool by_longest = !equal_shares && window <= 0 && !(OPT && extra.chunk > 0);
+    const int most_pages = by_longest ? (most_tokens + EI_PAGE - 1) / EI_PAGE : pages;
     per = max(1, (most_pages + n_splits - 1) / n_splits);
   }
   const int tile_begin = max(first_tile, (lo_page + split * per) * (EI_PAGE / kTile));
@@ -287,6 +262,131 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pa
   }
   (void)total_tiles;
 
+  // (2), (3) the wave's first tile of 16 keys; its page is looked up with the position's own
+  const int32_t* pages_of_seq = page_table + static_cast<size_t>(seq) * table_width;
+  auto tile_of = [&](int step) { return step < kept ? step : step + skipped; };
+  // (a step that the wave does not have: some tile of the sequence)
+  auto page_of = [&](int step) { return pages_of_seq[min(max(tile_of(step), 0), last_tile) / (EI_PAGE / kTile)]; };
+  int step = step_begin + wave;
+  int phys = page_of(step);
+  const int page_now = pages_of_seq[pos / EI_PAGE];
+  if constexpr (PREP) {
+    const float* trig = prep.rope_table != nullptr ? prep.rope_table + static_cast<size_t>(pos) * (2 * rhalf)
+                                                   : prep_src;
+    const unsigned at = turned ? pair : 0;
+    cs = trig[at];
+    sn = trig[at + rhalf];
+  }
+  const int ks = lane / LPR, dc = lane % LPR;       // value rows: key sub-index, 8-wide chunk
+  // keys: A operand, lane (key r16, c) holds k[key][j*32 + c*8 .. +8];
+  // values: lane (ks, dc) holds v[key0 + i*KPI + ks][dc*8 .. +8]
+  bf16x8 k_reg[DJ];
+  u32x4_t v_reg[VI];
+  auto place_of = [&](int page, int tile) {
+    return (static_cast<size_t>(max(page, 0)) * nkv + g) * EI_PAGE * D +
+           static_cast<size_t>(tile * kTile % EI_PAGE) * D;
+  };
+  // (all lanes of a wave without a tile ask for one place: a line and not eight kilobytes)
+  const unsigned k_lane = step < step_end ? r16 * D + c * 8 : 0;
+  const unsigned v_lane = step < step_end ? ks * D + dc * 8 : 0;
+  auto load_keys = [&](int page, int tile) {
+    const bf16_t* kp = k_pages + place_of(page, tile) + k_lane;
+#pragma unroll
+    for (int j = 0; j < DJ; ++j) k_reg[j] = *reinterpret_cast<const bf16x8*>(kp + j * 32);
+  };
+  auto load_values = [&](int page, int tile) {
+    // read once and whole lines at a time: not kept in the caches (the keys above are
+    // fetched in 64-byte pieces, two instructions a line, and do better cached)
+    const bf16_t* vp = v_pages + place_of(page, tile) + v_lane;
+#pragma unroll
+    for (int i = 0; i < VI; ++i)
+      v_reg[i] = __builtin_nontemporal_load(
+          reinterpret_cast<const u32x4_t*>(vp + static_cast<size_t>(i) * KPI * D));
+  };
+  {
+    const int tile = min(max(tile_of(step), 0), last_tile);
+    load_keys(phys, tile);
+    load_values(phys, tile);
+  }
+  asm volatile("" ::: "memory");
+
+  if constexpr (PREP) {
+    for (int h = wave; h < prep_heads; h += W) {
+      const int kind = kind_of(h);
+      const int slot = kind == 0 ? h : GB + kind - 1;
+      const float* norm_w = norm_of(h);
+      const bool rotate = kind != 2 && prep.rope_table != nullptr && turned;
+      const float* p = prep_src + column_of(h);
+      if (h != wave) ask_head(h);
+      float x = 0.f, y = 0.f;                      // slices in slice order
+#pragma unroll
+      for (int u = 0; u < kAsked; ++u)
+        if (u < prep.nsplit) {
+          x += xa[u];
+          y += ya[u];
+        }
+      for (int s0 = kAsked; s0 < prep.nsplit; s0 += kAsked) {
+        float xb[kAsked], yb[kAsked];
+#pragma unroll
+        for (int u = 0; u < kAsked; ++u) {
+          const float* slice = p + min(s0 + u, prep.nsplit - 1) * prep.split_stride;
+          xb[u] = slice[static_cast<unsigned>(i1)];
+          yb[u] = slice[static_cast<unsigned>(i2)];
+        }
+#pragma unroll
+        for (int u = 0; u < kAsked; ++u)
+          if (s0 + u < prep.nsplit) {
+            x += xb[u];
+            y += yb[u];
+          }
+      }
+      if (!active) x = y = 0.f;
+      float a = x, b = y;
+      if (norm_w != nullptr) {
+        const float sum = ei::wave_sum(x * x + y * y);
+        const float inv = rsqrtf(sum / static_cast<float>(D) + prep.eps);
+        a = (a * inv) * wx;
+        b = (b * inv) * wy;
+      }
+      if (rotate) {
+        const float ra = a * cs - b * sn;
+        const float rb = a * sn + b * cs;
+        a = ra;
+        b = rb;
+      }
+      if (active) {
+        const bf16_t a16 = ei::from_f32<bf16_t>(a), b16 = ei::from_f32<bf16_t>(b);
+        fin_lds[slot][i1] = a16;
+        fin_lds[slot][i2] = b16;
+        if (kind != 0 && hb == 0 && split == 0 && page_now >= 0 && !padding) {
+          bf16_t* dst = (kind == 1 ? prep.k_store : prep.v_store) +
+                        ((static_cast<size_t>(page_now) * nkv + g) * EI_PAGE + pos % EI_PAGE) * D;
+          dst[i1] = a16;
+          dst[i2] = b16;
+        }
+      }
+    }
+    // (a plain barrier after the wave's own LDS writes: __syncthreads would wait for the tile too)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);            // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+  }
+
+  // query heads as the B operand: lane (n = r16, c) holds q[head n][j*32 + c*8 .. +8]
+#pragma unroll
+  for (int j = 0; j < DJ; ++j) {
+    uint4 z = uint4{0u, 0u, 0u, 0u};
+    if constexpr (PREP) {
+      if (r16 < heads_here) z = *reinterpret_cast<const uint4*>(&fin_lds[r16][j * 32 + c * 8]);
+    } else {
+      if (r16 < heads_here) z = *reinterpret_cast<const uint4*>(&q_reg[j]);
+    }
+    q_reg[j] = *reinterpret_cast<bf16x8*>(&z);
+  }
+
   // (KEPT) the gate of the first element that this thread will write, asked for ahead of the walk
   const size_t wide_base = KEPT ? static_cast<size_t>(row) * extra.wide_row +
                                      static_cast<size_t>(head0) * D : 0;
@@ -303,47 +403,21 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pa
   for (int h = 0; h < GB; ++h)
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
-  const int ks = lane / LPR, dc = lane % LPR;       // value rows: key sub-index, 8-wide chunk
 
-  // One tile of 16 keys.  OWN: the tile holds the position itself and the block has made its
-  // key and value (PREP): they come from LDS.  That case has code of its own, so that in
-  // every other tile the score product waits for the keys alone and not for a patch.
-  auto process = [&](const int tile, auto own_tag) {
-    constexpr bool OWN = decltype(own_tag)::value;
+  // One tile of 16 keys, whose keys and values are in registers or on their way.
+  auto process = [&](const int tile) {
     const int key0 = tile * kTile;
-    const int phys = page_table[static_cast<size_t>(seq) * table_width + key0 / EI_PAGE];
-    if (phys < 0) return;                          // released by the window: all masked
-    const size_t page_base = (static_cast<size_t>(phys) * nkv + g) * EI_PAGE * D;
-    const int in_page = key0 % EI_PAGE;
-    // keys: A operand, lane (key r16, c) holds k[key][j*32 + c*8 .. +8]
-    bf16x8 k_reg[DJ];
-    const bf16_t* kp = k_pages + page_base + static_cast<size_t>(in_page + r16) * D + c * 8;
-#pragma unroll
-    for (int j = 0; j < DJ; ++j) k_reg[j] = *reinterpret_cast<const bf16x8*>(kp + j * 32);
-    // values: lane (ks, dc) holds v[key0 + i*KPI + ks][dc*8 .. +8]
-    uint4 v_reg[VI];
-    const bf16_t* vp = v_pages + page_base + static_cast<size_t>(in_page + ks) * D + dc * 8;
-#pragma unroll
-    for (int i = 0; i < VI; ++i)
-    {
-      // read once and whole lines at a time: not kept in the caches (the keys above are
-      // fetched in 64-byte pieces, two instructions a line, and do better cached)
-      const u32x4_t raw = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x4_t*>(vp + static_cast<size_t>(i) * KPI * D));
-      v_reg[i] = uint4{raw.x, raw.y, raw.z, raw.w};
-    }
-    if constexpr (OWN) {                           // the position's own key and value
+    if (PREP && own_key && tile == last_tile) {    // the position's own key and value, from LDS
       if (key0 + r16 == pos) {
 #pragma unroll
         for (int j = 0; j < DJ; ++j)
-          k_reg[j] = *reinterpret_cast<const bf16x8*>(&fin_lds[GB][j * 32 + c * 8]);
+          k_reg[j] = *reinterpret_cast<const bf16x8*>(&fin_lds[PREP ? GB : 0][j * 32 + c * 8]);
       }
 #pragma unroll
       for (int i = 0; i < VI; ++i)
         if (key0 + i * KPI + ks == pos)
-          v_reg[i] = *reinterpret_cast<const uint4*>(&fin_lds[GB + 1][dc * 8]);
+          v_reg[i] = *reinterpret_cast<const u32x4_t*>(&fin_lds[PREP ? GB + 1 : 0][dc * 8]);
     }
-
     f32x4 s = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < DJ; ++j)
@@ -391,7 +465,7 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pa
     for (int i = 0; i < VI; ++i) {
       const int key_local = i * KPI + ks;
       const bool live = key0 + key_local <= pos;    // later slots hold stale bytes
-      const uint4 raw = live ? v_reg[i] : uint4{0u, 0u, 0u, 0u};
+      const u32x4_t raw = live ? v_reg[i] : u32x4_t{0u, 0u, 0u, 0u};
       float v[8];
       v[0] = bf16_lo(raw.x); v[1] = bf16_hi(raw.x); v[2] = bf16_lo(raw.y); v[3] = bf16_hi(raw.y);
       v[4] = bf16_lo(raw.z); v[5] = bf16_hi(raw.z); v[6] = bf16_lo(raw.w); v[7] = bf16_hi(raw.w);
@@ -405,47 +479,68 @@ attn_decode_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pa
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
-  for (int step = step_begin + wave; step < step_end; step += W) {
-    const int tile = step < kept ? step : step + skipped;
-    if (PREP && own_key && tile == last_tile)
-      process(tile, std::integral_constant<bool, PREP>{});
-    else
-      process(tile, std::false_type{});
+  if (step < step_end) {
+    int phys_next = page_of(step + W);
+    if (phys >= 0) process(tile_of(step));         // (below 0: released by the window, all masked)
+    for (step += W; step < step_end; step += W) {
+      const int tile = tile_of(step);
+      phys = phys_next;
+      if (phys >= 0) {
+        load_keys(phys, tile);
+        load_values(phys, tile);
+      }
+      phys_next = page_of(step + W);
+      if (phys >= 0) process(tile);
+    }
   }
 
-  // sum the partial outputs of the KPI key sub-groups inside the wave
-#pragma unroll
-  for (int h = 0; h < GB; ++h)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float x = acc[h][e];
-#pragma unroll
-      for (int offset = LPR; offset < EI_WAVE; offset <<= 1) x += __shfl_xor(x, offset, EI_WAVE);
-      acc[h][e] = x;
-    }
-  if (c == 0) {
-    m_lds[wave][r16] = m_run;
-    l_lds[wave][r16] = l_run;
-  }
-  if (ks == 0) {
+  const int live_waves = max(0, min(W, step_end - step_begin));      // waves that had a tile
+  if (wave < live_waves) {
+    // sum the partial outputs of the KPI key sub-groups inside the wave
 #pragma unroll
     for (int h = 0; h < GB; ++h)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) o_lds[wave][h][dc * 8 + e] = acc[h][e];
+      for (int e = 0; e < 8; ++e) {
+        float x = acc[h][e];
+#pragma unroll
+        for (int offset = LPR; offset < EI_WAVE; offset <<= 1) x += __shfl_xor(x, offset, EI_WAVE);
+        acc[h][e] = x;
+      }
+    if (c == 0) {
+      m_lds[wave][r16] = m_run;
+      l_lds[wave][r16] = l_run;
+    }
+    if (ks == 0) {
+#pragma unroll
+      for (int h = 0; h < GB; ++h)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o_lds[wave][h][dc * 8 + e] = acc[h][e];
+    }
   }
   __syncthreads();
-  // merge the four waves: thread -> (head, d), strided
+  if (padding) return;
+  // merge the waves: thread -> (head, d), strided
   for (int idx = t; idx < heads_here * D; idx += (W * EI_WAVE)) {
     const int h = idx / D, d = idx % D;
-    float m = kLowest;
+    float m = kLowest, l = 0.f, o = 0.f;
+    if (live_waves == W) {
 #pragma unroll
-    for (int w = 0; w < W; ++w) m = fmaxf(m, m_lds[w][h]);
-    float l = 0.f, o = 0.f;
+      for (int w = 0; w < W; ++w) m = fmaxf(m, m_lds[w][h]);
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      const float f = expf(m_lds[w][h] - m);
-      l += l_lds[w][h] * f;
-      o += o_lds[w][h][d] * f;
+      for (int w = 0; w < W; ++w) {
+        const float f = expf(m_lds[w][h] - m);
+        l += l_lds[w][h] * f;
+        o += o_lds[w][h][d] * f;
+      }
+    } else {
+#pragma unroll 4
+      for (int w = 0; w < live_waves; ++w) m = fmaxf(m, m_lds[w][h]);
+#pragma unroll 4
+      for (int w = 0; w < live_waves; ++w) {
+        const float f = expf(m_lds[w][h] - m);
+        l += l_lds[w][h] * f;
+        o += o_lds[w][h][d] * f;
+      }
     }
     const int head = head0 + h;
     if constexpr (OPT) {
@@ -1195,22 +1290,25 @@ void launch_decode(dim3 grid, hipStream_t stream, const bf16_t* q, const bf16_t*
   if constexpr (GB <= 4) {               // the caller gives 16 waves at most 4 heads a block
     if (waves == 16) {
       attn_decode_kernel<D, GB, 16, PREP, EXT><<<grid, 16 * EI_WAVE, 0, stream>>>(
-          q, k, v, row_pos, row_seq, page_table, table_width, out, part_o, part_ml, nq, nkv,
-          head_blocks, window, scale, n_splits, longest, prep, extra);
+          row_pos, row_seq, page_table, longest ? longest : row_pos, k, v, table_width, q, out, part_o,
+          part_ml, nq, nkv, nq / nkv, head_blocks, 1.0f / static_cast<float>(head_blocks), window, scale,
+          n_splits, longest ? 0 : 1, prep, extra);
       return;
     }
   }
   if constexpr (GB <= 8) {               // and 8 waves at most 8
     if (waves == 8) {
       attn_decode_kernel<D, GB, 8, PREP, EXT><<<grid, 8 * EI_WAVE, 0, stream>>>(
-          q, k, v, row_pos, row_seq, page_table, table_width, out, part_o, part_ml, nq, nkv,
-          head_blocks, window, scale, n_splits, longest, prep, extra);
+          row_pos, row_seq, page_table, longest ? longest : row_pos, k, v, table_width, q, out, part_o,
+          part_ml, nq, nkv, nq / nkv, head_blocks, 1.0f / static_cast<float>(head_blocks), window, scale,
+          n_splits, longest ? 0 : 1, prep, extra);
       return;
     }
   }
   attn_decode_kernel<D, GB, 4, PREP, EXT><<<grid, 4 * EI_WAVE, 0, stream>>>(
-        q, k, v, row_pos, row_seq, page_table, table_width, out, part_o, part_ml, nq, nkv,
-        head_blocks, window, scale, n_splits, longest, prep, extra);
+        row_pos, row_seq, page_table, longest ? longest : row_pos, k, v, table_width, q, out, part_o,
+        part_ml, nq, nkv, nq / nkv, head_blocks, 1.0f / static_cast<float>(head_blocks), window, scale,
+          n_splits, longest ? 0 : 1, prep, extra);
 }
 
 }  // namespace
