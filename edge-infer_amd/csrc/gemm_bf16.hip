@@ -60,7 +60,7 @@ __global__ void __launch_bounds__(WAVES * EI_WAVE)
 skinny_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X,
                    float* __restrict__ out, bf16_t* __restrict__ gated_out, int M, int N, int K,
                    int k_per_split, int row_groups, ei::GateAct act,
-                   const float* __restrict__ bias, const float* __restrict__ stats, float eps) {
+                   const float* __restrict__ bias, const float* __restrict__ stats, int parts, float eps) {
   constexpr bool GATED = END == kGated || END == kGatedBias;
   constexpr int JN = KT / 32;             // MFMA steps per K-tile
   static_assert(KT == 256 || (KT == 128 && PACKED), "K-tiles of 256, or 128 with packed weights");
@@ -109,7 +109,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X,
 
   static_assert(!STATS || (PACKED && STRIPS == 1 && MB == 1 && END == kSums), "see ei::RowNorm");
   ei::RowFactors<1> factors;
-  if constexpr (STATS) factors.ask(stats, M, K, t);
+  if constexpr (STATS) factors.ask(stats, M, parts, t);
 
   f32x4 acc[MB][STRIPS];
 #pragma unroll
@@ -357,7 +357,7 @@ skinny_gemm_kernel(const bf16_t* __restrict__ W, const bf16_t* __restrict__ X,
 
   if constexpr (STATS) {
     __shared__ float factor[16];
-    factors.finish(factor, K, eps, t);
+    factors.finish(factor, parts, K, eps, t);
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 4; ++r) acc[0][0][r] *= factor[r16];
@@ -564,19 +564,19 @@ void launch_tile_kernel(const bf16_t* w, const bf16_t* x, float* out, bf16_t* ga
   dim3 grid(strip_blocks * row_groups, splits);
   if (waves == 4)
     skinny_gemm_kernel<MB, 4, PACKED, END, STRIPS, KT, STATS><<<grid, 4 * EI_WAVE, 0, stream>>>(
-        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias, rs.squares, rs.eps);
+        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias, rs.squares, rs.parts, rs.eps);
   else if (waves == 6)
     skinny_gemm_kernel<MB, 6, PACKED, END, STRIPS, KT, STATS><<<grid, 6 * EI_WAVE, 0, stream>>>(
-        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias, rs.squares, rs.eps);
+        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias, rs.squares, rs.parts, rs.eps);
   else
     skinny_gemm_kernel<MB, 8, PACKED, END, STRIPS, KT, STATS><<<grid, 8 * EI_WAVE, 0, stream>>>(
-        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias, rs.squares, rs.eps);
+        w, x, out, gated_out, M, N, K, k_per_split, row_groups, act, bias, rs.squares, rs.parts, rs.eps);
 }
 
 template <bool PACKED, int END>
 int launch_skinny(const void* X, const void* W, float* out, void* gated_out, int M, int N, int K,
                   int splits, hipStream_t stream, const ei::GateAct& act = ei::GateAct{0, 0.f, 1.f},
-                  const float* bias = nullptr, const ei::RowNorm& rs = ei::RowNorm{nullptr, 0.f}) {
+                  const float* bias = nullptr, const ei::RowNorm& rs = ei::RowNorm{nullptr, 0, 0.f}) {
   EI_REQUIRE(act.kind >= 0 && act.kind <= (END == kPlain ? 3 : 2),
              "gemm_bf16_skinny_gated: unknown activation");
   EI_REQUIRE(M >= 1 && M <= kMaxRows, "gemm_bf16_skinny: rows must lie in 1..256");
@@ -602,7 +602,8 @@ int launch_skinny(const void* X, const void* W, float* out, void* gated_out, int
   const bf16_t* w = static_cast<const bf16_t*>(W);
   bf16_t* g = static_cast<bf16_t*>(gated_out);
   EI_REQUIRE(!rs.squares || (PACKED && (END == kSums || END == kGated) && M <= ei::kWholeRows && K % 64 == 0 &&
-                             K <= ei::kStatsWidth && rs.eps > 0.f &&
+                             K <= ei::kStatsWidth && (rs.parts == K / 16 || rs.parts == K / 8) &&
+                             rs.parts <= ei::kStatsParts && rs.eps > 0.f &&
                              (reinterpret_cast<uintptr_t>(rs.squares) & 15) == 0),
              "gemm_bf16_skinny: a norm is finished for at most 16 rows of at most 4096 columns, a multiple of 64");
   if constexpr (PACKED && (END == kGated || END == kGatedBias || END == kPlain)) {
@@ -611,12 +612,12 @@ int launch_skinny(const void* X, const void* W, float* out, void* gated_out, int
       constexpr int how = END == kPlain ? ei::kActivatedRows : ei::kGatedRows;
       if (rs.squares) {
         if constexpr (END == kGated)
-          ei::launch_whole_product<how, true, false>(w, x, M, N, K, nullptr, nullptr, g, const_cast<float*>(rs.squares), rs.eps, act, stream);
+          ei::launch_whole_product<how, true, false>(w, x, M, N, K, nullptr, nullptr, g, const_cast<float*>(rs.squares), rs.parts, rs.eps, act, stream);
       } else if (END != kGated && bias) {
         if constexpr (END != kGated)
-          ei::launch_whole_product<how, false, true>(w, x, M, N, K, nullptr, bias, g, nullptr, 0.f, act, stream);
+          ei::launch_whole_product<how, false, true>(w, x, M, N, K, nullptr, bias, g, nullptr, 0, 0.f, act, stream);
       } else {
-        ei::launch_whole_product<how, false, false>(w, x, M, N, K, nullptr, nullptr, g, nullptr, 0.f, act, stream);
+        ei::launch_whole_product<how, false, false>(w, x, M, N, K, nullptr, nullptr, g, nullptr, 0, 0.f, act, stream);
       }
       EI_LAUNCH_CHECK();
     }
@@ -666,10 +667,10 @@ extern "C" int ei_gemm_bf16_skinny(const void* X, const void* W, float* out, int
 // memory channel busy; rows of W that are 2^n bytes apart do not.
 // `stats` (or null): the rows of X still have to be divided by their root mean square, see ei::RowNorm.
 extern "C" int ei_gemm_bf16_skinny_packed(const void* X, const void* Wp, float* out, int M, int N,
-                                          int K, int splits, const float* stats, float eps,
+                                          int K, int splits, const float* stats, int parts, float eps,
                                           hipStream_t stream) {
   return launch_skinny<true, kSums>(X, Wp, out, nullptr, M, N, K, splits, stream,
-                                    ei::GateAct{0, 0.f, 1.f}, nullptr, ei::RowNorm{stats, eps});
+                                    ei::GateAct{0, 0.f, 1.f}, nullptr, ei::RowNorm{stats, parts, eps});
 }
 
 // Gated feed-forward in one pass: W [N, K] holds, in strips of 16 rows, the gate rows of 16
@@ -679,7 +680,7 @@ extern "C" int ei_gemm_bf16_skinny_packed(const void* X, const void* Wp, float* 
 // of K in one slice.  `packed`: W is in the streaming layout of ei_gemm_bf16_skinny_packed.
 extern "C" int ei_gemm_bf16_skinny_gated(const void* X, const void* W, void* act, int M, int N,
                                          int K, int packed, int kind, float limit, float alpha,
-                                         const float* bias, const float* stats, float eps,
+                                         const float* bias, const float* stats, int parts, float eps,
                                          hipStream_t stream) {
   const ei::GateAct how{kind, limit, alpha};
   EI_REQUIRE(!stats || (packed && !bias), "gemm_bf16_skinny_gated: sums of squares go with packed weights and no bias");
@@ -687,7 +688,7 @@ extern "C" int ei_gemm_bf16_skinny_gated(const void* X, const void* W, void* act
     return launch_skinny<true, kGatedBias>(X, W, nullptr, act, M, N, K, 1, stream, how, bias);
   if (packed)
     return launch_skinny<true, kGated>(X, W, nullptr, act, M, N, K, 1, stream, how, nullptr,
-                                       ei::RowNorm{stats, eps});
+                                       ei::RowNorm{stats, parts, eps});
   if (bias)
     return launch_skinny<false, kGatedBias>(X, W, nullptr, act, M, N, K, 1, stream, how, bias);
   return launch_skinny<false, kGated>(X, W, nullptr, act, M, N, K, 1, stream, how);
@@ -703,20 +704,24 @@ extern "C" int ei_gemm_bf16_skinny_act(const void* X, const void* W, void* out, 
 }
 
 // residual [M, N] float32 += X [M, K] bfloat16 . W^T in place, for at most 16 rows and W in the
-// streaming layout; rows [M, N] bfloat16 and squares [M, N / 16] float32 are what a norm of the
+// streaming layout; rows [M, N] bfloat16 and squares [M, parts] float32, parts N / 16 or, for at
+// most 8 rows and an N of at most 2048, N / 8, are what a norm of the
 // residual with this weight (float32 [N]) leaves to the products that read it (ei::kAddRows).
 extern "C" int ei_gemm_bf16_add(const void* X, const void* Wp, float* residual, const float* weight,
-                                void* rows, float* squares, int M, int N, int K, hipStream_t stream) {
+                                void* rows, float* squares, int parts, int M, int N, int K,
+                                hipStream_t stream) {
   EI_REQUIRE(X && Wp && residual && weight && rows && squares, "gemm_bf16_add: null pointer");
   EI_REQUIRE(M >= 1 && M <= ei::kWholeRows, "gemm_bf16_add: rows must lie in 1..16");
   EI_REQUIRE(N >= 16 && N % 16 == 0 && K >= 8 && K % 8 == 0,
              "gemm_bf16_add: N must be a multiple of 16, K of 8");
+  EI_REQUIRE(parts == N / 16 || (parts == N / 8 && M <= 8 && parts <= ei::kStatsParts),
+             "gemm_bf16_add: a sum of squares for 16 columns or, for at most 8 rows of 2048, for 8");
   EI_REQUIRE(((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Wp) |
                reinterpret_cast<uintptr_t>(residual) | reinterpret_cast<uintptr_t>(weight) |
                reinterpret_cast<uintptr_t>(rows)) & 15) == 0,
              "gemm_bf16_add: pointers must be 16-byte aligned");
   ei::launch_whole_product<ei::kAddRows, false, false>(
       static_cast<const bf16_t*>(Wp), static_cast<const bf16_t*>(X), M, N, K, residual, weight,
-      static_cast<bf16_t*>(rows), squares, 0.f, ei::GateAct{0, 0.f, 1.f}, stream);
+      static_cast<bf16_t*>(rows), squares, parts, 0.f, ei::GateAct{0, 0.f, 1.f}, stream);
   EI_LAUNCH_CHECK();
 }

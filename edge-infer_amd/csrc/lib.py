@@ -253,11 +253,12 @@ _SIGNATURES = {
         "ei_gemm_bf16_skinny": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                 c_void_p],
         "ei_gemm_bf16_skinny_packed": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
-                                       c_void_p, c_float, c_void_p],
+                                       c_void_p, c_int, c_float, c_void_p],
         "ei_gemm_bf16_skinny_gated": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
-                                      c_int, c_float, c_float, c_void_p, c_void_p, c_float, c_void_p],
+                                      c_int, c_float, c_float, c_void_p, c_void_p, c_int, c_float,
+                                      c_void_p],
         "ei_gemm_bf16_add": [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
-                             c_int, c_void_p],
+                             c_int, c_int, c_void_p],
         "ei_gemm_bf16_skinny_act": [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                     c_int, c_void_p, c_void_p],
     },
@@ -2550,27 +2551,35 @@ WHOLE_ROWS = 16         # most rows of the products whose sums are whole inside 
 
 
 def _row_stats(stats, m: int, k: int, what: str):
-    """(pointer, eps) of `stats`: None, or (sums of squares [m, k / 16], eps) of rows x that still have
-    to be divided by their root mean square, see `gemm_bf16_add`."""
+    """(pointer, parts, eps) of `stats`: None, or (sums of squares [m, parts], eps) of rows x that still
+    have to be divided by their root mean square, see `gemm_bf16_add`."""
     if stats is None:
-        return None, 0.0
+        return None, 0, 0.0
     sums, eps = stats
-    if m > WHOLE_ROWS or k > STATS_WIDTH or k % 64 or tuple(sums.shape) != (m, k // 16):
+    if (m > WHOLE_ROWS or k > STATS_WIDTH or k % 64 or sums.dim() != 2 or sums.shape[0] != m
+            or sums.shape[1] not in (k // 16, k // 8) or sums.shape[1] > STATS_WIDTH // 16):
         raise KernelError(f"{what}: sums of squares {list(sums.shape)} do not belong to rows [{m}, {k}]")
-    return _gpu(sums, "stats", torch.float32), float(eps)
+    return _gpu(sums, "stats", torch.float32), sums.shape[1], float(eps)
+
+
+def add_parts(m: int, n: int) -> int:
+    """Sums of squares a row that `gemm_bf16_add` does best to leave for rows [m, n]: blocks of 8 columns
+    where blocks of 16 would leave half the chip idle and the rows allow it."""
+    return n // 8 if m <= 8 and n <= STATS_WIDTH // 2 else n // 16
 
 
 def gemm_bf16_add(x: torch.Tensor, packed: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                   rows: torch.Tensor, stats: torch.Tensor) -> None:
     """residual [m, n] (float32) += x . w^T for at most `WHOLE_ROWS` rows, with the weight given as
     `pack_weight(w)`; rows [m, n] = the new residual times `weight` [n], rounded to bfloat16, and
-    stats [m, n / 16] = the sums of the new residual's squares, 16 columns each: what the products
-    that read a norm of the residual need of it."""
+    stats [m, n / 16], or [m, n / 8] for at most 8 rows of at most 2048 (see `add_parts`), = the sums of
+    the new residual's squares, 16 or 8 columns each: what the products that read a norm of the
+    residual need of it."""
     lib = library("gemm_bf16")
     m, k = x.shape
     n = residual.shape[1]
     if (tuple(residual.shape) != (m, n) or tuple(rows.shape) != (m, n) or tuple(weight.shape) != (n,)
-            or n % 16 or tuple(stats.shape) != (m, n // 16)
+            or n % 16 or tuple(stats.shape) not in ((m, n // 16), (m, n // 8))
             or tuple(packed.shape) != (8 * ((k + 255) // 256), n // 16, 4, 16, 8)):
         raise KernelError(f"gemm_bf16_add: {list(x.shape)} x packed {list(packed.shape)} -> "
                           f"{list(residual.shape)}, {list(rows.shape)}, {list(stats.shape)} do not agree")
@@ -2578,7 +2587,7 @@ def gemm_bf16_add(x: torch.Tensor, packed: torch.Tensor, residual: torch.Tensor,
                                   _gpu(residual, "residual", torch.float32),
                                   _gpu(weight, "weight", torch.float32),
                                   _gpu(rows, "rows", torch.bfloat16),
-                                  _gpu(stats, "stats", torch.float32), m, n, k, _stream())
+                                  _gpu(stats, "stats", torch.float32), stats.shape[1], m, n, k, _stream())
     _check(lib, status, "gemm_bf16_add")
 
 

@@ -136,7 +136,8 @@ class Linear:
     def forward_add(self, ctx, x: torch.Tensor, to: AddTo) -> NormRows:
         """to.residual += x . W^T in place; returns the `NormRows` of `to.norm`."""
         rows = ctx.buffer(to.name, (x.shape[0], self.out_features), torch.bfloat16)
-        squares = ctx.buffer(to.name + ".squares", (x.shape[0], self.out_features // 16), torch.float32)
+        squares = ctx.buffer(to.name + ".squares",
+                             (x.shape[0], lib.add_parts(x.shape[0], self.out_features)), torch.float32)
         lib.gemm_bf16_add(x, self.packed, to.residual, to.norm.weight, rows, squares)
         return NormRows(rows, squares, to.norm.eps)
 

@@ -36,6 +36,35 @@ def test_add_product(m, n, k):
     assert torch.allclose(stats.cpu().to(F64), squares, rtol=16 * 2 * UNIT, atol=0.0)
 
 
+@pytest.mark.parametrize("m", [1, 3, 8])
+@pytest.mark.parametrize("n,k", [(64, 64), (1024, 1088), (1024, 2048), (16, 8), (1024, 3072), (2048, 3136),
+                                 (80, 4168), (2048, 8192)])
+def test_add_product_by_half_strips(m, n, k):
+    """Eight columns a block, and a product that finishes the norm from sums of eight columns."""
+    x, w = made((m, k), 1).to(BF16), made((n, k), 2, k ** -0.5).to(BF16)
+    residual, weight = made((m, n), 3), 1.0 + 0.1 * made((n,), 4)
+    dev = residual.cuda()
+    rows = torch.full((m, n), float("nan"), dtype=BF16, device="cuda")
+    stats = torch.full((m, n // 8), float("nan"), device="cuda")
+    assert lib.add_parts(m, n) == n // 8 and lib.add_parts(9, n) == n // 16 and lib.add_parts(m, 4096) == 256
+    lib.gemm_bf16_add(x.cuda(), lib.pack_weight(w.cuda()), dev, weight.cuda(), rows, stats)
+    exact = residual.to(F64) + x.to(F64) @ w.to(F64).t()
+    magnitude = residual.to(F64).abs() + x.to(F64).abs() @ w.to(F64).abs().t()
+    assert ((dev.cpu().to(F64) - exact).abs() <= (k + 2) * UNIT * magnitude).all()
+    assert torch.equal(rows.cpu(), (dev.cpu() * weight).to(BF16))
+    squares = dev.cpu().to(F64).square().view(m, n // 8, 8).sum(dim=2)
+    assert torch.allclose(stats.cpu().to(F64), squares, rtol=16 * UNIT, atol=0.0)
+    if n % 64:
+        return
+    reader = made((96, n), 7, n ** -0.5).to(BF16)
+    out = torch.empty((lib.skinny_gemm_splits(m, 96, n), m, 96), device="cuda")
+    lib.gemm_bf16_skinny_packed(rows, lib.pack_weight(reader.cuda()), 96, out, stats=(stats, 1e-6))
+    factor = (dev.cpu().to(F64).square().mean(dim=1, keepdim=True) + 1e-6).rsqrt()
+    want = (rows.cpu().to(F64) @ reader.to(F64).t()) * factor
+    bound = (2 * n + 8) * UNIT * (rows.cpu().to(F64).abs() @ reader.to(F64).abs().t()) * factor
+    assert ((out.cpu().to(F64).sum(dim=0) - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("m", [1, 5, 16])
 @pytest.mark.parametrize("n,k", [(64, 64), (96, 1024), (4096, 1024), (6144, 4096), (1600, 2048), (32, 448)])
 def test_products_finish_the_norm(m, n, k):
