@@ -10,18 +10,22 @@
 //
 // A block is four waves and up to 64 query rows (positions x heads of one kv group, 16 a
 // wave).  Keys come in tiles of 32 through LDS, as stored (a row a key, padded by 16 bytes),
-// the values of the tile transposed (a row a value element, 32 keys wide).  Scores are taken
+// and so do the values, where they are not the keys' own first elements.  Scores are taken
 // transposed, S^T = K Q^T with v_mfma_f32_16x16x32_bf16: the key tile is the A operand (lane
 // (key, c) reads 16 bytes of the key's row), the wave's query rows, held in registers for the
 // whole walk, the B operand; lane (c, n) then holds the scores of keys 4c .. 4c + 3 of either
 // half of the tile for query row n, which is, with the keys of a tile taken in the order
 // {4c .. 4c + 3, 16 + 4c .. 16 + 4c + 3}, exactly the B operand of O^T = V^T P^T; the A operand
-// of that product is two 8-byte reads of a row of the transposed values.  A lane's
+// of that product is two transposing reads of the rows as they lie (ds_read_b64_tr_b16; writing the
+// values transposed, two bytes at a time, took 2 of 16 us of a decode step's kernel, below).  A lane's
 // accumulators all belong to query row n, so the rescaling needs no exchange.
 #include "common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 namespace {
 
@@ -29,10 +33,14 @@ constexpr int kThreads = 256;
 constexpr int kRows = 64;         // query rows of a block
 constexpr int kKeys = 32;         // keys of a tile
 constexpr int kPadK = 8;          // elements of padding of a key row in LDS
-constexpr int kVtRow = kKeys + 8; // elements of a row of the transposed values in LDS
 constexpr float kLowest = -1.0e30f;
 
-template <int NK, int NDV>
+// SHARED (slices of the key range for at most 16 query rows a block, i.e. decoding): the four waves hold
+// the same query rows, take their scores each for itself and share the value elements out, where
+// otherwise one wave would do all of it.  A wave then holds a quarter of the sums, which leaves
+// registers for all of a tile's loads to travel together.  Keys of 576, values of 512, 16 heads, 64 keys a
+// block: 19.1 -> 16.1 us, and 14.0 with the transposing reads.
+template <int NK, int NDV, bool SHARED>
 __global__ void __launch_bounds__(kThreads)
 attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages,
                  const bf16_t* __restrict__ v_pages, const int32_t* __restrict__ item_seq,
@@ -47,8 +55,10 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
   const int DQ = KH * D;
   const int k_row = DQ + kPadK;                               // elements
   bf16_t* Kt = reinterpret_cast<bf16_t*>(lds_raw);            // [kKeys][k_row]
-  bf16_t* Vt = Kt + kKeys * k_row;                            // [DV][kVtRow]
-  const int nk = DQ / 32, ndv = DV / 16;
+  // the values of the tile, a row a key: the first elements of the keys' rows, or rows of their own
+  const int v_row = values_in_keys ? k_row : DV + kPadK;
+  bf16_t* Vs = values_in_keys ? Kt : Kt + kKeys * k_row;      // [kKeys][v_row]
+  const int nk = DQ / 32;
 
   const int item = blockIdx.x;
   const int g = blockIdx.y / head_blocks, hb = blockIdx.y % head_blocks;
@@ -59,9 +69,13 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
   const int row0 = item_row0[item];
   const int G = nq / nkv;
   const int t = threadIdx.x;
-  const int wave = t / EI_WAVE, lane = t % EI_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(t / EI_WAVE), lane = t % EI_WAVE;
   const int n = lane % 16, c = lane / 16;
-  const int rho = wave * 16 + n;                              // the block's query row
+  const int rho = SHARED ? n : wave * 16 + n;                 // the block's query row
+  // the wave's blocks of 16 value elements: d0 .. d0 + ND - 1, of which it has `nd`
+  constexpr int ND = SHARED ? (NDV + 3) / 4 : NDV;
+  const int d0 = SHARED ? wave * ND : 0;
+  const int nd = min(ND, DV / 16 - d0);
   const int pi = rho / HB, head_in_group = hb * HB + rho % HB;
   const bool valid = pi < npos && head_in_group < G;
   const int head = g * G + head_in_group;
@@ -81,9 +95,9 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
   }
 
   float m_run = kLowest, l_run = 0.f;
-  f32x4 acc[NDV];
+  f32x4 acc[ND];
 #pragma unroll
-  for (int d = 0; d < NDV; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int d = 0; d < ND; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   const int hi_key = row_pos[row0 + npos - 1];
   const int lo_key = window > 0 ? max(0, row_pos[row0] - window + 1) : 0;
@@ -92,6 +106,10 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
   const int p_begin = lo_page + split * per;
   const int p_end = min(lo_page + (split + 1) * per, hi_page + 1);
   const int k_chunks = DQ / 8, v_chunks = DV / 8;
+  // where the lane points in its transposing reads: of each 16 lanes, lane 4 q + e receives element e of
+  // the 8-byte pieces that lanes q, q + 4, q + 8, q + 12 point at, which are to be value elements
+  // 4 q .. 4 q + 3 of keys 4 c .. 4 c + 3
+  const bf16_t* v_lane = Vs + (4 * c + (n >> 2)) * v_row + 4 * (n & 3);
 
   for (int p = p_begin; p < p_end; ++p) {
     const int phys = page_table[static_cast<size_t>(seq) * table_width + p];
@@ -107,7 +125,7 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
       // batch are unconditional, from clamped places (a live key of the tile, the last chunk),
       // so that they travel together instead of each waiting behind a branch.
       // (the widest query rows leave no registers for it: two waves a SIMD count for more there)
-      constexpr int kBatch = NK > 18 ? 1 : 5;
+      constexpr int kBatch = SHARED ? 9 : NK > 18 ? 1 : 5;
       const int last_live = min(kKeys - 1, hi_key - key0);
       const int k_total = kKeys * k_chunks;
       for (int base = 0; base < k_total; base += kThreads * kBatch) {
@@ -127,14 +145,6 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
             const int key = ch % kKeys, col = (ch / kKeys) * 8;
             const uint4 v = key <= last_live ? val[u] : uint4{0u, 0u, 0u, 0u};   // stale slots: zeros
             *reinterpret_cast<uint4*>(Kt + key * k_row + col) = v;
-            if (values_in_keys && col < DV) {
-              const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                Vt[(col + 2 * i) * kVtRow + key] = static_cast<bf16_t>(w[i] & 0xffffu);
-                Vt[(col + 2 * i + 1) * kVtRow + key] = static_cast<bf16_t>(w[i] >> 16);
-              }
-            }
           }
         }
       }
@@ -154,13 +164,8 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
             const int ch = base + u * kThreads + t;
             if (ch < v_total) {
               const int key = ch % kKeys, col = (ch / kKeys) * 8;
-              const uint4 v = key <= last_live ? val[u] : uint4{0u, 0u, 0u, 0u};
-              const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                Vt[(col + 2 * i) * kVtRow + key] = static_cast<bf16_t>(w[i] & 0xffffu);
-                Vt[(col + 2 * i + 1) * kVtRow + key] = static_cast<bf16_t>(w[i] >> 16);
-              }
+              *reinterpret_cast<uint4*>(Vs + key * v_row + col) =
+                  key <= last_live ? val[u] : uint4{0u, 0u, 0u, 0u};
             }
           }
         }
@@ -204,12 +209,11 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
       l_run = l_run * alpha + tile_sum;
       m_run = m_new;
 #pragma unroll
-      for (int d = 0; d < NDV; ++d) {
-        if (d < ndv) {
-          const bf16_t* vr = Vt + (d * 16 + n) * kVtRow + 4 * c;
-          const uint2 lo = *reinterpret_cast<const uint2*>(vr);
-          const uint2 hi = *reinterpret_cast<const uint2*>(vr + 16);
-          const uint4 both = uint4{lo.x, lo.y, hi.x, hi.y};
+      for (int d = 0; d < ND; ++d) {
+        if (d < nd) {
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(v_lane + (d0 + d) * 16));
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(v_lane + (d0 + d) * 16 + 16 * v_row));
+          const s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
           f32x4 a = acc[d];
           a[0] *= alpha; a[1] *= alpha; a[2] *= alpha; a[3] *= alpha;
           acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, both), p_reg,
@@ -226,7 +230,7 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
     const float alpha = expf(m_run - m_new);
     l_run = l_run * alpha + expf(sink - m_new);
 #pragma unroll
-    for (int d = 0; d < NDV; ++d) {
+    for (int d = 0; d < ND; ++d) {
       acc[d][0] *= alpha; acc[d][1] *= alpha; acc[d][2] *= alpha; acc[d][3] *= alpha;
     }
     m_run = m_new;
@@ -235,25 +239,25 @@ attn_wide_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_page
   if (n_splits == 1) {
     float inv = l_run > 0.f ? 1.f / l_run : 0.f;
     if (gate) inv *= 1.0f / (1.0f + expf(-gate[static_cast<size_t>(row) * nq + head]));
-    bf16_t* dst = out + (static_cast<size_t>(row) * nq + head) * DV + 4 * c;
+    bf16_t* dst = out + (static_cast<size_t>(row) * nq + head) * DV + d0 * 16 + 4 * c;
 #pragma unroll
-    for (int d = 0; d < NDV; ++d) {
-      if (d < ndv) {
+    for (int d = 0; d < ND; ++d) {
+      if (d < nd) {
         const float y[4] = {acc[d][0] * inv, acc[d][1] * inv, acc[d][2] * inv, acc[d][3] * inv};
         ei::Vec4<bf16_t>::store(dst + d * 16, y);
       }
     }
   } else {
     const size_t slot = (static_cast<size_t>(row) * nq + head) * n_splits + split;
-    float* dst = part_o + slot * DV + 4 * c;
+    float* dst = part_o + slot * DV + d0 * 16 + 4 * c;
 #pragma unroll
-    for (int d = 0; d < NDV; ++d) {
-      if (d < ndv) {
+    for (int d = 0; d < ND; ++d) {
+      if (d < nd) {
         const float y[4] = {acc[d][0], acc[d][1], acc[d][2], acc[d][3]};
         ei::Vec4<float>::store(dst + d * 16, y);
       }
     }
-    if (c == 0) {
+    if (c == 0 && d0 == 0) {
       part_ml[slot * 2] = m_run;
       part_ml[slot * 2 + 1] = l_run;
     }
@@ -300,9 +304,9 @@ struct Launch {
   const void* function;
 };
 
-template <int NK, int NDV>
+template <int NK, int NDV, bool SHARED>
 const void* kernel_of() {
-  return reinterpret_cast<const void*>(&attn_wide_kernel<NK, NDV>);
+  return reinterpret_cast<const void*>(&attn_wide_kernel<NK, NDV, SHARED>);
 }
 
 int heads_per_block(int G) { return G < kRows ? G : kRows; }
@@ -352,21 +356,23 @@ extern "C" int ei_attention_wide(const void* q, const void* k_pages, const void*
   const int HB = heads_per_block(G);
   const int head_blocks = (G + HB - 1) / HB;
   EI_REQUIRE(static_cast<long long>(nkv) * head_blocks <= 65535, "attention_wide: too many heads");
-  static const Launch table[] = {
-      {4, 4, kernel_of<4, 4>()},     {8, 8, kernel_of<8, 8>()},     {16, 4, kernel_of<16, 4>()},
-      {16, 8, kernel_of<16, 8>()},   {18, 16, kernel_of<18, 16>()}, {18, 32, kernel_of<18, 32>()},
-      {32, 8, kernel_of<32, 8>()},   {32, 32, kernel_of<32, 32>()},
-  };
+#define EI_WIDE(SHARED)                                                                       \
+  {4, 4, kernel_of<4, 4, SHARED>()},     {8, 8, kernel_of<8, 8, SHARED>()},                   \
+  {16, 4, kernel_of<16, 4, SHARED>()},   {16, 8, kernel_of<16, 8, SHARED>()},                 \
+  {18, 16, kernel_of<18, 16, SHARED>()}, {18, 32, kernel_of<18, 32, SHARED>()},               \
+  {32, 8, kernel_of<32, 8, SHARED>()},   {32, 32, kernel_of<32, 32, SHARED>()},
+  constexpr int kForms = 8;
+  static const Launch table[2 * kForms] = {EI_WIDE(false) EI_WIDE(true)};
+#undef EI_WIDE
+  // (with slices an item is one position, so a block's query rows are the heads it takes)
+  const Launch* forms = table + (n_splits > 1 && HB <= 16 ? kForms : 0);
   const int nk = DQ / 32, ndv = DV / 16;
   const Launch* chosen = nullptr;
-  for (const Launch& entry : table)
-    if (entry.nk >= nk && entry.ndv >= ndv) {
-      chosen = &entry;
-      break;
-    }
+  for (int i = 0; i < kForms && !chosen; ++i)
+    if (forms[i].nk >= nk && forms[i].ndv >= ndv) chosen = forms + i;
   EI_REQUIRE(chosen != nullptr, "attention_wide: no kernel for these head sizes");
-  const size_t lds = sizeof(bf16_t) * (static_cast<size_t>(kKeys) * (DQ + kPadK) +
-                                       static_cast<size_t>(DV) * kVtRow);
+  const size_t lds = sizeof(bf16_t) * static_cast<size_t>(kKeys) *
+                     (DQ + kPadK + (values_in_keys ? 0 : DV + kPadK));
   EI_REQUIRE(lds <= 160 * 1024, "attention_wide: head sizes too large for the LDS");
   if (lds > 64 * 1024) {        // beyond the default bound of a launch: ask for it, once a kernel
     static bool raised[sizeof(table) / sizeof(table[0])] = {false};
